@@ -15,23 +15,21 @@
 #include "batch.hpp"
 #include "common.hpp"
 #include "extrema.hpp"
+#include "spline_rules.hpp"
+#include "tile3.hpp"
 
 namespace pa {
 namespace {
 
-constexpr int kThreads = 256;
 constexpr int kTileVals = kTS * kTS * kTS;
 constexpr int kXcds = 8;  // MI355X: 8 XCDs, 32 CUs each
 
 enum Kind { BLUE, YELLOW, HOLLOW, HOLLOW_R, YELLOW_R, BLUE_R, LINE, FACE, CUBE };
-enum Mode { COMPRESS, DECOMPRESS, TUNE };
 
 __device__ __forceinline__ int sidx(int x, int y, int z) { return (z * kTS + y) * kTS + x; }
 
-// Per-tile context.  IN = true for a tile that is not the last one along
-// any axis: all 17^3 points lie inside the field and every boundary test of
-// the stencils is decided at compile time.
-template <typename T, bool IN = false>
+// Per-tile context of the tuner and of 2-D tiles: a plain [17][17][17] tile.
+template <typename T>
 struct Ctx {
     T* s;             // LDS tile
     int ox, oy, oz;   // tile origin
@@ -46,36 +44,13 @@ struct Ctx {
     // the tile is not the last one along axis A (0 = x, 1 = y, 2 = z)
     template <int A>
     __device__ __forceinline__ bool c1() const {
-        return IN || (A == 0 ? c1x : (A == 1 ? c1y : c1z));
-    }
-    // global coordinate v along axis A lies inside the field
-    template <int A>
-    __device__ __forceinline__ bool inf(int v) const {
-        return IN || v < (A == 0 ? g.nx : (A == 1 ? g.ny : g.nz));
+        return A == 0 ? c1x : (A == 1 ? c1y : c1z);
     }
 };
 
 // code i of the hand-off buffer (int32, or int16 when q16)
 __device__ __forceinline__ int32_t code_at(const int32_t* q, bool q16, uint32_t i) {
     return q16 ? (int32_t)reinterpret_cast<const int16_t*>(q)[i] : q[i];
-}
-
-template <typename T>
-__device__ __forceinline__ T cubic(T a, T b, T c, T d, bool natural) {
-    if (natural) return ((((T)-3 * a + (T)23 * b) + (T)23 * c) - (T)3 * d) / (T)40;
-    return (((-a + (T)9 * b) + (T)9 * c) - d) / (T)16;
-}
-template <typename T>
-__device__ __forceinline__ T quad_l(T t0, T t1, T t2) {
-    return ((-t0 + (T)6 * t1) + (T)3 * t2) / (T)8;
-}
-template <typename T>
-__device__ __forceinline__ T quad_r(T t1, T t2, T t3) {
-    return (((T)3 * t1 + (T)6 * t2) - t3) / (T)8;
-}
-template <typename T>
-__device__ __forceinline__ T lin(T t1, T t2) {
-    return (t1 + t2) / (T)2;
 }
 
 // get_interp_order (InterpolationPredictor.cu:1538-1545)
@@ -87,8 +62,8 @@ __device__ __forceinline__ int interp_order(int c, int g, int N, bool c1) {
 }
 
 // 1-D rule along axis A (0 = x, 1 = y, 2 = z), InterpolationPredictor.cu:1269-1326
-template <typename T, int U, int A, bool IN>
-__device__ __forceinline__ T pred_1d(const Ctx<T, IN>& t, int x, int y, int z) {
+template <typename T, int U, int A>
+__device__ __forceinline__ T pred_1d(const Ctx<T>& t, int x, int y, int z) {
     const int c = A == 0 ? x : (A == 1 ? y : z);
     const int o = A == 0 ? t.ox : (A == 1 ? t.oy : t.oz);
     const int N = A == 0 ? t.g.nx : (A == 1 ? t.g.ny : t.g.nz);
@@ -124,8 +99,8 @@ __device__ __forceinline__ void taps(int c, int (&id)[4]) {
 }
 
 // FACE rule, InterpolationPredictor.cu:1546-1669
-template <typename T, int U, bool IN>
-__device__ __forceinline__ T pred_face(const Ctx<T, IN>& t, int x, int y, int z) {
+template <typename T, int U>
+__device__ __forceinline__ T pred_face(const Ctx<T>& t, int x, int y, int z) {
     int idz[4], idy[4], idx[4];
     taps<U>(z, idz);
     taps<U>(y, idy);
@@ -203,8 +178,8 @@ __device__ __forceinline__ T pred_face(const Ctx<T, IN>& t, int x, int y, int z)
 }
 
 // CUBE rule, InterpolationPredictor.cu:1671-1723
-template <typename T, int U, bool IN>
-__device__ __forceinline__ T pred_cube(const Ctx<T, IN>& t, int x, int y, int z) {
+template <typename T, int U>
+__device__ __forceinline__ T pred_cube(const Ctx<T>& t, int x, int y, int z) {
     int idz[4], idy[4], idx[4];
     taps<U>(z, idz);
     taps<U>(y, idy);
@@ -300,18 +275,14 @@ __device__ __forceinline__ void stage_point(int p, int& x, int& y, int& z) {
     }
 }
 
-// Whether point (x, y, z) of the tile is predicted in this sweep: inside the
-// tile (the +1 halo included for inclusive stages; the last stage of the
-// tile row keeps its far plane) and inside the field.
-template <typename T, bool IN>
-__device__ __forceinline__ bool visited(const Ctx<T, IN>& t, int x, int y, int z, bool inclusive) {
-    const bool in = inclusive ? (x <= 16 && y <= 16 && z <= 16)
-                              : (x < 16 && y < 16 && z < 16 + (t.template c1<2>() ? 0 : 1));
-    return in && t.template inf<0>(t.ox + x) && t.template inf<1>(t.oy + y) && t.template inf<2>(t.oz + z);
+// Whether point (x, y, z) of the tile (halo included) lies inside the field.
+template <typename T>
+__device__ __forceinline__ bool visited(const Ctx<T>& t, int x, int y, int z) {
+    return t.ox + x < t.g.nx && t.oy + y < t.g.ny && t.oz + z < t.g.nz;
 }
 
-template <typename T, int U, int K, bool IN>
-__device__ __forceinline__ T predict(const Ctx<T, IN>& t, int x, int y, int z) {
+template <typename T, int U, int K>
+__device__ __forceinline__ T predict(const Ctx<T>& t, int x, int y, int z) {
     if constexpr (K == BLUE || K == BLUE_R) {
         return pred_1d<T, U, 2>(t, x, y, z);
     } else if constexpr (K == YELLOW || K == YELLOW_R) {
@@ -334,508 +305,48 @@ constexpr int level_of() {
     return U == 1 ? 0 : (U == 2 ? 1 : (U == 4 ? 2 : 3));
 }
 
-// The lane id through an opaque move: index arithmetic derived from it in
-// one phase of the kernel is not merged with that of another phase and kept
-// live in registers between them.
-__device__ __forceinline__ int lane_id() {
-    int v;
-    asm volatile("v_mov_b32 %0, %1" : "=v"(v) : "v"((int)threadIdx.x));
-    __builtin_assume(v >= 0 && v < kThreads);
-    return v;
-}
-
-// Barrier for LDS producer/consumer hand-off between stages: waits for this
-// wave's LDS operations only, so outstanding global loads (prefetched codes)
-// and stores (emitted codes) stay in flight across it.
-__device__ __forceinline__ void lds_barrier() {
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
-// Quantise v against pred, write the reconstruction back and return the
-// code (InterpolationPredictor.cu:1327-1341).
-template <typename T>
-__device__ __forceinline__ int32_t quantize_val(T& v, T pred, T eb_r, T ebx2) {
-    const T err = v - pred;
-    T code = (err < (T)0 ? -err : err) * eb_r + (T)1;
-    code = err < (T)0 ? -code : code;
-    const int qv = (int)(code / (T)2);
-    code = (T)qv;
-    v = pred + code * ebx2;
-    return qv;
-}
-
-template <typename T, bool IN>
-__device__ __forceinline__ int32_t quantize(const Ctx<T, IN>& t, T& v, T pred) {
-    return quantize_val(v, pred, t.eb_r, t.ebx2);
-}
-
-// Decompression first fills the LDS slot of every point with the bit
-// pattern of its own code (anchors hold their value, points of skipped
-// levels 0); a stage then reads the slot of the point it reconstructs and
-// overwrites it with pred + code * ebx2.  Predictions read only points of
-// earlier stages, which already hold values.
-__device__ __forceinline__ float code_slot(int32_t q, float) { return __int_as_float(q); }
-__device__ __forceinline__ double code_slot(int32_t q, double) {
-    return __longlong_as_double((long long)(uint32_t)q);
-}
-__device__ __forceinline__ int32_t slot_code(float v) { return __float_as_int(v); }
-__device__ __forceinline__ int32_t slot_code(double v) { return (int32_t)(uint32_t)__double_as_longlong(v); }
-
-// Where a compression stage puts its codes: straight to the level-major
-// array (levels 1-3), into registers with their LDS slots (the first two
-// stages of level 0, whose values later stages still read), or into the
-// point's own LDS slot (the last stage of level 0: no later stage reads its
-// values).  Level 0's codes then leave the tile as whole rows.
-enum Sink { TO_GLOBAL, TO_REGS, TO_SLOT };
-constexpr int kRegCodes = 8;  // points per lane of a level-0 stage (line or point form)
-struct RegCodes {
-    int32_t code[kRegCodes];
-    int32_t slot[kRegCodes];  // -1: no own point
-};
-
 // ----------------------------------------------------------- point form --
-// Lane l visits points p = l + 256 * it of the stage (tuner, and the
-// multi-dimensional stages).
-template <typename T, int U, int K, int M, bool IN, int SINK = TO_GLOBAL>
-__device__ __forceinline__ void stage(Ctx<T, IN>& t, bool inclusive, RegCodes* rc = nullptr) {
+// The tuner's sweep: lane l visits points p = l + 256 * it of the stage and
+// adds up |x - pred|; nothing is written back.
+template <typename T, int U, int K>
+__device__ __forceinline__ void stage(Ctx<T>& t) {
     constexpr int TOTAL = stage_total<U, K>();
-    constexpr int LEVEL = level_of<U>();
-    static_assert(SINK != TO_REGS || stage_iters<U, K>() <= kRegCodes, "register codes: at most 8 points per lane");
     const int lane = lane_id();
-    if constexpr (SINK == TO_REGS) {
-#pragma unroll
-        for (int k = 0; k < kRegCodes; ++k) rc->slot[k] = -1;
-    }
 #pragma unroll
     for (int it = 0; it < stage_iters<U, K>(); ++it) {
         const int p = lane + it * kThreads;
         if (TOTAL % kThreads != 0 && p >= TOTAL) break;
         int x, y, z;
         stage_point<U, K>(p, x, y, z);
-        if (!visited(t, x, y, z, inclusive)) continue;
-        const T pred = predict<T, U, K>(t, x, y, z);
-        T& v = t.s[sidx(x, y, z)];
-        if constexpr (M == TUNE) {
-            const T e = v - pred;
-            t.acc += (double)(e < (T)0 ? -e : e);
-        } else if constexpr (M == COMPRESS) {
-            const int32_t qv = quantize(t, v, pred);
-            const bool own = x < 16 && y < 16 && z < 16;
-            if constexpr (SINK == TO_GLOBAL) {
-                if (own) t.qc_out[lm_index<LEVEL>(t.g, t.ox + x, t.oy + y, t.oz + z)] = qv;
-            } else if constexpr (SINK == TO_REGS) {
-                rc->code[it] = qv;
-                rc->slot[it] = own ? sidx(x, y, z) : -1;
-            } else {
-                v = code_slot(qv, T());
-            }
-        } else {
-            v = pred + (T)slot_code(v) * t.ebx2;
-        }
-    }
-    lds_barrier();
-}
-
-// ------------------------------------------------------------ line form --
-// 1-D stages along y or z run line by line: lane l owns one line along the
-// prediction axis A (consecutive lanes are consecutive lines along x, so
-// their codes are neighbours in memory), reads the N + 1 known values of the
-// line once and predicts its N points with compile-time stencils.  Which
-// stencil a point uses depends only on its position along A and on the
-// tile's place in the field, so the choice is the same for every lane.
-// The values produced are those of the per-point rule above (same formula,
-// same operation order); only the lane assignment differs, and points of one
-// stage never read each other.
-enum Stencil { S_KEEP, S_LIN, S_QUAD_R, S_QUAD_L, S_CUBIC };
-
-template <int U, int K, bool EXCL>
-struct LineShape {
-    static constexpr int N = 16 / (2 * U);
-    static constexpr int A = (K == BLUE || K == BLUE_R) ? 2 : ((K == YELLOW || K == YELLOW_R) ? 1 : 0);
-    // P: first other axis (x, or y when A = x); Q: second (z, or y when A = z)
-    static constexpr bool FULL_P = (K == HOLLOW || K == YELLOW_R || K == BLUE_R);
-    static constexpr bool FULL_Q = (K == YELLOW || K == HOLLOW || K == BLUE_R);
-    static constexpr int SP = FULL_P ? U : 2 * U;
-    static constexpr int SQ = FULL_Q ? U : 2 * U;
-    // the exclusive last stage of level 0 visits x < 16, y < 16, z < 16 (its
-    // z = 16 plane would lie outside the field: only the last tile along z
-    // may visit it, and there oz + 16 >= nz)
-    static constexpr int CP = EXCL ? 16 : (FULL_P ? 2 * N + 1 : N + 1);
-    static constexpr int CQ = EXCL ? 16 : (FULL_Q ? 2 * N + 1 : N + 1);
-    static constexpr int LINES = CP * CQ;
-    static constexpr int ITERS = (LINES + kThreads - 1) / kThreads;
-    static constexpr int SLOTS = ITERS * N;
-    static constexpr int STA = A == 0 ? 1 : (A == 1 ? kTS : kTS * kTS);
-};
-
-// Stencil of point j of a line (position c = (2j+1)U along the axis), the
-// rule of InterpolationPredictor.cu:1269-1326 with c2 = (j >= 1) and
-// c3 = (j <= N - 2).
-template <int U>
-__device__ __forceinline__ int stencil_of(int j, int N, bool c1, int o, int nax) {
-    const int gc = o + (2 * j + 1) * U;
-    const bool c2 = j >= 1, c3 = j <= N - 2, c4 = gc + 3 * U < nax, c5 = gc + U < nax;
-    if ((c1 && !c2 && !c3) || (!c1 && !c2 && !(c3 && c4) && c5)) return S_LIN;
-    if ((c1 && !c2 && c3) || (!c1 && !c2 && c3 && c4)) return S_QUAD_R;
-    if ((c1 && c2 && !c3) || (!c1 && c2 && !(c3 && c4) && c5)) return S_QUAD_L;
-    if ((c1 && c2 && c3) || (!c1 && c2 && c3 && c4)) return S_CUBIC;
-    return S_KEEP;
-}
-
-template <typename T>
-__device__ __forceinline__ T apply_stencil(int k, T t0, T t1, T t2, T t3) {
-    switch (k) {
-        case S_LIN: return lin(t1, t2);
-        case S_QUAD_R: return quad_r(t1, t2, t3);
-        case S_QUAD_L: return quad_l(t0, t1, t2);
-        case S_CUBIC: return cubic(t0, t1, t2, t3, false);
-        default: return t1;
+        if (!visited(t, x, y, z)) continue;
+        const T e = t.s[sidx(x, y, z)] - predict<T, U, K>(t, x, y, z);
+        t.acc += (double)(e < (T)0 ? -e : e);
     }
 }
 
-struct LineLane {
-    int base;       // LDS index of the line's c = 0 point
-    bool on;        // line inside the tile's sweep and the field
-    bool own;       // line inside the 16^3 tile proper (codes are stored)
-    uint32_t idx0;  // level-major index of point j = 0
-    uint32_t st;    // level-major stride between consecutive points
-};
-
-template <typename T, int U, int K, bool EXCL, bool IN>
-__device__ __forceinline__ LineLane line_lane(const Ctx<T, IN>& t, int it) {
-    using S = LineShape<U, K, EXCL>;
-    LineLane r;
-    const int l = lane_id() + it * kThreads;
-    const int ip = l % S::CP, iq = l / S::CP;
-    const int pc = S::SP * ip, qc = S::SQ * iq;
-    int x, y, z;  // point j = 0
-    if constexpr (S::A == 0) { x = U; y = pc; z = qc; }
-    else if constexpr (S::A == 1) { x = pc; y = U; z = qc; }
-    else { x = pc; y = qc; z = U; }
-    const int gx = t.ox + x, gy = t.oy + y, gz = t.oz + z;
-    bool on = (S::LINES % kThreads == 0 || l < S::LINES);
-    if constexpr (S::A != 0) on = on && t.template inf<0>(gx);
-    if constexpr (S::A != 1) on = on && t.template inf<1>(gy);
-    if constexpr (S::A != 2) on = on && t.template inf<2>(gz);
-    r.on = on;
-    r.own = x < 16 && y < 16 && z < 16;
-    r.base = sidx(x, y, z) - U * S::STA;
-    constexpr int LEVEL = level_of<U>();
-    r.idx0 = lm_index<LEVEL>(t.g, gx, gy, gz);
-    r.st = 0;
-    if constexpr (S::N >= 2) {
-        // the index is affine along the line: the varying coordinate keeps
-        // its parity and its halves grow by one per point
-        const uint32_t i1 = S::A == 0 ? lm_index<LEVEL>(t.g, gx + 2 * U, gy, gz)
-                                     : (S::A == 1 ? lm_index<LEVEL>(t.g, gx, gy + 2 * U, gz)
-                                                  : lm_index<LEVEL>(t.g, gx, gy, gz + 2 * U));
-        r.st = i1 - r.idx0;
-    }
-    return r;
-}
-
-template <typename T, int U, int K, bool EXCL, int M, bool IN, int SINK = TO_GLOBAL>
-__device__ __forceinline__ void line_stage(Ctx<T, IN>& t, RegCodes* rc = nullptr) {
-    using S = LineShape<U, K, EXCL>;
-    constexpr int N = S::N;
-    static_assert(SINK != TO_REGS || S::ITERS * N <= kRegCodes, "register codes: at most 8 points per lane");
-    if constexpr (SINK == TO_REGS) {
-#pragma unroll
-        for (int k = 0; k < kRegCodes; ++k) rc->slot[k] = -1;
-    }
-    const int o = S::A == 0 ? t.ox : (S::A == 1 ? t.oy : t.oz);
-    const int nax = S::A == 0 ? t.g.nx : (S::A == 1 ? t.g.ny : t.g.nz);
-    const bool c1 = t.template c1<S::A>();
-#pragma unroll
-    for (int it = 0; it < S::ITERS; ++it) {
-        const LineLane ln = line_lane<T, U, K, EXCL>(t, it);
-        if (!ln.on) continue;
-        T k[N + 1];
-#pragma unroll
-        for (int j = 0; j <= N; ++j) k[j] = t.s[ln.base + 2 * j * U * S::STA];
-#pragma unroll
-        for (int j = 0; j < N; ++j) {
-            if (!t.template inf<S::A>(o + (2 * j + 1) * U)) break;  // beyond the field; so are later points
-            const T pred = apply_stencil(stencil_of<U>(j, N, c1, o, nax), k[j > 0 ? j - 1 : 0], k[j], k[j + 1],
-                                         k[j + 2 <= N ? j + 2 : 0]);
-            const int slot = ln.base + (2 * j + 1) * U * S::STA;
-            T& v = t.s[slot];
-            if constexpr (M == COMPRESS) {
-                const int32_t qv = quantize(t, v, pred);
-                if constexpr (SINK == TO_GLOBAL) {
-                    if (ln.own) t.qc_out[ln.idx0 + j * ln.st] = qv;
-                } else if constexpr (SINK == TO_REGS) {
-                    rc->code[it * N + j] = qv;
-                    rc->slot[it * N + j] = ln.own ? slot : -1;
-                } else {
-                    v = code_slot(qv, T());
-                }
-            } else {
-                v = pred + (T)slot_code(v) * t.ebx2;
-            }
-        }
-    }
-    lds_barrier();
-}
-
-// ---------------------------------------------------------------- levels --
-// The three stages of one level; outside tuning the last stage of level 0
-// uses the exclusive border (InterpolationPredictor.cu:1940-2025).
-template <typename T, bool IN>
-__device__ __forceinline__ void level0_codes_out(Ctx<T, IN>& t, const RegCodes& a, const RegCodes& b);
-
-template <typename T, int U, int M, bool IN>
-__device__ __forceinline__ void level(Ctx<T, IN>& t, bool md, bool rev) {
-    constexpr bool EX = M != TUNE && U == 1;
-    if constexpr (M == COMPRESS && U == 1) {
-        RegCodes a, b;
-        if (md) {
-            stage<T, 1, LINE, M, IN, TO_REGS>(t, true, &a);
-            stage<T, 1, FACE, M, IN, TO_REGS>(t, true, &b);
-            stage<T, 1, CUBE, M, IN, TO_SLOT>(t, false);
-        } else if (rev) {
-            line_stage<T, 1, HOLLOW_R, false, M, IN, TO_REGS>(t, &a);
-            line_stage<T, 1, YELLOW_R, false, M, IN, TO_REGS>(t, &b);
-            line_stage<T, 1, BLUE_R, true, M, IN, TO_SLOT>(t);
-        } else {
-            line_stage<T, 1, BLUE, false, M, IN, TO_REGS>(t, &a);
-            line_stage<T, 1, YELLOW, false, M, IN, TO_REGS>(t, &b);
-            line_stage<T, 1, HOLLOW, true, M, IN, TO_SLOT>(t);
-        }
-        level0_codes_out(t, a, b);
-        return;
-    }
+// the three stages of one level
+template <typename T, int U>
+__device__ __forceinline__ void level(Ctx<T>& t, bool md, bool rev) {
     if (md) {
-        stage<T, U, LINE, M>(t, true);
-        stage<T, U, FACE, M>(t, true);
-        stage<T, U, CUBE, M>(t, !EX);
-    } else if constexpr (M == TUNE) {
-        if (rev) {
-            stage<T, U, HOLLOW_R, M>(t, true);
-            stage<T, U, YELLOW_R, M>(t, true);
-            stage<T, U, BLUE_R, M>(t, true);
-        } else {
-            stage<T, U, BLUE, M>(t, true);
-            stage<T, U, YELLOW, M>(t, true);
-            stage<T, U, HOLLOW, M>(t, true);
-        }
+        stage<T, U, LINE>(t);
+        stage<T, U, FACE>(t);
+        stage<T, U, CUBE>(t);
     } else if (rev) {
-        line_stage<T, U, HOLLOW_R, false, M>(t);
-        line_stage<T, U, YELLOW_R, false, M>(t);
-        line_stage<T, U, BLUE_R, EX, M>(t);
+        stage<T, U, HOLLOW_R>(t);
+        stage<T, U, YELLOW_R>(t);
+        stage<T, U, BLUE_R>(t);
     } else {
-        line_stage<T, U, BLUE, false, M>(t);
-        line_stage<T, U, YELLOW, false, M>(t);
-        line_stage<T, U, HOLLOW, EX, M>(t);
+        stage<T, U, BLUE>(t);
+        stage<T, U, YELLOW>(t);
+        stage<T, U, HOLLOW>(t);
     }
 }
 
-// Decompression start: the slot of every tile point (17^3, halo included)
-// gets its code, its anchor or 0.  Level L's points are the multiples of
-// U = 2^L in the tile that are not all multiples of 2U.  Along a row (y, z)
-// of level L the level-major index is affine in x (the compaction formula,
-// InterpolationPredictor.cu:2070-2083): with i = x / U,
-//   rows with y/U or z/U odd hold every i:  idx = base_L(y, z) + ox/U + i,
-//   other rows hold the odd i only:          idx = base_L(y, z) + ox/(2U) + i/2.
-// The 404 row bases of a tile (17^2 + 9^2 + 5^2 + 3^2) are computed once
-// into LDS; then every code load is one table read and an add, and all
-// loads are issued before the first slot is written.
-constexpr int kRows0 = 289, kRows1 = 81, kRows2 = 25, kRows3 = 9;
-constexpr int kRowTab = kRows0 + kRows1 + kRows2 + kRows3;  // 404
-template <int L>
-constexpr int row_off() {
-    return L == 0 ? 0 : (L == 1 ? kRows0 : (L == 2 ? kRows0 + kRows1 : kRows0 + kRows1 + kRows2));
-}
-
-template <int L>
-__device__ __forceinline__ int32_t row_base(const Geom& g, int gy, int gz) {
-    // 32-bit unsigned arithmetic, exact below code_len < 2^31 (as lm_index)
-    const uint32_t b = (uint32_t)gy >> L, c = (uint32_t)gz >> L;
-    uint32_t r = b * (uint32_t)g.lx[L] + c * (uint32_t)g.lxy[L] + (uint32_t)g.prefix[L] -
-                 ((c + 1) >> 1) * (uint32_t)g.lxy[L + 1];
-    if ((c & 1) == 0) r -= ((b + 1) >> 1) * (uint32_t)g.lx[L + 1];
-    return (int32_t)r;
-}
-
-// Level 0's codes of the 16^3 tile, all in their LDS slots once the
-// register-held ones join them, written out row by row: lane (x, y) =
-// (l mod 16, l / 16) takes z = 0..15; a row (y, z) with y or z odd holds
-// every x (16 adjacent codes), the others the odd x (8 adjacent codes).
-// Row bases advance by 2 lxy0 - lxy1 from z to z + 2.
-template <typename T, bool IN>
-__device__ __forceinline__ void level0_codes_out(Ctx<T, IN>& t, const RegCodes& a, const RegCodes& b) {
-#pragma unroll
-    for (int k = 0; k < kRegCodes; ++k) {
-        if (a.slot[k] >= 0) t.s[a.slot[k]] = code_slot(a.code[k], T());
-        if (b.slot[k] >= 0) t.s[b.slot[k]] = code_slot(b.code[k], T());
-    }
-    lds_barrier();
-    const int lane = lane_id();
-    const int x = lane & 15, y = lane >> 4;
-    const int gx = t.ox + x, gy = t.oy + y;
-    if (!(t.template inf<0>(gx) && t.template inf<1>(gy))) return;
-    const uint32_t step2 = (uint32_t)(2 * t.g.lxy[0] - t.g.lxy[1]);
-    const uint32_t base_e = (uint32_t)row_base<0>(t.g, gy, t.oz), base_o = (uint32_t)row_base<0>(t.g, gy, t.oz + 1);
-    const uint32_t off_full = (uint32_t)gx, off_half = (uint32_t)((t.ox >> 1) + (x >> 1));
-#pragma unroll
-    for (int z = 0; z < 16; ++z) {
-        if (!t.template inf<2>(t.oz + z)) break;
-        const bool full = ((y | z) & 1) != 0;
-        if (full || (x & 1)) {
-            const uint32_t base = ((z & 1) ? base_o : base_e) + (uint32_t)(z >> 1) * step2;
-            t.qc_out[base + (full ? off_full : off_half)] = slot_code(t.s[sidx(x, y, z)]);
-        }
-    }
-}
-
-template <typename T, int L, bool IN>
-__device__ __forceinline__ void row_entry(const Ctx<T, IN>& t, int32_t* tab, int row) {
-    constexpr int U = 1 << L, E = 16 / U + 1;
-    const int gy = t.oy + U * (row % E), gz = t.oz + U * (row / E);
-    tab[row_off<L>() + row] = (t.template inf<1>(gy) && t.template inf<2>(gz)) ? row_base<L>(t.g, gy, gz) : 0;
-}
-
-template <typename T, bool IN>
-__device__ __forceinline__ void fill_rows(const Ctx<T, IN>& t, int32_t* tab) {
-    const int lane = lane_id();
-    row_entry<T, 0>(t, tab, lane);
-    if (lane + kThreads < kRows0) row_entry<T, 0>(t, tab, lane + kThreads);
-    if (lane < kRows1) row_entry<T, 1>(t, tab, lane);
-    else if (lane < kRows1 + kRows2) row_entry<T, 2>(t, tab, lane - kRows1);
-    else if (lane < kRows1 + kRows2 + kRows3) row_entry<T, 3>(t, tab, lane - kRows1 - kRows2);
-}
-
-// Level 0: lane l keeps x = l mod 16 and takes rows r = l / 16 + 16 it; the
-// x = 16 column is a second, short pass.  Levels 1-3: lane l takes lattice
-// point p = l + 256 it of the level's E^3 lattice (x fastest).
-constexpr int kFill0Iters = (kRows0 + 15) / 16;                   // 19
+// rows of a plain tile, and the passes that take them 16 rows (or the x = 16
+// column 256 points) at a time
+constexpr int kRows0 = kTS * kTS;  // 289
+constexpr int kFill0Iters = (kRows0 + 15) / 16;                      // 19
 constexpr int kFill0EdgeIters = (kRows0 + kThreads - 1) / kThreads;  // 2
-template <int L>
-struct FillShape {
-    static constexpr int U = 1 << L, E = 16 / U + 1, TOTAL = E * E * E;
-    static constexpr int ITERS = (TOTAL + kThreads - 1) / kThreads;
-};
-
-// Row r0 + 16 it of the 17 x 17 rows of a tile (r0 = lane / 16 < 16):
-// (y, z) = (r0 - it, it), or (r0 - it + 17, it - 1) when r0 < it (16 is
-// -1 mod 17), and (16, 16) for the last row (it = 18, r0 = 0 only).
-struct RowYZ {
-    int y, z;
-    bool valid;
-};
-template <int IT>
-__device__ __forceinline__ RowYZ row_yz(int r0) {
-    RowYZ w;
-    if constexpr (IT == kFill0Iters - 1) {
-        w.y = 16;
-        w.z = 16;
-        w.valid = r0 == 0;
-    } else {
-        const bool wrap = r0 < IT;
-        w.y = r0 - IT + (wrap ? kTS : 0);
-        w.z = IT - (wrap ? 1 : 0);
-        w.valid = true;
-    }
-    return w;
-}
-
-template <typename T, int IT, bool IN>
-__device__ __forceinline__ void fill0_one(const Ctx<T, IN>& t, const int32_t* tab, bool load, int r0, int x, bool xin,
-                                          uint32_t off_full, uint32_t off_half, int32_t& v) {
-    const RowYZ w = row_yz<IT>(r0);
-    const bool full = ((w.y | w.z) & 1) != 0;
-    v = 0;
-    if (load && w.valid && xin && (full || (x & 1)) && t.template inf<1>(t.oy + w.y) && t.template inf<2>(t.oz + w.z))
-        v = code_at(t.qc_in, t.q16, (uint32_t)tab[r0 + 16 * IT] + (full ? off_full : off_half));
-}
-
-template <typename T, int IT, bool IN>
-__device__ __forceinline__ void fill0_iter(const Ctx<T, IN>& t, const int32_t* tab, bool load, int r0, int x,
-                                           bool xin, uint32_t off_full, uint32_t off_half,
-                                           int32_t (&v)[kFill0Iters]) {
-    if constexpr (IT < kFill0Iters) {
-        fill0_one<T, IT>(t, tab, load, r0, x, xin, off_full, off_half, v[IT]);
-        fill0_iter<T, IT + 1>(t, tab, load, r0, x, xin, off_full, off_half, v);
-    }
-}
-
-template <typename T, bool IN>
-__device__ __forceinline__ void fill0_load(const Ctx<T, IN>& t, const int32_t* tab, bool load,
-                                           int32_t (&v)[kFill0Iters], int32_t (&e)[kFill0EdgeIters]) {
-    const int lane = lane_id();
-    const int x = lane & 15, r0 = lane >> 4;
-    const bool xin = t.template inf<0>(t.ox + x);
-    fill0_iter<T, 0>(t, tab, load, r0, x, xin, (uint32_t)(t.ox + x), (uint32_t)((t.ox >> 1) + (x >> 1)), v);
-#pragma unroll
-    for (int it = 0; it < kFill0EdgeIters; ++it) {  // x = 16: level 0 where y or z is odd
-        const int r = lane + kThreads * it;
-        const int y = r % kTS, z = r / kTS;
-        e[it] = 0;
-        if (load && r < kRows0 && ((y | z) & 1) && t.template inf<0>(t.ox + 16) && t.template inf<1>(t.oy + y) &&
-            t.template inf<2>(t.oz + z))
-            e[it] = code_at(t.qc_in, t.q16, (uint32_t)tab[r] + (uint32_t)(t.ox + 16));
-    }
-}
-
-template <typename T, int IT>
-__device__ __forceinline__ void fill0_put(T* s, int r0, int x, const int32_t (&v)[kFill0Iters]) {
-    if constexpr (IT < kFill0Iters) {
-        const RowYZ w = row_yz<IT>(r0);
-        if (w.valid && (((w.y | w.z) & 1) || (x & 1))) s[(r0 + 16 * IT) * kTS + x] = code_slot(v[IT], T());
-        fill0_put<T, IT + 1>(s, r0, x, v);
-    }
-}
-
-template <typename T>
-__device__ __forceinline__ void fill0_store(T* s, const int32_t (&v)[kFill0Iters],
-                                            const int32_t (&e)[kFill0EdgeIters]) {
-    const int lane = lane_id();
-    const int x = lane & 15, r0 = lane >> 4;
-    fill0_put<T, 0>(s, r0, x, v);
-#pragma unroll
-    for (int it = 0; it < kFill0EdgeIters; ++it) {
-        const int r = lane + kThreads * it;
-        const int y = r % kTS, z = r / kTS;
-        if (r < kRows0 && ((y | z) & 1)) s[r * kTS + 16] = code_slot(e[it], T());
-    }
-}
-
-template <typename T, int L, bool IN>
-__device__ __forceinline__ void fill_load(const Ctx<T, IN>& t, const int32_t* tab, bool load,
-                                          int32_t (&v)[FillShape<L>::ITERS]) {
-    using F = FillShape<L>;
-    const int lane = lane_id();
-#pragma unroll
-    for (int it = 0; it < F::ITERS; ++it) {
-        const int p = lane + it * kThreads;
-        const int i = p % F::E, row = p / F::E, j = row % F::E, k = row / F::E;
-        const bool full = ((j | k) & 1) != 0;
-        const bool mine = (F::TOTAL % kThreads == 0 || p < F::TOTAL) && (full || (i & 1));
-        v[it] = 0;
-        if (load && mine && t.template inf<0>(t.ox + i * F::U) && t.template inf<1>(t.oy + j * F::U) &&
-            t.template inf<2>(t.oz + k * F::U))
-            v[it] = code_at(t.qc_in, t.q16,
-                            (uint32_t)(tab[row_off<L>() + row] + (full ? (t.ox >> L) + i : (t.ox >> (L + 1)) + (i >> 1))));
-    }
-}
-
-template <typename T, int L>
-__device__ __forceinline__ void fill_store(T* s, const int32_t (&v)[FillShape<L>::ITERS]) {
-    using F = FillShape<L>;
-    const int lane = lane_id();
-#pragma unroll
-    for (int it = 0; it < F::ITERS; ++it) {
-        const int p = lane + it * kThreads;
-        const int i = p % F::E, row = p / F::E, j = row % F::E, k = row / F::E;
-        if ((F::TOTAL % kThreads == 0 || p < F::TOTAL) && ((i | j | k) & 1))
-            s[sidx(i * F::U, j * F::U, k * F::U)] = code_slot(v[it], T());
-    }
-}
-
-template <typename T>
-struct LevelEb {
-    T eb_r[4], ebx2[4];
-};
 
 // Level bounds from a device block laid out as {absolute eb, range,
 // eb_r[4] and ebx2[4] in float64, then eb_r[4] and ebx2[4] in float32}.
@@ -866,12 +377,12 @@ __device__ __forceinline__ LevelEb<T> load_level_ebs(const double* e) {
 // (288, taken by r0 = 0 at it = 18) is (16, 16).  The x = 16 column is a
 // second, short pass.  Field offsets below 2^31 (the layout's limit) are
 // 32-bit.
-template <typename T, bool IN>
-__device__ __forceinline__ void load_tile(const Ctx<T, IN>& t, const T* data) {
+template <typename T>
+__device__ __forceinline__ void load_tile(const Ctx<T>& t, const T* data) {
     const int lane = lane_id();
     const int x = lane & 15, r0 = lane >> 4;
     const uint32_t nx = (uint32_t)t.g.nx, nxy = nx * (uint32_t)t.g.ny;
-    const bool xin = t.template inf<0>(t.ox + x);
+    const bool xin = t.ox + x < t.g.nx;
     const T* base = data + ((uint32_t)t.oz * nxy + (uint32_t)t.oy * nx + (uint32_t)t.ox);
     const uint32_t lane_off = (uint32_t)r0 * nx + (uint32_t)x;
     const uint32_t step = nxy - nx, wrap_off = 17 * nx - nxy;  // per row step; back by 17 rows of y
@@ -883,7 +394,7 @@ __device__ __forceinline__ void load_tile(const Ctx<T, IN>& t, const T* data) {
         const uint32_t off =
             last ? 16 * nx + 16 * nxy + (uint32_t)x : lane_off + (uint32_t)it * step + (wrap ? wrap_off : 0u);
         v[it] = (T)0;
-        if ((it < kFill0Iters - 1 || r0 == 0) && xin && t.template inf<1>(t.oy + y) && t.template inf<2>(t.oz + z))
+        if ((it < kFill0Iters - 1 || r0 == 0) && xin && t.oy + y < t.g.ny && t.oz + z < t.g.nz)
             v[it] = base[off];
     }
 #pragma unroll
@@ -891,7 +402,7 @@ __device__ __forceinline__ void load_tile(const Ctx<T, IN>& t, const T* data) {
         const int r = lane + kThreads * it;
         const int y = r % kTS, z = r / kTS;
         e[it] = (T)0;
-        if (r < kRows0 && t.template inf<0>(t.ox + 16) && t.template inf<1>(t.oy + y) && t.template inf<2>(t.oz + z))
+        if (r < kRows0 && t.ox + 16 < t.g.nx && t.oy + y < t.g.ny && t.oz + z < t.g.nz)
             e[it] = base[(uint32_t)y * nx + (uint32_t)z * nxy + 16u];
     }
 #pragma unroll
@@ -959,69 +470,6 @@ __device__ __forceinline__ void clear_gaps(const SplineArgs<T>& a) {
     }
 }
 
-// Per-tile context of tile (bx, by, bz).
-template <typename T, bool IN>
-__device__ __forceinline__ Ctx<T, IN> tile_ctx(const SplineArgs<T>& a, T* tile, int bx, int by, int bz, bool q16) {
-    const Geom& g = a.g;
-    Ctx<T, IN> t;
-    t.s = tile;
-    t.ox = bx * 16;
-    t.oy = by * 16;
-    t.oz = bz * 16;
-    t.c1x = t.ox + 16 < g.nx;
-    t.c1y = t.oy + 16 < g.ny;
-    t.c1z = t.oz + 16 < g.nz;
-    t.g = g;
-    t.qc_out = a.qc_out;
-    t.qc_in = a.qc_in;
-    t.q16 = q16;
-    t.natural = false;
-    t.acc = 0.0;
-    return t;
-}
-
-// ------------------------------------------------------- decompression --
-// A tile's codes and corner anchors in registers, between their loads and
-// their LDS slots.
-template <typename T>
-struct TileCodes {
-    int32_t v3[FillShape<3>::ITERS], v2[FillShape<2>::ITERS], v1[FillShape<1>::ITERS], v0[kFill0Iters],
-        e0[kFill0EdgeIters];
-    T anc;
-    int aslot;
-};
-
-// Issues the loads of every code of the tile (levels up to maxlevel) from the
-// row table of the tile in LDS, and of its eight corner anchors
-// (x_reset_scratch_data 1051-1061).
-template <typename T, bool IN>
-__device__ __forceinline__ void codes_load(const Ctx<T, IN>& t, const int32_t* rowtab, int maxlevel,
-                                           const T* anchors_in, int bx, int by, int bz, TileCodes<T>& c) {
-    const Geom& g = t.g;
-    fill_load<T, 3>(t, rowtab, 3 <= maxlevel, c.v3);
-    fill_load<T, 2>(t, rowtab, 2 <= maxlevel, c.v2);
-    fill_load<T, 1>(t, rowtab, 1 <= maxlevel, c.v1);
-    fill0_load<T>(t, rowtab, 0 <= maxlevel, c.v0, c.e0);
-    c.anc = (T)0;
-    c.aslot = -1;
-    if (threadIdx.x < 8) {
-        const int cx = threadIdx.x & 1, cy = (threadIdx.x >> 1) & 1, cz = threadIdx.x >> 2;
-        const int ax = bx + cx, ay = by + cy, az = bz + cz;
-        c.aslot = sidx(16 * cx, 16 * cy, 16 * cz);
-        if (anchors_in && ax < g.gx && ay < g.gy && az < g.gz)
-            c.anc = anchors_in[ax + (int64_t)ay * g.gx + (int64_t)az * g.gx * g.gy];
-    }
-}
-
-template <typename T>
-__device__ __forceinline__ void codes_store(T* tile, const TileCodes<T>& c) {
-    fill_store<T, 3>(tile, c.v3);
-    fill_store<T, 2>(tile, c.v2);
-    fill_store<T, 1>(tile, c.v1);
-    fill0_store<T>(tile, c.v0, c.e0);
-    if (c.aslot >= 0) tile[c.aslot] = c.anc;
-}
-
 // ------------------------------------------ codes from the bit-planes --
 // A progressive round whose window is narrow reads each tile's codes from
 // the decoded bit-planes instead of a code hand-off: the inverse shuffle
@@ -1035,6 +483,19 @@ __device__ __forceinline__ void codes_store(T* tile, const TileCodes<T>& c) {
 // m gathers bit m of each window plane k at bit 31 - k, and the negabinary
 // inverse of that word is the round's code, as the inverse shuffle
 // computes it.
+constexpr int kRows1 = 81, kRows2 = 25, kRows3 = 9, kRowTab = kRows0 + kRows1 + kRows2 + kRows3;  // 404
+
+// level-major index of row (gy, gz) of level L, less the x part
+template <int L>
+__device__ __forceinline__ int32_t row_base(const Geom& g, int gy, int gz) {
+    // 32-bit unsigned arithmetic, exact below code_len < 2^31 (as lm_index)
+    const uint32_t b = (uint32_t)gy >> L, c = (uint32_t)gz >> L;
+    uint32_t r = b * (uint32_t)g.lx[L] + c * (uint32_t)g.lxy[L] + (uint32_t)g.prefix[L] -
+                 ((c + 1) >> 1) * (uint32_t)g.lxy[L + 1];
+    if ((c & 1) == 0) r -= ((b + 1) >> 1) * (uint32_t)g.lx[L + 1];
+    return (int32_t)r;
+}
+
 struct PlaneRow {
     int row;     // row (j, k) = (row mod E, row / E) of the level's lattice
     bool full;   // the row holds every i, or the odd i only
@@ -1048,7 +509,7 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef u32x2 u32x2_a4 __attribute__((aligned(4)));
 
 template <int L, typename T, bool IN>
-__device__ __forceinline__ void plane_row_load(const Ctx<T, IN>& t, const PlaneSrc& ps, int row, int maxlevel, int b,
+__device__ __forceinline__ void plane_row_load(const Tile<T, IN>& t, const PlaneSrc& ps, int row, int maxlevel, int b,
                                                int e, PlaneRow& r) {
     constexpr int U = 1 << L, E = 16 / U + 1;
     const int j = row % E, k = row / E;
@@ -1056,11 +517,11 @@ __device__ __forceinline__ void plane_row_load(const Ctx<T, IN>& t, const PlaneS
     r.full = ((j | k) & 1) != 0;
     const int n = r.full ? E : (E - 1) / 2;
     r.nv = 0;
-    if (L <= maxlevel && t.template inf<1>(t.oy + U * j) && t.template inf<2>(t.oz + U * k)) {
+    if (L <= maxlevel && t.template in<1>(U * j) && t.template in<2>(U * k)) {
         if (IN) {
             r.nv = n;
         } else {  // i = m (full) or 2m + 1 (odd i) with ox + U i < nx
-            const int ilim = (t.g.nx - t.ox + U - 1) >> L;
+            const int ilim = (t.rx + U - 1) >> L;
             r.nv = min(n, r.full ? ilim : ilim >> 1);
         }
     }
@@ -1122,7 +583,7 @@ __device__ __forceinline__ void plane_row_store(T* s, const PlaneRow& r, int b) 
     // right by b (b < 32 wherever a plane was read; else the byte is 0)
     const int sb = b & 31;
     const int n = r.full ? E : (E - 1) / 2;
-    const int first = sidx(r.full ? 0 : U, U * j, U * k), step = r.full ? U : 2 * U;
+    const int first = tslot(r.full ? 0 : U, U * j, U * k), step = r.full ? U : 2 * U;
 #pragma unroll
     for (int m = 0; m < E; ++m) {
         if (m < n) {
@@ -1142,13 +603,11 @@ struct PlaneCodes {
     PlaneRow r0, r1;
     int wb[4];  // per level lr = 3 - L
     T anc;
-    int aslot;
 };
 
 template <typename T, bool IN>
-__device__ __forceinline__ void plane_codes_load(const Ctx<T, IN>& t, const PlaneSrc& ps, int maxlevel,
+__device__ __forceinline__ void plane_codes_load(const Tile<T, IN>& t, const PlaneSrc& ps, int maxlevel,
                                                  const T* anchors_in, int bx, int by, int bz, PlaneCodes<T>& c) {
-    const Geom& g = t.g;
     int we[4];
 #pragma unroll
     for (int lr = 0; lr < 4; ++lr) {
@@ -1163,19 +622,11 @@ __device__ __forceinline__ void plane_codes_load(const Ctx<T, IN>& t, const Plan
     else if (rg < k1) plane_row_load<1>(t, ps, rg - kRows0, maxlevel, c.wb[2], we[2], c.r1);
     else if (rg < k2) plane_row_load<2>(t, ps, rg - k1, maxlevel, c.wb[1], we[1], c.r1);
     else if (rg < kRowTab) plane_row_load<3>(t, ps, rg - k2, maxlevel, c.wb[0], we[0], c.r1);
-    c.anc = (T)0;
-    c.aslot = -1;
-    if (threadIdx.x < 8) {
-        const int cx = threadIdx.x & 1, cy = (threadIdx.x >> 1) & 1, cz = threadIdx.x >> 2;
-        const int ax = bx + cx, ay = by + cy, az = bz + cz;
-        c.aslot = sidx(16 * cx, 16 * cy, 16 * cz);
-        if (anchors_in && ax < g.gx && ay < g.gy && az < g.gz)
-            c.anc = anchors_in[ax + (int64_t)ay * g.gx + (int64_t)az * g.gx * g.gy];
-    }
+    c.anc = anchor_load(t, anchors_in, bx, by, bz);
 }
 
 template <typename T, bool IN>
-__device__ __forceinline__ void plane_codes_store(const Ctx<T, IN>& t, const PlaneCodes<T>& c) {
+__device__ __forceinline__ void plane_codes_store(const Tile<T, IN>& t, const PlaneCodes<T>& c) {
     constexpr int k1 = kRows0 + kRows1, k2 = k1 + kRows2;
     const int rg = lane_id() + kThreads;
     plane_row_store<0>(t.s, c.r0, c.wb[3]);
@@ -1183,55 +634,46 @@ __device__ __forceinline__ void plane_codes_store(const Ctx<T, IN>& t, const Pla
     else if (rg < k1) plane_row_store<1>(t.s, c.r1, c.wb[2]);
     else if (rg < k2) plane_row_store<2>(t.s, c.r1, c.wb[1]);
     else if (rg < kRowTab) plane_row_store<3>(t.s, c.r1, c.wb[0]);
-    if (c.aslot >= 0) t.s[c.aslot] = c.anc;
+    anchor_store(t, c.anc);
 }
 
 // The previous reconstruction of the tile (delta form); lane: (x, y) =
 // (l mod 16, l / 16), iteration: z.
 constexpr int kOutIters = 4096 / kThreads;
 template <typename T, bool IN>
-__device__ __forceinline__ void prev_load(const Ctx<T, IN>& t, const T* old, T (&prev)[kOutIters]) {
-    const Geom& g = t.g;
+__device__ __forceinline__ void prev_load(const Tile<T, IN>& t, const T* old, T (&prev)[kOutIters]) {
     const int lane = lane_id();
-    const int gx = t.ox + (lane & 15), gy = t.oy + (lane >> 4);
-    const bool in_xy = t.template inf<0>(gx) && t.template inf<1>(gy);
-    const int64_t nxy = (int64_t)g.nx * g.ny;
-    const T* src = old + (int64_t)gx + (int64_t)gy * g.nx + (int64_t)t.oz * nxy;
+    const int x = lane & 15, y = lane >> 4;
+    const bool on = t.template in<0>(x) && t.template in<1>(y);
+    const int64_t nxy = (int64_t)t.g.nx * t.g.ny;
+    const T* src = old + (t.oz * nxy + (int64_t)(t.oy + y) * t.g.nx + t.ox + x);
 #pragma unroll
     for (int z = 0; z < kOutIters; ++z) {
         prev[z] = (T)0;
         // read once, here only: no cache allocation (reconstruction 158 -> 154 us)
-        if (in_xy && t.template inf<2>(t.oz + z)) prev[z] = __builtin_nontemporal_load(&src[z * nxy]);
+        if (on && t.template in<2>(z)) prev[z] = __builtin_nontemporal_load(src);
+        src += nxy;
     }
 }
 
 // The reconstructed tile (plus the previous one in the delta form) to `out`.
 template <typename T, bool IN>
-__device__ __forceinline__ void tile_out(const Ctx<T, IN>& t, bool delta, const T (&prev)[kOutIters], T* out) {
-    const Geom& g = t.g;
+__device__ __forceinline__ void tile_out(const Tile<T, IN>& t, bool delta, const T (&prev)[kOutIters], T* out) {
     const int lane = lane_id();
     const int x = lane & 15, y = lane >> 4;
-    const int gx = t.ox + x, gy = t.oy + y;
-    const bool in_xy = t.template inf<0>(gx) && t.template inf<1>(gy);
-    const int64_t nxy = (int64_t)g.nx * g.ny;
-    T* dst = out + (int64_t)gx + (int64_t)gy * g.nx + (int64_t)t.oz * nxy;
+    if (!(t.template in<0>(x) && t.template in<1>(y))) return;
+    const int64_t nxy = (int64_t)t.g.nx * t.g.ny;
+    const T* src = t.s + tslot(x, y, 0);
+    T* dst = out + (t.oz * nxy + (int64_t)(t.oy + y) * t.g.nx + t.ox + x);
 #pragma unroll
     for (int z = 0; z < kOutIters; ++z) {
-        if (in_xy && t.template inf<2>(t.oz + z)) {
-            const T v = t.s[sidx(x, y, z)];
+        if (t.template in<2>(z)) {
+            const T v = src[z * kZP];
             // written once and read only by a later round: no cache allocation
-            __builtin_nontemporal_store(delta ? v + prev[z] : v, &dst[z * nxy]);
+            __builtin_nontemporal_store(delta ? v + prev[z] : v, dst);
         }
+        dst += nxy;
     }
-}
-
-// The four levels of a tile, coarsest first.
-template <typename T, int M, bool IN>
-__device__ __forceinline__ void tile_levels(Ctx<T, IN>& t, const LevelEb<T>& le, const uint8_t (&fl)[8], int maxlevel) {
-    if (3 <= maxlevel) { t.eb_r = le.eb_r[3]; t.ebx2 = le.ebx2[3]; level<T, 8, M>(t, fl[3], fl[7]); }
-    if (2 <= maxlevel) { t.eb_r = le.eb_r[2]; t.ebx2 = le.ebx2[2]; level<T, 4, M>(t, fl[2], fl[6]); }
-    if (1 <= maxlevel) { t.eb_r = le.eb_r[1]; t.ebx2 = le.ebx2[1]; level<T, 2, M>(t, fl[1], fl[5]); }
-    if (0 <= maxlevel) { t.eb_r = le.eb_r[0]; t.ebx2 = le.ebx2[0]; level<T, 1, M>(t, fl[0], fl[4]); }
 }
 
 // One tile: compress (load, predict, quantise, store codes) or decompress
@@ -1245,12 +687,9 @@ enum CodeSrc { CODES_32, CODES_16, CODES_PLANES };
 // previous values' loads are unconditional in interior tiles and the code
 // slots wait for the code loads alone
 template <typename T, int M, bool IN, int CS = CODES_32, bool DELTA = false>
-__device__ __forceinline__ void tile_run(const SplineArgs<T>& a, T* tile, int32_t* rowtab, int bx, int by, int bz) {
+__device__ __forceinline__ void tile_run(const SplineArgs<T>& a, T* tile, int bx, int by, int bz) {
     const Geom& g = a.g;
-    Ctx<T, IN> t = tile_ctx<T, IN>(a, tile, bx, by, bz, CS == CODES_16);
-    uint8_t fl[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) fl[i] = a.flags8[i];
+    Tile<T, IN> t = make_tile<T, IN>(g, tile, bx, by, bz, a.qc_out);
     const int maxlevel = a.d_maxlevel ? *a.d_maxlevel : 4;
 
     // decompression: every code of the tile and the previous reconstruction
@@ -1259,7 +698,7 @@ __device__ __forceinline__ void tile_run(const SplineArgs<T>& a, T* tile, int32_
     // previous values (needed only at the output) are still in flight
     T prev[kOutIters];
     if constexpr (M == COMPRESS) {
-        load_tile(t, a.data);
+        tile_load(t, a.data);
         __syncthreads();
         if (threadIdx.x == 0) a.anchors[bx + (int64_t)by * g.gx + (int64_t)bz * g.gx * g.gy] = tile[0];
     } else {
@@ -1267,10 +706,6 @@ __device__ __forceinline__ void tile_run(const SplineArgs<T>& a, T* tile, int32_
         // flight ahead of other workgroups' stage arithmetic (reconstruction
         // 1-2 us faster)
         __builtin_amdgcn_s_setprio(3);
-        if constexpr (CS != CODES_PLANES) {  // the plane loads compute their row bases themselves
-            fill_rows(t, rowtab);
-            lds_barrier();
-        }
         if constexpr (CS == CODES_PLANES) {
             PlaneCodes<T> c;
             plane_codes_load(t, a.ps, maxlevel, a.anchors_in, bx, by, bz, c);
@@ -1279,25 +714,27 @@ __device__ __forceinline__ void tile_run(const SplineArgs<T>& a, T* tile, int32_
             plane_codes_store(t, c);
         } else {
             TileCodes<T> c;
-            codes_load(t, rowtab, maxlevel, a.anchors_in, bx, by, bz, c);
+            if constexpr (CS == CODES_16)
+                codes_load(t, reinterpret_cast<const int16_t*>(a.qc_in), maxlevel, a.anchors_in, bx, by, bz, c);
+            else
+                codes_load(t, a.qc_in, maxlevel, a.anchors_in, bx, by, bz, c);
             if constexpr (DELTA) prev_load(t, a.old, prev);
             __builtin_amdgcn_s_setprio(0);
-            codes_store(tile, c);
+            codes_store(t, c);
         }
         __syncthreads();
     }
 
-    tile_levels<T, M>(t, a.le, fl, maxlevel);
+    tile_levels<T, M>(t, a.le, a.flags8, maxlevel);
 
     if constexpr (M == DECOMPRESS) tile_out(t, DELTA, prev, a.out);
 }
 
 // a decompressing tile of either form: delta (a.old given) or anchored
 template <typename T, bool IN, int CS>
-__device__ __forceinline__ void tile_run_dec(const SplineArgs<T>& a, T* tile, int32_t* rowtab, int bx, int by,
-                                             int bz) {
-    if (a.old) tile_run<T, DECOMPRESS, IN, CS, true>(a, tile, rowtab, bx, by, bz);
-    else tile_run<T, DECOMPRESS, IN, CS, false>(a, tile, rowtab, bx, by, bz);
+__device__ __forceinline__ void tile_run_dec(const SplineArgs<T>& a, T* tile, int bx, int by, int bz) {
+    if (a.old) tile_run<T, DECOMPRESS, IN, CS, true>(a, tile, bx, by, bz);
+    else tile_run<T, DECOMPRESS, IN, CS, false>(a, tile, bx, by, bz);
 }
 
 // ------------------------------------------------------------ 2-D fields --
@@ -1346,7 +783,7 @@ __device__ __forceinline__ void plane_stage(Ctx<T>& t, int lane) {
         else pred = pred_face<T, U>(t, x, y, 0);
         T& v = t.s[sidx(x, y, 0)];
         if constexpr (M == COMPRESS) {
-            const int32_t qv = quantize(t, v, pred);
+            const int32_t qv = quantize_val(v, pred, t.eb_r, t.ebx2);
             if (x < 16 && y < 16) t.qc_out[lm_index<LEVEL>(t.g, t.ox + x, t.oy + y, 0)] = qv;
         } else {
             v = pred + (T)slot_code(v) * t.ebx2;
@@ -1501,6 +938,33 @@ __host__ __device__ inline bool plane_field(const Geom& g) { return g.nz == 1 &&
 // the halo point, in registers; a workgroup covers 256 consecutive tiles.
 // Field values, codes and output pass through LDS so that every global
 // access is coalesced.
+enum Stencil { S_KEEP, S_LIN, S_QUAD_R, S_QUAD_L, S_CUBIC };
+
+// Stencil of point j of a line (position c = (2j+1)U along the axis), the
+// rule of InterpolationPredictor.cu:1269-1326 with c2 = (j >= 1) and
+// c3 = (j <= N - 2).
+template <int U>
+__device__ __forceinline__ int stencil_of(int j, int N, bool c1, int o, int nax) {
+    const int gc = o + (2 * j + 1) * U;
+    const bool c2 = j >= 1, c3 = j <= N - 2, c4 = gc + 3 * U < nax, c5 = gc + U < nax;
+    if ((c1 && !c2 && !c3) || (!c1 && !c2 && !(c3 && c4) && c5)) return S_LIN;
+    if ((c1 && !c2 && c3) || (!c1 && !c2 && c3 && c4)) return S_QUAD_R;
+    if ((c1 && c2 && !c3) || (!c1 && c2 && !(c3 && c4) && c5)) return S_QUAD_L;
+    if ((c1 && c2 && c3) || (!c1 && c2 && c3 && c4)) return S_CUBIC;
+    return S_KEEP;
+}
+
+template <typename T>
+__device__ __forceinline__ T apply_stencil(int k, T t0, T t1, T t2, T t3) {
+    switch (k) {
+        case S_LIN: return lin(t1, t2);
+        case S_QUAD_R: return quad_r(t1, t2, t3);
+        case S_QUAD_L: return quad_l(t0, t1, t2);
+        case S_CUBIC: return cubic(t0, t1, t2, t3, false);
+        default: return t1;
+    }
+}
+
 constexpr int kLineTiles = kThreads;             // tiles per workgroup, one per lane
 constexpr int kLinePts = 16 * kLineTiles;        // field points per workgroup
 constexpr int kLineSlots = 17 * kLineTiles + 1;  // staged values: tile l point k at 17 l + k (k < 16)
@@ -1690,8 +1154,7 @@ __host__ __device__ inline bool line_field(const Geom& g) { return g.ny == 1 && 
 // at compile time.
 template <typename T, int M>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void spline_kernel(SplineArgs<T> a) {
-    __shared__ T tile[kTileVals];
-    __shared__ int32_t rowtab[M == DECOMPRESS ? kRowTab : 1];
+    __shared__ T tile[kTileLds];
     clear_gaps<T, M>(a);
     // XCD-aware tile order: workgroups are dealt round-robin to the 8 XCDs,
     // so workgroup b runs on XCD b mod 8; each XCD takes a contiguous range
@@ -1706,20 +1169,20 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     const SplineArgs<T> r = resolve(a);
     if constexpr (M == DECOMPRESS) {
         if (r.planes) {
-            if (interior) tile_run_dec<T, true, CODES_PLANES>(r, tile, rowtab, bx, by, bz);
-            else tile_run_dec<T, false, CODES_PLANES>(r, tile, rowtab, bx, by, bz);
+            if (interior) tile_run_dec<T, true, CODES_PLANES>(r, tile, bx, by, bz);
+            else tile_run_dec<T, false, CODES_PLANES>(r, tile, bx, by, bz);
             return;
         }
         if (r.q16) {
-            if (interior) tile_run_dec<T, true, CODES_16>(r, tile, rowtab, bx, by, bz);
-            else tile_run_dec<T, false, CODES_16>(r, tile, rowtab, bx, by, bz);
+            if (interior) tile_run_dec<T, true, CODES_16>(r, tile, bx, by, bz);
+            else tile_run_dec<T, false, CODES_16>(r, tile, bx, by, bz);
             return;
         }
-        if (interior) tile_run_dec<T, true, CODES_32>(r, tile, rowtab, bx, by, bz);
-        else tile_run_dec<T, false, CODES_32>(r, tile, rowtab, bx, by, bz);
+        if (interior) tile_run_dec<T, true, CODES_32>(r, tile, bx, by, bz);
+        else tile_run_dec<T, false, CODES_32>(r, tile, bx, by, bz);
     } else {
-        if (interior) tile_run<T, M, true>(r, tile, rowtab, bx, by, bz);
-        else tile_run<T, M, false>(r, tile, rowtab, bx, by, bz);
+        if (interior) tile_run<T, M, true>(r, tile, bx, by, bz);
+        else tile_run<T, M, false>(r, tile, bx, by, bz);
     }
 }
 
@@ -1749,18 +1212,18 @@ __device__ __forceinline__ void tune_block(const T* __restrict__ data, const Geo
     // candidate table of auto_tuning_interpolation (pre_compute_att 110-141, 898-962)
     t.natural = cand >= 9 && cand <= 11;
     switch (cand) {
-        case 0: level<T, 8, TUNE>(t, false, false); break;
-        case 1: level<T, 8, TUNE>(t, false, true); break;
-        case 2: level<T, 8, TUNE>(t, true, true); break;
-        case 3: level<T, 4, TUNE>(t, false, false); break;
-        case 4: level<T, 4, TUNE>(t, false, true); break;
-        case 5: level<T, 4, TUNE>(t, true, true); break;
-        case 6: case 9: level<T, 2, TUNE>(t, false, false); break;
-        case 7: case 10: level<T, 2, TUNE>(t, false, true); break;
-        case 8: case 11: level<T, 2, TUNE>(t, true, true); break;
-        case 12: level<T, 1, TUNE>(t, false, false); break;
-        case 13: level<T, 1, TUNE>(t, false, true); break;
-        default: level<T, 1, TUNE>(t, true, true); break;
+        case 0: level<T, 8>(t, false, false); break;
+        case 1: level<T, 8>(t, false, true); break;
+        case 2: level<T, 8>(t, true, true); break;
+        case 3: level<T, 4>(t, false, false); break;
+        case 4: level<T, 4>(t, false, true); break;
+        case 5: level<T, 4>(t, true, true); break;
+        case 6: case 9: level<T, 2>(t, false, false); break;
+        case 7: case 10: level<T, 2>(t, false, true); break;
+        case 8: case 11: level<T, 2>(t, true, true); break;
+        case 12: level<T, 1>(t, false, false); break;
+        case 13: level<T, 1>(t, false, true); break;
+        default: level<T, 1>(t, true, true); break;
     }
     red[threadIdx.x] = t.acc;
     __syncthreads();
@@ -2092,8 +1555,7 @@ template <typename T>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void batch_spline_kernel(
     const BatchField* __restrict__ fields, const int64_t* __restrict__ prefix, int lo, int hi, int64_t base,
     int64_t ntiles, int xcd_order) {
-    __shared__ T tile[kTileVals];
-    __shared__ int32_t rowtab[1];
+    __shared__ T tile[kTileLds];
     const int64_t b = blockIdx.x, xcd = b % kXcds, per = ntiles / kXcds, extra = ntiles % kXcds;
     const int64_t gt = base + (xcd_order ? xcd * per + (xcd < extra ? xcd : extra) + b / kXcds : b);
     const int f = find_field(prefix, lo, hi, gt);
@@ -2112,8 +1574,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     }
     const int bx = (int)(tix % g.gx), by = (int)((tix / g.gx) % g.gy), bz = (int)(tix / ((int64_t)g.gx * g.gy));
     const bool interior = bx * 16 + 16 < g.nx && by * 16 + 16 < g.ny && bz * 16 + 16 < g.nz;
-    if (interior) tile_run<T, COMPRESS, true>(a, tile, rowtab, bx, by, bz);
-    else tile_run<T, COMPRESS, false>(a, tile, rowtab, bx, by, bz);
+    if (interior) tile_run<T, COMPRESS, true>(a, tile, bx, by, bz);
+    else tile_run<T, COMPRESS, false>(a, tile, bx, by, bz);
 }
 
 // Reconstruction units of a batch of retrieval rounds, jobs [lo, hi) (one
@@ -2123,8 +1585,7 @@ template <typename T>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void retr_spline_kernel(
     const RetrJob* __restrict__ jobs, const int64_t* __restrict__ prefix, int lo, int hi, int64_t base,
     int64_t nunits) {
-    __shared__ T tile[kTileVals];
-    __shared__ int32_t rowtab[kRowTab];
+    __shared__ T tile[kTileLds];
     const int64_t b = blockIdx.x, xcd = b % kXcds, per = nunits / kXcds, extra = nunits % kXcds;
     const int64_t gt = base + xcd * per + (xcd < extra ? xcd : extra) + b / kXcds;
     const int j = find_field(prefix, lo, hi, gt);
@@ -2164,17 +1625,17 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     const int bx = (int)(tix % g.gx), by = (int)((tix / g.gx) % g.gy), bz = (int)(tix / ((int64_t)g.gx * g.gy));
     const bool interior = bx * 16 + 16 < g.nx && by * 16 + 16 < g.ny && bz * 16 + 16 < g.nz;
     if (a.planes) {
-        if (interior) tile_run_dec<T, true, CODES_PLANES>(a, tile, rowtab, bx, by, bz);
-        else tile_run_dec<T, false, CODES_PLANES>(a, tile, rowtab, bx, by, bz);
+        if (interior) tile_run_dec<T, true, CODES_PLANES>(a, tile, bx, by, bz);
+        else tile_run_dec<T, false, CODES_PLANES>(a, tile, bx, by, bz);
         return;
     }
     if (a.q16) {
-        if (interior) tile_run_dec<T, true, CODES_16>(a, tile, rowtab, bx, by, bz);
-        else tile_run_dec<T, false, CODES_16>(a, tile, rowtab, bx, by, bz);
+        if (interior) tile_run_dec<T, true, CODES_16>(a, tile, bx, by, bz);
+        else tile_run_dec<T, false, CODES_16>(a, tile, bx, by, bz);
         return;
     }
-    if (interior) tile_run_dec<T, true, CODES_32>(a, tile, rowtab, bx, by, bz);
-    else tile_run_dec<T, false, CODES_32>(a, tile, rowtab, bx, by, bz);
+    if (interior) tile_run_dec<T, true, CODES_32>(a, tile, bx, by, bz);
+    else tile_run_dec<T, false, CODES_32>(a, tile, bx, by, bz);
 }
 
 // ------------------------------------------------------------- host side --
