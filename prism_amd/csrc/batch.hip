@@ -171,7 +171,7 @@ int upload(pa_batch_plan* p, hipStream_t st) {
                                         f.rel ? pa::batch_ext_blocks(&f.L, f.dtype, pa::kExtChoices[3]) : 0,
                                         f.tnblocks,
                                         pa::batch_gap_blocks(f),
-                                        pa::batch_tile_units(&f.L),
+                                        pa::batch_tile_units(&f.L, f.dtype),
                                         pa::batch_shuf_blocks(&f.L),
                                         (f.L.nchunks + 7) / 8 * 8,  // encoder launch slots: whole workgroups
                                         pa::batch_merge_blocks(&f.L, f.dtype)};
@@ -485,7 +485,7 @@ extern "C" int pa_retrieve_batch(const pa_retrieve_job* jobs, int nj, void* h_ta
             if (st != PA_OK) return st;
             j.keys = keys + (size_t)k * 33 * 33;
             p_unshuf[k + 1] = p_unshuf[k] + pa::retr_unshuf_blocks(&j.L);
-            p_unit[k + 1] = p_unit[k] + pa::batch_tile_units(&j.L);
+            p_unit[k + 1] = p_unit[k] + pa::retr_tile_units(&j.L, j.dtype);
             max_chunks += j.L.nchunks;
             nj32 += pass == 0;
             ++k;

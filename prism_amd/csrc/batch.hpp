@@ -16,7 +16,7 @@ struct BatchDev {
     const int64_t* p_ext;    // extrema workgroups
     const int64_t* p_tune;   // tuner sample blocks (x 15 candidates in grid.y)
     const int64_t* p_gap;    // code-gap workgroups
-    const int64_t* p_tile;   // spline work units (a tile; 4 tiles of a 2-D, 256 of a 1-D field)
+    const int64_t* p_tile;   // spline workgroups (a tile; 4 tiles of a 2-D, 256 of a 1-D field)
     const int64_t* p_shuf;   // shuffle workgroups
     const int64_t* p_chunk;  // encoder launch slots (one per wave64): chunks rounded up to a multiple of 8
     const int64_t* p_merge;  // trailer workgroups
@@ -37,7 +37,8 @@ constexpr int kEncodeChoices[3] = {2, 4, 8};   // encode_waves candidates
 int64_t batch_ext_blocks(const pa_layout* L, int dtype, int ext_batches);
 int64_t batch_gap_blocks(const BatchField& f);
 int64_t batch_shuf_blocks(const pa_layout* L);
-int64_t batch_tile_units(const pa_layout* L);  // spline workgroups
+int64_t batch_tile_units(const pa_layout* L, int dtype);  // spline workgroups
+int64_t retr_tile_units(const pa_layout* L, int dtype);   // reconstruction workgroups
 int64_t batch_merge_blocks(const pa_layout* L, int dtype);
 // host-side preparation of a descriptor (layout filled): tuner sampling,
 // alpha, code gaps
@@ -48,7 +49,7 @@ struct RetrDev {
     const RetrJob* jobs;
     int nj, nj32;
     const int64_t* p_unshuf;  // inverse-shuffle workgroups
-    const int64_t* p_unit;    // reconstruction work units
+    const int64_t* p_unit;    // reconstruction workgroups (float32: twice the spline's)
     int64_t* p_chunk;         // selected chunks (device-computed exclusive prefix, nj + 1)
     int64_t n_unshuf, n_unit, n_unit32, max_chunks;
 };

@@ -353,17 +353,11 @@ constexpr int kFill0EdgeIters = (kRows0 + kThreads - 1) / kThreads;  // 2
 template <typename T>
 __device__ __forceinline__ LevelEb<T> load_level_ebs(const double* e) {
     LevelEb<T> le;
-    if constexpr (sizeof(T) == 4) {
-        const float* q = reinterpret_cast<const float*>(e + 10);
-        for (int i = 0; i < 4; ++i) {
-            le.eb_r[i] = q[i];
-            le.ebx2[i] = q[4 + i];
-        }
-    } else {
-        for (int i = 0; i < 4; ++i) {
-            le.eb_r[i] = e[2 + i];
-            le.ebx2[i] = e[6 + i];
-        }
+    const T* q = reinterpret_cast<const T*>(e + (sizeof(T) == 4 ? 10 : 2));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        le.eb_r[i] = scalar_load(q + i);
+        le.ebx2[i] = scalar_load(q + 4 + i);
     }
     return le;
 }
@@ -611,8 +605,8 @@ __device__ __forceinline__ void plane_codes_load(const Tile<T, IN>& t, const Pla
     int we[4];
 #pragma unroll
     for (int lr = 0; lr < 4; ++lr) {
-        c.wb[lr] = ps.begin[lr];
-        we[lr] = ps.end[lr];
+        c.wb[lr] = scalar_load(ps.begin + lr);
+        we[lr] = scalar_load(ps.end + lr);
     }
     const int lane = lane_id();
     constexpr int k1 = kRows0 + kRows1, k2 = k1 + kRows2;
@@ -637,47 +631,44 @@ __device__ __forceinline__ void plane_codes_store(const Tile<T, IN>& t, const Pl
     anchor_store(t, c.anc);
 }
 
-// The previous reconstruction of the tile (delta form); lane: (x, y) =
-// (l mod 16, l / 16), iteration: z.
-constexpr int kOutIters = 4096 / kThreads;
+// The previous reconstruction of the group (delta form): a row lane's column,
+// z = 0..15.
+constexpr int kOutIters = 16;
 template <typename T, bool IN>
-__device__ __forceinline__ void prev_load(const Tile<T, IN>& t, const T* old, T (&prev)[kOutIters]) {
-    const int lane = lane_id();
-    const int x = lane & 15, y = lane >> 4;
-    const bool on = t.template in<0>(x) && t.template in<1>(y);
-    const int64_t nxy = (int64_t)t.g.nx * t.g.ny;
-    const T* src = old + (t.oz * nxy + (int64_t)(t.oy + y) * t.g.nx + t.ox + x);
+__device__ __forceinline__ void prev_load(const Tile<T, IN>& m, const T* old, T (&prev)[kOutIters]) {
+    const RowLane<kGroup<T, DECOMPRESS>> r;
+    const bool on = m.template in<0>(r.X) && m.template in<1>(r.y);
+    const uint32_t nx = (uint32_t)m.g.nx, nxy = nx * (uint32_t)m.g.ny;
+    Column<const T, IN> src(old + ((uint64_t)m.oz * nxy + (uint64_t)m.oy * nx + m.ox), nx, nxy, r.X, r.y);
 #pragma unroll
     for (int z = 0; z < kOutIters; ++z) {
         prev[z] = (T)0;
-        // read once, here only: no cache allocation (reconstruction 158 -> 154 us)
-        if (on && t.template in<2>(z)) prev[z] = __builtin_nontemporal_load(src);
-        src += nxy;
+        if (on && m.template in<2>(z)) prev[z] = src.at();
+        src.next();
     }
 }
 
-// The reconstructed tile (plus the previous one in the delta form) to `out`.
+// The reconstructed group (plus the previous one in the delta form) to `out`.
 template <typename T, bool IN>
-__device__ __forceinline__ void tile_out(const Tile<T, IN>& t, bool delta, const T (&prev)[kOutIters], T* out) {
-    const int lane = lane_id();
-    const int x = lane & 15, y = lane >> 4;
-    if (!(t.template in<0>(x) && t.template in<1>(y))) return;
-    const int64_t nxy = (int64_t)t.g.nx * t.g.ny;
-    const T* src = t.s + tslot(x, y, 0);
-    T* dst = out + (t.oz * nxy + (int64_t)(t.oy + y) * t.g.nx + t.ox + x);
+__device__ __forceinline__ void tile_out(const Tile<T, IN>& m, bool delta, const T (&prev)[kOutIters], T* out) {
+    const RowLane<kGroup<T, DECOMPRESS>> r;
+    if (!(m.template in<0>(r.X) && m.template in<1>(r.y))) return;
+    const uint32_t nx = (uint32_t)m.g.nx, nxy = nx * (uint32_t)m.g.ny;
+    const T* src = m.s + r.slot(r.y, 0);
+    Column<T, IN> dst(out + ((uint64_t)m.oz * nxy + (uint64_t)m.oy * nx + m.ox), nx, nxy, r.X, r.y);
 #pragma unroll
     for (int z = 0; z < kOutIters; ++z) {
-        if (t.template in<2>(z)) {
+        if (m.template in<2>(z)) {
             const T v = src[z * kZP];
             // written once and read only by a later round: no cache allocation
-            __builtin_nontemporal_store(delta ? v + prev[z] : v, dst);
+            __builtin_nontemporal_store(delta ? v + prev[z] : v, &dst.at());
         }
-        dst += nxy;
+        dst.next();
     }
 }
 
-// One tile: compress (load, predict, quantise, store codes) or decompress
-// (fill the code slots, reconstruct, add old, store).
+// One group of tiles: compress (load, predict, quantise, store codes) or
+// decompress (fill the code slots, reconstruct, add old, store).
 // Where a decompressing tile finds its codes (resolved per launch, one
 // kernel body each): int32 or int16 codes of a hand-off array, or the
 // round's decoded bit-planes.
@@ -687,10 +678,15 @@ enum CodeSrc { CODES_32, CODES_16, CODES_PLANES };
 // previous values' loads are unconditional in interior tiles and the code
 // slots wait for the code loads alone
 template <typename T, int M, bool IN, int CS = CODES_32, bool DELTA = false>
-__device__ __forceinline__ void tile_run(const SplineArgs<T>& a, T* tile, int bx, int by, int bz) {
+__device__ __forceinline__ void tile_run(const SplineArgs<T>& a, T* lds, int px, int by, int bz) {
     const Geom& g = a.g;
-    Tile<T, IN> t = make_tile<T, IN>(g, tile, bx, by, bz, a.qc_out);
-    const int maxlevel = a.d_maxlevel ? *a.d_maxlevel : 4;
+    constexpr int P = kGroup<T, M>;
+    // this wave's tile, and the group taken as one tile of 16 P + 1 columns
+    const int h = P == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / kThreads), bx = px * P + h;
+    Tile<T, IN> t = make_tile<T, IN>(g, lds + h * kTileLds, bx, by, bz, a.qc_out);
+    const Tile<T, IN> m = make_tile<T, IN>(g, lds, px * P, by, bz, a.qc_out, 16 * P + 1);
+    const int maxlevel = a.d_maxlevel ? scalar_load(a.d_maxlevel) : 4;
+    const uint32_t fl = flags_load(a.flags8);
 
     // decompression: every code of the tile and the previous reconstruction
     // (delta form) are requested before any is needed, the codes first:
@@ -698,9 +694,9 @@ __device__ __forceinline__ void tile_run(const SplineArgs<T>& a, T* tile, int bx
     // previous values (needed only at the output) are still in flight
     T prev[kOutIters];
     if constexpr (M == COMPRESS) {
-        tile_load(t, a.data);
+        tile_load(t, m, a.data);
         __syncthreads();
-        if (threadIdx.x == 0) a.anchors[bx + (int64_t)by * g.gx + (int64_t)bz * g.gx * g.gy] = tile[0];
+        if (lane_id() == 0 && bx < g.gx) a.anchors[bx + (int64_t)by * g.gx + (int64_t)bz * g.gx * g.gy] = t.s[0];
     } else {
         // a raised wave priority while the tile's loads are issued puts them in
         // flight ahead of other workgroups' stage arithmetic (reconstruction
@@ -709,32 +705,33 @@ __device__ __forceinline__ void tile_run(const SplineArgs<T>& a, T* tile, int bx
         if constexpr (CS == CODES_PLANES) {
             PlaneCodes<T> c;
             plane_codes_load(t, a.ps, maxlevel, a.anchors_in, bx, by, bz, c);
-            if constexpr (DELTA) prev_load(t, a.old, prev);
+            if constexpr (DELTA) prev_load(m, a.old, prev);
             __builtin_amdgcn_s_setprio(0);
             plane_codes_store(t, c);
         } else {
             TileCodes<T> c;
             if constexpr (CS == CODES_16)
-                codes_load(t, reinterpret_cast<const int16_t*>(a.qc_in), maxlevel, a.anchors_in, bx, by, bz, c);
+                codes_load(t, m, reinterpret_cast<const int16_t*>(a.qc_in), maxlevel, a.anchors_in, bx, by, bz, c);
             else
-                codes_load(t, a.qc_in, maxlevel, a.anchors_in, bx, by, bz, c);
-            if constexpr (DELTA) prev_load(t, a.old, prev);
+                codes_load(t, m, a.qc_in, maxlevel, a.anchors_in, bx, by, bz, c);
+            if constexpr (DELTA) prev_load(m, a.old, prev);
             __builtin_amdgcn_s_setprio(0);
-            codes_store(t, c);
+            codes_store(t, m, c);
         }
         __syncthreads();
     }
 
-    tile_levels<T, M>(t, a.le, a.flags8, maxlevel);
+    tile_levels<T, M>(t, a.le, flags_mask(fl), maxlevel);
 
-    if constexpr (M == DECOMPRESS) tile_out(t, DELTA, prev, a.out);
+    if constexpr (M == COMPRESS) codes_out(m);
+    else tile_out(m, DELTA, prev, a.out);
 }
 
 // a decompressing tile of either form: delta (a.old given) or anchored
 template <typename T, bool IN, int CS>
-__device__ __forceinline__ void tile_run_dec(const SplineArgs<T>& a, T* tile, int bx, int by, int bz) {
-    if (a.old) tile_run<T, DECOMPRESS, IN, CS, true>(a, tile, bx, by, bz);
-    else tile_run<T, DECOMPRESS, IN, CS, false>(a, tile, bx, by, bz);
+__device__ __forceinline__ void tile_run_dec(const SplineArgs<T>& a, T* lds, int px, int by, int bz) {
+    if (a.old) tile_run<T, DECOMPRESS, IN, CS, true>(a, lds, px, by, bz);
+    else tile_run<T, DECOMPRESS, IN, CS, false>(a, lds, px, by, bz);
 }
 
 // ------------------------------------------------------------ 2-D fields --
@@ -818,7 +815,7 @@ template <typename T, int M>
 __device__ __forceinline__ void plane_tiles(const SplineArgs<T>& a, T* lds, int64_t unit) {
     const Geom& g = a.g;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int64_t tile = unit * kPlaneWaves + wave;
+    const int64_t tile = unit * (blockDim.x >> 6) + wave;
     if (tile >= (int64_t)g.gx * g.gy) return;  // no workgroup barrier follows
     const int bx = (int)(tile % g.gx), by = (int)(tile / g.gx);
     Ctx<T> t;
@@ -913,7 +910,7 @@ __device__ __forceinline__ SplineArgs<T> resolve(const SplineArgs<T>& a) {
     SplineArgs<T> r = a;
     if (a.le_dev) r.le = load_level_ebs<T>(a.le_dev);
     if (a.narrow) {
-        const int32_t src = *a.narrow;
+        const int32_t src = scalar_load(a.narrow);
         r.q16 = src == 1;
         r.planes = src == 2 && a.ps.bp != nullptr;
     }
@@ -1147,42 +1144,49 @@ __global__ __launch_bounds__(kThreads) void line_kernel(SplineArgs<T> a) {
 
 __host__ __device__ inline bool line_field(const Geom& g) { return g.ny == 1 && g.nz == 1; }
 
+// Waves per SIMD the registers must leave room for: float64, what the LDS
+// allows (4 workgroups of 4 waves per CU); float32, 6 (8 would spill: 512^3
+// compression 469 against 372 us).
+template <typename T>
+constexpr int kTileWaves = sizeof(T) == 4 ? 6 : 4;
+
 // kernel `interpolation` (compress) and `interpolation_reverse` /
 // `interpolation_progressive_reverse` (decompress: anchors, or zero anchors
 // plus old for the delta form).  Tiles away from the far faces of the field
 // (all 17^3 points inside) run a variant whose boundary tests are resolved
 // at compile time.
 template <typename T, int M>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void spline_kernel(SplineArgs<T> a) {
-    __shared__ T tile[kTileLds];
+__global__ __launch_bounds__((kGroupThreads<T, M>)) __attribute__((amdgpu_waves_per_eu(kTileWaves<T>))) void spline_kernel(SplineArgs<T> a) {
+    __shared__ T tile[kGroup<T, M> * kTileLds];
     clear_gaps<T, M>(a);
     // XCD-aware tile order: workgroups are dealt round-robin to the 8 XCDs,
     // so workgroup b runs on XCD b mod 8; each XCD takes a contiguous range
     // of tiles (x fastest) and the cache lines that neighbouring tiles share
     // (halo rows and columns, level-major code runs) meet in one L2.
     const Geom& g = a.g;
-    const int64_t ntiles = (int64_t)g.gx * g.gy * g.gz;
+    const int64_t ntiles = (int64_t)groups_x<kGroup<T, M>>(g) * g.gy * g.gz;
     const int64_t b = blockIdx.x, xcd = b % kXcds, per = ntiles / kXcds, extra = ntiles % kXcds;
     const int64_t tix = xcd * per + (xcd < extra ? xcd : extra) + b / kXcds;
-    const int bx = (int)(tix % g.gx), by = (int)((tix / g.gx) % g.gy), bz = (int)(tix / ((int64_t)g.gx * g.gy));
-    const bool interior = bx * 16 + 16 < g.nx && by * 16 + 16 < g.ny && bz * 16 + 16 < g.nz;
+    const int gpx = groups_x<kGroup<T, M>>(g);
+    const int px = (int)(tix % gpx), by = (int)((tix / gpx) % g.gy), bz = (int)(tix / ((int64_t)gpx * g.gy));
+    const bool interior = interior_group<kGroup<T, M>>(g, px, by, bz);
     const SplineArgs<T> r = resolve(a);
     if constexpr (M == DECOMPRESS) {
         if (r.planes) {
-            if (interior) tile_run_dec<T, true, CODES_PLANES>(r, tile, bx, by, bz);
-            else tile_run_dec<T, false, CODES_PLANES>(r, tile, bx, by, bz);
+            if (interior) tile_run_dec<T, true, CODES_PLANES>(r, tile, px, by, bz);
+            else tile_run_dec<T, false, CODES_PLANES>(r, tile, px, by, bz);
             return;
         }
         if (r.q16) {
-            if (interior) tile_run_dec<T, true, CODES_16>(r, tile, bx, by, bz);
-            else tile_run_dec<T, false, CODES_16>(r, tile, bx, by, bz);
+            if (interior) tile_run_dec<T, true, CODES_16>(r, tile, px, by, bz);
+            else tile_run_dec<T, false, CODES_16>(r, tile, px, by, bz);
             return;
         }
-        if (interior) tile_run_dec<T, true, CODES_32>(r, tile, bx, by, bz);
-        else tile_run_dec<T, false, CODES_32>(r, tile, bx, by, bz);
+        if (interior) tile_run_dec<T, true, CODES_32>(r, tile, px, by, bz);
+        else tile_run_dec<T, false, CODES_32>(r, tile, px, by, bz);
     } else {
-        if (interior) tile_run<T, M, true>(r, tile, bx, by, bz);
-        else tile_run<T, M, false>(r, tile, bx, by, bz);
+        if (interior) tile_run<T, M, true>(r, tile, px, by, bz);
+        else tile_run<T, M, false>(r, tile, px, by, bz);
     }
 }
 
@@ -1552,10 +1556,10 @@ __global__ void batch_keys_init_kernel(BatchField* fields, int nf) {
 // order of spline_kernel taken over the concatenated list of work units: a
 // tile, 4 tiles of a 2-D field or 256 tiles of a 1-D field.
 template <typename T>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void batch_spline_kernel(
+__global__ __launch_bounds__((kGroupThreads<T, COMPRESS>)) __attribute__((amdgpu_waves_per_eu(kTileWaves<T>))) void batch_spline_kernel(
     const BatchField* __restrict__ fields, const int64_t* __restrict__ prefix, int lo, int hi, int64_t base,
     int64_t ntiles, int xcd_order) {
-    __shared__ T tile[kTileLds];
+    __shared__ T tile[kGroup<T, COMPRESS> * kTileLds];
     const int64_t b = blockIdx.x, xcd = b % kXcds, per = ntiles / kXcds, extra = ntiles % kXcds;
     const int64_t gt = base + (xcd_order ? xcd * per + (xcd < extra ? xcd : extra) + b / kXcds : b);
     const int f = find_field(prefix, lo, hi, gt);
@@ -1564,28 +1568,30 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                           F.flags, nullptr, F.qc, nullptr, static_cast<T*>(F.anchors), nullptr, nullptr, nullptr};
     const Geom& g = a.g;
     const int64_t tix = gt - prefix[f];
-    if (line_field(g)) {
-        line_tiles<T, COMPRESS>(a, tile, tix);
+    if (line_field(g)) {  // one unit per 256 lanes
+        const int h = threadIdx.x / kThreads;
+        line_tiles<T, COMPRESS>(a, tile + h * kLineSlots, tix * kGroup<T, COMPRESS> + h);
         return;
     }
     if (plane_field(g)) {
         plane_tiles<T, COMPRESS>(a, tile, tix);
         return;
     }
-    const int bx = (int)(tix % g.gx), by = (int)((tix / g.gx) % g.gy), bz = (int)(tix / ((int64_t)g.gx * g.gy));
-    const bool interior = bx * 16 + 16 < g.nx && by * 16 + 16 < g.ny && bz * 16 + 16 < g.nz;
-    if (interior) tile_run<T, COMPRESS, true>(a, tile, bx, by, bz);
-    else tile_run<T, COMPRESS, false>(a, tile, bx, by, bz);
+    const int gpx = groups_x<kGroup<T, COMPRESS>>(g);
+    const int px = (int)(tix % gpx), by = (int)((tix / gpx) % g.gy), bz = (int)(tix / ((int64_t)gpx * g.gy));
+    const bool interior = interior_group<kGroup<T, COMPRESS>>(g, px, by, bz);
+    if (interior) tile_run<T, COMPRESS, true>(a, tile, px, by, bz);
+    else tile_run<T, COMPRESS, false>(a, tile, px, by, bz);
 }
 
 // Reconstruction units of a batch of retrieval rounds, jobs [lo, hi) (one
 // dtype): the anchored form on a field's first round, the delta form on old
 // after that; levels above the round's maxlevel are skipped.
 template <typename T>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void retr_spline_kernel(
+__global__ __launch_bounds__((kGroupThreads<T, DECOMPRESS>)) __attribute__((amdgpu_waves_per_eu(kTileWaves<T>))) void retr_spline_kernel(
     const RetrJob* __restrict__ jobs, const int64_t* __restrict__ prefix, int lo, int hi, int64_t base,
     int64_t nunits) {
-    __shared__ T tile[kTileLds];
+    __shared__ T tile[kGroup<T, DECOMPRESS> * kTileLds];
     const int64_t b = blockIdx.x, xcd = b % kXcds, per = nunits / kXcds, extra = nunits % kXcds;
     const int64_t gt = base + xcd * per + (xcd < extra ? xcd : extra) + b / kXcds;
     const int j = find_field(prefix, lo, hi, gt);
@@ -1597,7 +1603,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
         le.ebx2[i] = sizeof(T) == 4 ? (T)J.le32[4 + i] : (T)J.le64[4 + i];
     }
     // the round's code source: 0 int32 or 1 int16 codes in qc, 2 the planes
-    const int32_t src = J.state[9];
+    const int32_t src = scalar_load(J.state + 9);
     SplineArgs<T> a{nullptr, J.g, le, nullptr, nullptr, src == 1, J.flags, J.state + 8, nullptr, J.qc, nullptr,
                     J.first ? static_cast<const T*>(J.anchors) : nullptr,
                     J.first ? nullptr : static_cast<const T*>(J.old), static_cast<T*>(J.out)};
@@ -1614,28 +1620,30 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     }
     const Geom& g = a.g;
     const int64_t tix = gt - prefix[j];
-    if (line_field(g)) {
-        line_tiles<T, DECOMPRESS>(a, tile, tix);
+    if (line_field(g)) {  // one unit per 256 lanes
+        const int h = threadIdx.x / kThreads;
+        line_tiles<T, DECOMPRESS>(a, tile + h * kLineSlots, tix * kGroup<T, DECOMPRESS> + h);
         return;
     }
     if (plane_field(g)) {
         plane_tiles<T, DECOMPRESS>(a, tile, tix);
         return;
     }
-    const int bx = (int)(tix % g.gx), by = (int)((tix / g.gx) % g.gy), bz = (int)(tix / ((int64_t)g.gx * g.gy));
-    const bool interior = bx * 16 + 16 < g.nx && by * 16 + 16 < g.ny && bz * 16 + 16 < g.nz;
+    const int gpx = groups_x<kGroup<T, DECOMPRESS>>(g);
+    const int px = (int)(tix % gpx), by = (int)((tix / gpx) % g.gy), bz = (int)(tix / ((int64_t)gpx * g.gy));
+    const bool interior = interior_group<kGroup<T, DECOMPRESS>>(g, px, by, bz);
     if (a.planes) {
-        if (interior) tile_run_dec<T, true, CODES_PLANES>(a, tile, bx, by, bz);
-        else tile_run_dec<T, false, CODES_PLANES>(a, tile, bx, by, bz);
+        if (interior) tile_run_dec<T, true, CODES_PLANES>(a, tile, px, by, bz);
+        else tile_run_dec<T, false, CODES_PLANES>(a, tile, px, by, bz);
         return;
     }
     if (a.q16) {
-        if (interior) tile_run_dec<T, true, CODES_16>(a, tile, bx, by, bz);
-        else tile_run_dec<T, false, CODES_16>(a, tile, bx, by, bz);
+        if (interior) tile_run_dec<T, true, CODES_16>(a, tile, px, by, bz);
+        else tile_run_dec<T, false, CODES_16>(a, tile, px, by, bz);
         return;
     }
-    if (interior) tile_run_dec<T, true, CODES_32>(a, tile, bx, by, bz);
-    else tile_run_dec<T, false, CODES_32>(a, tile, bx, by, bz);
+    if (interior) tile_run_dec<T, true, CODES_32>(a, tile, px, by, bz);
+    else tile_run_dec<T, false, CODES_32>(a, tile, px, by, bz);
 }
 
 // ------------------------------------------------------------- host side --
@@ -1682,7 +1690,8 @@ int launch_spline(const pa_layout* L, const T* data, double eb, double rel_eb, c
         hipLaunchKernelGGL((plane_kernel<T, M>), dim3((unsigned)((ntiles + kPlaneWaves - 1) / kPlaneWaves)),
                            dim3(kThreads), 0, st, args);
     else
-        hipLaunchKernelGGL((spline_kernel<T, M>), dim3((unsigned)ntiles), dim3(kThreads), 0, st, args);
+        hipLaunchKernelGGL((spline_kernel<T, M>), dim3((unsigned)(groups_x<kGroup<T, M>>(g) * ((int64_t)g.gy * g.gz))),
+                           dim3(kGroupThreads<T, M>), 0, st, args);
     PA_LAUNCH_CHECK();
     return PA_OK;
 }
@@ -1956,7 +1965,7 @@ int pa::batch_keys_init(const BatchDev& b, hipStream_t st) {
 
 int pa::batch_spline(const BatchDev& b, hipStream_t st) {
     if (b.n_tile32 > 0) {
-        hipLaunchKernelGGL(batch_spline_kernel<float>, dim3((unsigned)b.n_tile32), dim3(kThreads), 0, st, b.fields,
+        hipLaunchKernelGGL(batch_spline_kernel<float>, dim3((unsigned)b.n_tile32), dim3(kGroupThreads<float, COMPRESS>), 0, st, b.fields,
                            b.p_tile, 0, b.nf32, (int64_t)0, b.n_tile32, b.xcd_order);
         PA_LAUNCH_CHECK();
     }
@@ -1968,12 +1977,22 @@ int pa::batch_spline(const BatchDev& b, hipStream_t st) {
     return PA_OK;
 }
 
-int64_t pa::batch_tile_units(const pa_layout* L) {
+// workgroups of the batched spline launches for one field
+template <int P>
+static int64_t spline_units(const pa_layout* L) {
     const Geom g = make_geom(L);
     const int64_t ntiles = (int64_t)g.gx * g.gy * g.gz;
-    if (line_field(g)) return (ntiles + kLineTiles - 1) / kLineTiles;
-    if (plane_field(g)) return (ntiles + kPlaneWaves - 1) / kPlaneWaves;
-    return ntiles;
+    const int per = P * (line_field(g) ? kLineTiles : kPlaneWaves);
+    if (line_field(g) || plane_field(g)) return (ntiles + per - 1) / per;
+    return (int64_t)groups_x<P>(g) * g.gy * g.gz;
+}
+
+int64_t pa::batch_tile_units(const pa_layout* L, int dtype) {
+    return dtype == PA_F32 ? spline_units<kGroup<float, COMPRESS>>(L) : spline_units<kGroup<double, COMPRESS>>(L);
+}
+
+int64_t pa::retr_tile_units(const pa_layout* L, int dtype) {
+    return dtype == PA_F32 ? spline_units<kGroup<float, DECOMPRESS>>(L) : spline_units<kGroup<double, DECOMPRESS>>(L);
 }
 
 void pa::retr_level_ebs(RetrJob& j, double eb, double rel_eb) {
@@ -1989,7 +2008,7 @@ void pa::retr_level_ebs(RetrJob& j, double eb, double rel_eb) {
 
 int pa::retr_reconstruct(const RetrDev& r, hipStream_t st) {
     if (r.n_unit32 > 0) {
-        hipLaunchKernelGGL(retr_spline_kernel<float>, dim3((unsigned)r.n_unit32), dim3(kThreads), 0, st, r.jobs,
+        hipLaunchKernelGGL(retr_spline_kernel<float>, dim3((unsigned)r.n_unit32), dim3(kGroupThreads<float, DECOMPRESS>), 0, st, r.jobs,
                            r.p_unit, 0, r.nj32, (int64_t)0, r.n_unit32);
         PA_LAUNCH_CHECK();
     }

@@ -43,8 +43,21 @@ constexpr int slot_half() {
     return A == 0 ? U : (A == 1 ? (U == 1 ? kYO : U / 2 * kYP) : U * kZP);
 }
 
+// A workgroup holds kGroup tiles adjacent along x, 256 lanes each.  A float32
+// tile's rows are 64 bytes, half a cache line: a copy of a 512^3 float32 field
+// in the tiles' access pattern (halo included) takes 322 us, 248 us in pairs
+// (258 us in fours).  Decompression, which is bound by its accesses, takes
+// pairs (round 4 of that field 287 us against 319 us one by one); compression,
+// which is bound by its stages, is faster with 256-lane workgroups (342
+// against 372 us: half as many waves meet at each of its 13 barriers).
+template <typename T, int M>
+constexpr int kGroup = sizeof(T) == 4 && M == DECOMPRESS ? 2 : 1;
+template <typename T, int M>
+constexpr int kGroupThreads = kGroup<T, M> * kThreads;
+
 // IN: not the last tile along any axis, all 17^3 points inside the field
-// (every stencil then is decided at compile time).  rx, ry, rz: points of the
+// (every stencil then is decided at compile time), and rows short enough for
+// 32-bit offsets.  rx, ry, rz: points of the
 // tile inside the field along each axis, halo included (17: not the last).
 template <typename T, bool IN>
 struct Tile {
@@ -62,20 +75,52 @@ struct Tile {
     __device__ __forceinline__ bool in3(int x, int y, int z) const { return IN || (x < rx && y < ry && z < rz); }
 };
 
+// every tile of group px is such a tile
+template <int P>
+__device__ __forceinline__ bool interior_group(const Geom& g, int px, int by, int bz) {
+    return (px + 1) * (16 * P) < g.nx && by * 16 + 16 < g.ny && bz * 16 + 16 < g.nz && g.nx < (1 << 24);
+}
+
+// groups along x
+template <int P>
+__host__ __device__ inline int groups_x(const Geom& g) {
+    return (g.gx + P - 1) / P;
+}
+
+// width: points along x the tile (or a group of tiles, taken as one) may
+// have.  A group's second tile may lie outside the field (rx <= 0): its
+// lanes then find no point inside.
 template <typename T, bool IN>
-__device__ __forceinline__ Tile<T, IN> make_tile(const Geom& g, T* s, int bx, int by, int bz, int32_t* qc_out) {
+__device__ __forceinline__ Tile<T, IN> make_tile(const Geom& g, T* s, int bx, int by, int bz, int32_t* qc_out,
+                                                 int width = kTS) {
     Tile<T, IN> t;
     t.s = s;
     t.ox = bx * 16;
     t.oy = by * 16;
     t.oz = bz * 16;
-    t.rx = min(g.nx - t.ox, kTS);
+    t.rx = min(g.nx - t.ox, width);
     t.ry = min(g.ny - t.oy, kTS);
     t.rz = min(g.nz - t.oz, kTS);
     t.g = g;
     t.qc_out = qc_out;
     return t;
 }
+
+// Lane of the phases that move rows between memory and the group's tiles:
+// column X = 0 .. 16 P - 1 of the group of P, row y.
+template <int P>
+struct RowLane {
+    int X, y;
+    __device__ __forceinline__ RowLane() {
+        const int v = thread_id();
+        X = v & (16 * P - 1);
+        y = (int)((unsigned)v / (16 * P));
+    }
+    // slot of point (x, y', z') of the lane's column in the group's LDS
+    __device__ __forceinline__ int slot(int yy, int zz) const {
+        return (X >> 4) * kTileLds + tslot(X & 15, yy, zz);
+    }
+};
 
 // ---------------------------------------------------------------- stencils --
 // Point j of a line of N = 8 / U points lies between the known values j and
@@ -97,7 +142,7 @@ __device__ __forceinline__ Rank rank_of(int j, int last) {
 template <typename T, int N, bool IN>
 __device__ __forceinline__ T pred_line(int j, int last, T v0, T v1, T v2, T v3) {
     if constexpr (IN) {
-        if (N == 1) return lin(v1, v2);
+        if (N == 1) return lin(v1, v2);  // (j is a constant)
         return j == 0 ? quad_r(v1, v2, v3) : (j == N - 1 ? quad_l(v0, v1, v2) : cubic(v0, v1, v2, v3));
     } else {
         T p = v1;
@@ -108,24 +153,25 @@ __device__ __forceinline__ T pred_line(int j, int last, T v0, T v1, T v2, T v3) 
 }
 
 // ------------------------------------------------------------------ stages --
-// Where a compressing stage puts its codes: straight to the level-major
-// array (levels 1-3), into registers (the first two stages of level 0, whose
-// values later stages still read), or into the points' own slots (the last
-// stage of level 0).  Level 0's codes then leave the tile as whole rows.
-enum Sink { TO_GLOBAL, TO_REGS, TO_SLOT };
+// Codes of a compressing tile stay in registers with their points' slots
+// until the last stage (whose own codes go straight into its points' slots) is
+// done: no stage reads values after that, every code then joins its slot, and
+// all levels leave the tile as rows.  (Codes of levels 1-3 stored from their
+// stages instead are scattered 4-byte writes, five times the requests, and
+// their index arithmetic lengthens the chain of short stages.)
+template <int N>
 struct RegCodes {
-    int32_t code[8];
-    int slot, step;  // slot of code 0 (-1: none to store), distance of the slots
+    int32_t code[N];
+    int slot, step;  // slot of code 0 (-1: none), distance of the slots
+    __device__ __forceinline__ RegCodes() : slot(-1), step(0) {}
 };
 
-// Level-major index step from point j of a line along A to point j + 1 (the
-// coordinate keeps its parity); y, z: the line's fixed coordinates.
-template <int L, int A, typename T, bool IN>
-__device__ __forceinline__ uint32_t lm_step(const Tile<T, IN>& t, int y, int z) {
-    if constexpr (A == 0) return (((y | z) >> L) & 1) ? 2u : 1u;
-    if constexpr (A == 1)
-        return 2u * (uint32_t)t.g.lx[L] - (((z >> L) & 1) ? 0u : (uint32_t)t.g.lx[L + 1]);
-    return 2u * (uint32_t)t.g.lxy[L] - (uint32_t)t.g.lxy[L + 1];
+template <int N, typename T>
+__device__ __forceinline__ void join_slots(T* s, const RegCodes<N>& r) {
+    if (r.slot >= 0) {
+#pragma unroll
+        for (int k = 0; k < N; ++k) s[r.slot + k * r.step] = code_slot(r.code[k], T());
+    }
 }
 
 template <int L, typename T, bool IN>
@@ -133,183 +179,264 @@ __device__ __forceinline__ uint32_t lm_at(const Tile<T, IN>& t, int x, int y, in
     return lm_index<L>(t.g, t.ox + x, t.oy + y, t.oz + z);
 }
 
+// Levels 1-3 have few points, and the chain of their nine stages is bound by
+// its length in instructions: there a lane takes a part of a line, kPart points
+// (of the 4, 2 or 1 of its level), instead of all of it.
 template <int U>
-constexpr int level_of_unit() {
-    return U == 1 ? 0 : (U == 2 ? 1 : (U == 4 ? 2 : 3));
+constexpr int kPart = U == 1 ? 8 : (U == 2 ? 2 : 1);
+template <int U>
+constexpr int kParts = 8 / U / kPart<U>;  // 1, 2, 2, 1 per line
+
+// The wave that takes a stage's first 64 lanes.  The coarse levels' stages
+// keep one to three of the four waves busy: they are dealt so that no lane
+// would have to hold codes of two stages in one of its level's registers (see
+// level3), and the waves' work evens out.
+template <int U, int STAGE, bool MD>
+constexpr int stage_wave() {
+    if (U == 1) return 0;
+    if (U == 2) return MD ? (STAGE == 1 ? 2 : 0) : (STAGE == 0 ? 0 : (STAGE == 1 ? 2 : 1));
+    return STAGE;
 }
 
 // One point: its slot's value (or code) against pred.
-template <typename T, int M, int SINK, bool IN>
+template <typename T, int M, bool LAST, bool IN>
 __device__ __forceinline__ void put_point(Tile<T, IN>& t, int slot, T v, T pred, int32_t& code) {
     if constexpr (M == COMPRESS) {
         code = quantize_val(v, pred, t.eb_r, t.ebx2);
-        t.s[slot] = SINK == TO_SLOT ? code_slot(code, T()) : v;
+        t.s[slot] = LAST ? code_slot(code, T()) : v;
     } else {
         t.s[slot] = pred + (T)slot_code(v) * t.ebx2;
     }
 }
 
-// The N points of one line per lane: known values at slots base + j * step,
-// points at base + half + j * step (step and half: compile-time constants,
-// or per-lane values where the lanes' lines differ in direction).
-template <typename T, int U, int M, int SINK, bool IN, class Step, class Half>
-__device__ __forceinline__ void line_points(Tile<T, IN>& t, int base, Step step, Half half, int r, bool own,
-                                            uint32_t idx, uint32_t idx_step, RegCodes* rc) {
+// Part h of a line per lane (all of it at level 0): known values at slots base
+// + j * step, points at base + half + j * step (step and half: compile-time
+// constants, or per-lane values where the lanes' lines differ in direction).
+// A part of level 1 is one end of its line: the point at the end and the one
+// next to it, which has four known values around it (w0 .. w3, from known
+// value h on).
+template <typename T, int U, int M, bool LAST, bool IN, class Step, class Half>
+__device__ __forceinline__ void line_points(Tile<T, IN>& t, int base, Step step, Half half, int r, int h,
+                                            RegCodes<kPart<U>>& rc) {
     constexpr int N = 8 / U;
     const int last = (int)((unsigned)(r - 1) / (2 * U));
-    T k[N + 1], v[N];
+    if constexpr (U == 1) {
+        T k[N + 1], v[N];
 #pragma unroll
-    for (int j = 0; j <= N; ++j) k[j] = t.s[base + j * step];
+        for (int j = 0; j <= N; ++j) k[j] = t.s[base + j * step];
 #pragma unroll
-    for (int j = 0; j < N; ++j) v[j] = t.s[base + half + j * step];
+        for (int j = 0; j < N; ++j) v[j] = t.s[base + half + j * step];
 #pragma unroll
-    for (int j = 0; j < N; ++j) {
-        const T pred = pred_line<T, N, IN>(j, last, k[j > 0 ? j - 1 : 0], k[j], k[j + 1], k[j + 2 <= N ? j + 2 : N]);
-        int32_t code;
-        put_point<T, M, SINK>(t, base + half + j * step, v[j], pred, code);
-        if constexpr (M == COMPRESS && SINK == TO_GLOBAL) {
-            if (own && (IN || (2 * j + 1) * U < r)) t.qc_out[idx + j * idx_step] = code;
+        for (int j = 0; j < N; ++j) {
+            const T pred = pred_line<T, N, IN>(j, last, k[j > 0 ? j - 1 : 0], k[j], k[j + 1], k[j + 2 <= N ? j + 2 : N]);
+            int32_t code = 0;
+            put_point<T, M, LAST>(t, base + half + j * step, v[j], pred, code);
+            if constexpr (M == COMPRESS && !LAST) rc.code[j] = code;
         }
-        if constexpr (M == COMPRESS && SINK == TO_REGS) rc->code[j] = code;
-    }
-    if constexpr (M == COMPRESS && SINK == TO_REGS) {
-        rc->slot = own ? base + half : -1;
-        rc->step = step;
+        if constexpr (!LAST) {  // (the last stage leaves the first one's codes alone)
+            rc.slot = base + half;
+            rc.step = step;
+        }
+    } else if constexpr (U == 2) {
+        const int w = base + h * step, inner = base + half + (1 + h) * step, end = base + half + 3 * h * step;
+        const T w0 = t.s[w], w1 = t.s[w + step], w2 = t.s[w + 2 * step], w3 = t.s[w + 3 * step];
+        const T vi = t.s[inner], ve = t.s[end];
+        T pi, pe;
+        if constexpr (IN) {
+            const T qr = quad_r(w0, w1, w2), ql = quad_l(w1, w2, w3);
+            pi = cubic(w0, w1, w2, w3);
+            pe = h == 0 ? qr : ql;
+        } else {
+            pi = pred_line<T, N, false>(1 + h, last, w0, w1, w2, w3);
+            pe = pred_line<T, N, false>(3 * h, last, w1, h == 0 ? w0 : w2, h == 0 ? w1 : w3, w2);
+        }
+        int32_t ci = 0, ce = 0;
+        put_point<T, M, LAST>(t, inner, vi, pi, ci);
+        put_point<T, M, LAST>(t, end, ve, pe, ce);
+        if constexpr (M == COMPRESS) {
+            rc.code[0] = ci;
+            rc.code[1] = ce;
+        }
+        rc.slot = inner;
+        rc.step = end - inner;
+    } else {
+        const T w0 = t.s[base], w1 = t.s[base + step], w2 = t.s[base + (N == 2 ? 2 : 1) * step];
+        const int slot = base + half + h * step;
+        const T v = t.s[slot];
+        T pred;
+        if constexpr (N == 1) {
+            pred = pred_line<T, 1, IN>(0, last, w0, w0, w1, w1);
+        } else if constexpr (IN) {
+            const T qr = quad_r(w0, w1, w2), ql = quad_l(w0, w1, w2);
+            pred = h == 0 ? qr : ql;
+        } else {
+            pred = pred_line<T, 2, false>(h, last, w0, h == 0 ? w0 : w1, h == 0 ? w1 : w2, w2);
+        }
+        put_point<T, M, LAST>(t, slot, v, pred, rc.code[0]);
+        rc.slot = slot;
     }
 }
 
 // A 1-D stage: lines along A over the other two axes, P (the lower) fastest;
-// ALLP / ALLQ: at every multiple of U, or at the even ones.  EXCL: the last
+// ALLP / ALLQ: at every multiple of U, or at the even ones.  LAST: the last
 // stage of level 0, own points only (x, y, z < 16).
-template <typename T, int U, int A, bool ALLP, bool ALLQ, bool EXCL, int M, int SINK, bool IN>
-__device__ __forceinline__ void line_stage(Tile<T, IN>& t, RegCodes* rc = nullptr) {
-    constexpr int N = 8 / U, L = level_of_unit<U>();
-    constexpr int CP = EXCL ? 16 : (ALLP ? 2 * N + 1 : N + 1), CQ = EXCL ? 16 : (ALLQ ? 2 * N + 1 : N + 1);
-    static_assert(CP * CQ <= kThreads, "one line per lane");
-    if constexpr (M == COMPRESS && SINK == TO_REGS) rc->slot = -1;
-    const int l = lane_id();
-    if (l < CP * CQ) {
-        const int p = (l % CP) * (ALLP ? U : 2 * U), q = (l / CP) * (ALLQ ? U : 2 * U);
+template <typename T, int U, int STAGE, int A, bool ALLP, bool ALLQ, int M, bool IN>
+__device__ __forceinline__ void line_stage(Tile<T, IN>& t, RegCodes<kPart<U>>& rc) {
+    constexpr int N = 8 / U;
+    constexpr bool LAST = U == 1 && STAGE == 2;
+    constexpr int CP = LAST ? 16 : (ALLP ? 2 * N + 1 : N + 1), CQ = LAST ? 16 : (ALLQ ? 2 * N + 1 : N + 1);
+    static_assert(kParts<U> * CP * CQ <= kThreads, "one part of a line per lane");
+    const int l = lane_id(stage_wave<U, STAGE, false>());
+    if (l < kParts<U> * CP * CQ) {
+        const int h = kParts<U> == 1 ? 0 : l / (CP * CQ), m = l - h * (CP * CQ);
+        const int p = (m % CP) * (ALLP ? U : 2 * U), q = (m / CP) * (ALLQ ? U : 2 * U);
         const int x = A == 0 ? 0 : p, y = A == 1 ? 0 : (A == 0 ? p : q), z = A == 2 ? 0 : q;
-        if (t.template in<A == 0 ? 1 : 0>(p) && t.template in<A == 2 ? 1 : 2>(q)) {
-            const bool own = p < 16 && q < 16;
-            uint32_t idx = 0, idx_step = 0;
-            if constexpr (M == COMPRESS && SINK == TO_GLOBAL) {
-                idx = lm_at<L>(t, A == 0 ? U : x, A == 1 ? U : y, A == 2 ? U : z);
-                idx_step = lm_step<L, A>(t, y, z);
-            }
-            line_points<T, U, M, SINK>(t, tslot(x, y, z), std::integral_constant<int, slot_step<U, A>()>{},
+        if (t.template in<A == 0 ? 1 : 0>(p) && t.template in<A == 2 ? 1 : 2>(q))
+            line_points<T, U, M, LAST>(t, tslot(x, y, z), std::integral_constant<int, slot_step<U, A>()>{},
                                        std::integral_constant<int, slot_half<U, A>()>{},
-                                       A == 0 ? t.rx : (A == 1 ? t.ry : t.rz), own, idx, idx_step, rc);
-        }
+                                       A == 0 ? t.rx : (A == 1 ? t.ry : t.rz), h, rc);
     }
     lds_barrier();
 }
 
 // LINE points (one odd coordinate): the lines along x, y and z through the
 // points with both other coordinates even, in one sweep.
-template <typename T, int U, int M, int SINK, bool IN>
-__device__ __forceinline__ void lines3_stage(Tile<T, IN>& t, RegCodes* rc = nullptr) {
-    constexpr int N = 8 / U, C = N + 1, L = level_of_unit<U>();
-    static_assert(3 * C * C <= kThreads, "one line per lane");
-    if constexpr (M == COMPRESS && SINK == TO_REGS) rc->slot = -1;
-    const int l = lane_id();
-    if (l < 3 * C * C) {
-        const int grp = l / (C * C), m = l % (C * C), i = 2 * U * (m % C), j = 2 * U * (m / C);
+template <typename T, int U, int M, bool IN>
+__device__ __forceinline__ void lines3_stage(Tile<T, IN>& t, RegCodes<kPart<U>>& rc) {
+    constexpr int N = 8 / U, C = N + 1, LINES = 3 * C * C;
+    static_assert(kParts<U> * LINES <= kThreads, "one part of a line per lane");
+    const int l = lane_id(stage_wave<U, 0, true>());
+    if (l < kParts<U> * LINES) {
+        const int h = kParts<U> == 1 ? 0 : (l >= LINES ? 1 : 0), ln = l - h * LINES;
+        const int grp = ln / (C * C), m = ln % (C * C), i = 2 * U * (m % C), j = 2 * U * (m / C);
         const int x = grp == 0 ? 0 : i, y = grp == 0 ? i : (grp == 1 ? 0 : j), z = grp == 2 ? 0 : j;
         if (t.in3(x, y, z)) {
             const int step = grp == 0 ? slot_step<U, 0>() : (grp == 1 ? slot_step<U, 1>() : slot_step<U, 2>());
             const int half = grp == 0 ? slot_half<U, 0>() : (grp == 1 ? slot_half<U, 1>() : slot_half<U, 2>());
-            const int r = grp == 0 ? t.rx : (grp == 1 ? t.ry : t.rz);
-            uint32_t idx = 0, idx_step = 0;
-            if constexpr (M == COMPRESS && SINK == TO_GLOBAL) {
-                idx = lm_at<L>(t, grp == 0 ? U : x, grp == 1 ? U : y, grp == 2 ? U : z);
-                idx_step = grp == 0 ? lm_step<L, 0>(t, 0, 0) : (grp == 1 ? lm_step<L, 1>(t, 0, 0) : lm_step<L, 2>(t, 0, 0));
-            }
-            line_points<T, U, M, SINK>(t, tslot(x, y, z), step, half, r, i < 16 && j < 16, idx, idx_step, rc);
+            line_points<T, U, M, false>(t, tslot(x, y, z), step, half, grp == 0 ? t.rx : (grp == 1 ? t.ry : t.rz), h, rc);
         }
     }
     lds_barrier();
 }
 
-// FACE points (two odd coordinates, InterpolationPredictor.cu:1546-1669): a
-// lane takes a line of N points along A (z, or y for the points with even
-// z) at one odd position jb of the other odd axis B.  The two directions'
-// formulas compete by rank: equal ranks are averaged, the higher one wins,
-// and where neither has a far neighbour the point continues the plane
-// through its three known neighbours.
-template <typename T, int U, int M, int SINK, bool IN>
-__device__ __forceinline__ void faces_stage(Tile<T, IN>& t, RegCodes* rc = nullptr) {
-    constexpr int N = 8 / U, C = N + 1, L = level_of_unit<U>();
-    static_assert(3 * N * C <= kThreads, "one line per lane");
-    if constexpr (M == COMPRESS && SINK == TO_REGS) rc->slot = -1;
-    const int l = lane_id();
-    if (l < 3 * N * C) {
-        // groups: (y, z) odd at even x; (x, z) odd at even y; (x, y) odd at even z
-        const int grp = l / (N * C), m = l % (N * C);
-        const int jb = grp == 1 ? m % N : m / C, ic = grp == 1 ? m / N : m % C;
-        const int c = 2 * U * ic, b = 2 * U * jb;  // even axis; left neighbour along B
+// The prediction of a point from its two directions: the formulas compete by
+// rank (InterpolationPredictor.cu:1546-1669): equal ranks are averaged, the
+// higher one wins, and where neither has a far neighbour the point continues
+// the plane through its three known neighbours.  Point ja of a line along
+// one axis with known values a0..a3 around it (last known index lasta), jb
+// and b0..b3 along the other; corner: slot of the known value below both.
+// IN: fa, the rank along A, is a constant.
+template <typename T, int N, bool IN>
+__device__ __forceinline__ T pred_face2(const T* corner, Rank fa, int ja, int lasta, T a0, T a1, T a2, T a3, int jb,
+                                        int lastb, T b0, T b1, T b2, T b3) {
+    const Rank fb = rank_of<N, IN>(jb, lastb);
+    if constexpr (IN) {
+        // every value first, then selections: a branch per lane costs more
+        if (N == 1) return (lin(a1, a2) + lin(b1, b2)) / (T)2;
+        const T ar = quad_r(a1, a2, a3), al = quad_l(a0, a1, a2), br = quad_r(b1, b2, b3), bl = quad_l(b0, b1, b2);
+        const T edge = ((ja == 0 ? ar : al) + (jb == 0 ? br : bl)) / (T)2;
+        if (N == 2) return edge;
+        const T cb = cubic(b0, b1, b2, b3);
+        if (fa != R_CUBIC) return fb == R_CUBIC ? cb : edge;
+        const T ca = cubic(a0, a1, a2, a3), two = (ca + cb) / (T)2;
+        return fb == R_CUBIC ? two : ca;
+    } else {
+        const T pa = pred_line<T, N, false>(ja, lasta, a0, a1, a2, a3);
+        const T pb = pred_line<T, N, false>(jb, lastb, b0, b1, b2, b3);
+        T pred = fa > fb ? pa : pb;
+        if (fa == fb) pred = fa == R_NONE ? (a1 + b1) - *corner : (pa + pb) / (T)2;
+        return pred;
+    }
+}
+
+// FACE points (two odd coordinates): a lane takes a line (or part h of one)
+// along A (z, or y for the points with even z) at one odd position jb of the
+// other odd axis B: the known values of the line are read once, four taps along
+// B per point.
+template <typename T, int U, int M, bool IN>
+__device__ __forceinline__ void faces_stage(Tile<T, IN>& t, RegCodes<kPart<U>>& rc) {
+    constexpr int N = 8 / U, C = N + 1, LINES = 3 * N * C;
+    static_assert(kParts<U> * LINES <= kThreads, "one part of a line per lane");
+    const int l = lane_id(stage_wave<U, 1, true>());
+    if (l < kParts<U> * LINES) {
+        // groups: (y, z) odd at even x, x fastest; (x, z) odd at even y, x
+        // fastest; (x, y) odd at even z, z fastest
+        const int h = kParts<U> == 1 ? 0 : (l >= LINES ? 1 : 0), ln = l - h * LINES;
+        const int grp = ln / (N * C), m = ln - grp * (N * C);
+        const int q = grp == 1 ? m / N : m / C, p = grp == 1 ? m - q * N : m - q * C;
+        const int jb = grp == 1 ? p : q, c = 2 * U * (grp == 1 ? q : p), b = 2 * U * jb;
         const int x = grp == 0 ? c : b, y = grp == 0 ? b : (grp == 1 ? c : 0), z = grp == 2 ? c : 0;
         if (t.in3(grp == 0 ? x : x + U, grp == 1 ? y : y + U, grp == 2 ? z : z + U)) {
             const int sa = grp == 2 ? slot_step<U, 1>() : slot_step<U, 2>();
             const int ha = grp == 2 ? slot_half<U, 1>() : slot_half<U, 2>();
             const int sb = grp == 0 ? slot_step<U, 1>() : slot_step<U, 0>();
             const int hb = grp == 0 ? slot_half<U, 1>() : slot_half<U, 0>();
-            const int left = tslot(x, y, z);  // A and B even
-            const int ka = left + hb;         // A even, B odd: known values along A
-            const int own_slot = ka + ha;     // the points
-            const int p1 = left + ha, p0 = p1 - (jb > 0 ? sb : 0), p2 = p1 + sb, p3 = p2 + (jb < N - 1 ? sb : 0);
+            const T* left = t.s + tslot(x, y, z);  // A and B even
+            const T* ka = left + hb;               // A even, B odd: known values along A
+            const int own = tslot(x, y, z) + hb + ha;  // the points
+            const T *p1 = left + ha, *p0 = p1 - (jb > 0 ? sb : 0), *p2 = p1 + sb, *p3 = p2 + (jb < N - 1 ? sb : 0);
             const int ra = grp == 2 ? t.ry : t.rz, rb = grp == 0 ? t.ry : t.rx;
             const int lasta = (int)((unsigned)(ra - 1) / (2 * U)), lastb = (int)((unsigned)(rb - 1) / (2 * U));
-            const bool own = c < 16;
-            uint32_t idx = 0, idx_step = 0;
-            if constexpr (M == COMPRESS && SINK == TO_GLOBAL) {
-                idx = lm_at<L>(t, grp == 0 ? x : x + U, grp == 1 ? y : y + U, grp == 2 ? z : z + U);
-                idx_step = grp == 2 ? lm_step<L, 1>(t, 0, 0) : lm_step<L, 2>(t, 0, 0);
-            }
-            const bool b3 = jb > 0 && jb + 2 <= N && (IN || lastb >= jb + 2);  // B's formula is the cubic
-            T k[N + 1];
+            if constexpr (U == 1) {
+                T k[N + 1], v[N];
 #pragma unroll
-            for (int j = 0; j <= N; ++j) k[j] = t.s[ka + j * sa];
+                for (int j = 0; j <= N; ++j) k[j] = ka[j * sa];
 #pragma unroll
-            for (int j = 0; j < N; ++j) {
-                const int o = j * sa;
-                const T v0 = t.s[p0 + o], v1 = t.s[p1 + o], v2 = t.s[p2 + o], v3 = t.s[p3 + o];
-                const T a0 = k[j > 0 ? j - 1 : 0], a1 = k[j], a2 = k[j + 1], a3 = k[j + 2 <= N ? j + 2 : N];
-                T pred;
-                if constexpr (IN) {
-                    const T pa = pred_line<T, N, true>(j, N, a0, a1, a2, a3);
-                    if (N == 1) {
-                        pred = (pa + lin(v1, v2)) / (T)2;
-                    } else if (j == 0 || j == N - 1) {
-                        const T qb = jb == 0 ? quad_r(v1, v2, v3) : quad_l(v0, v1, v2);
-                        pred = (pa + qb) / (T)2;
-                        if (N > 2) pred = b3 ? cubic(v0, v1, v2, v3) : pred;
-                    } else {
-                        const T both = (pa + cubic(v0, v1, v2, v3)) / (T)2;
-                        pred = b3 ? both : pa;
+                for (int j = 0; j < N; ++j) v[j] = t.s[own + j * sa];
+                // taps of G points are read together, ahead of the writes of
+                // the points before them
+                constexpr int G = sizeof(T) == 8 ? 2 : 4;
+#pragma unroll
+                for (int j0 = 0; j0 < N; j0 += G) {
+                    T w[4][G];
+#pragma unroll
+                    for (int d = 0; d < G; ++d) {
+                        const int o = (j0 + d) * sa;
+                        w[0][d] = p0[o];
+                        w[1][d] = p1[o];
+                        w[2][d] = p2[o];
+                        w[3][d] = p3[o];
                     }
-                } else {
-                    const Rank fa = rank_of<N, false>(j, lasta), fb = rank_of<N, false>(jb, lastb);
-                    const T pa = pred_line<T, N, false>(j, lasta, a0, a1, a2, a3);
-                    T pb = fb == R_CUBIC ? cubic(v0, v1, v2, v3) : quad_l(v0, v1, v2);
-                    if (jb == 0) pb = fb == R_QUAD ? quad_r(v1, v2, v3) : lin(v1, v2);
-                    pred = fa > fb ? pa : pb;
-                    if (fa == fb) {
-                        if (fa == R_NONE) pred = (a1 + v1) - t.s[left + o];
-                        else pred = (pa + pb) / (T)2;
+#pragma unroll
+                    for (int d = 0; d < G; ++d) {
+                        const int j = j0 + d;
+                        const T pred = pred_face2<T, N, IN>(left + j * sa, rank_of<N, IN>(j, lasta), j, lasta,
+                                                            k[j > 0 ? j - 1 : 0], k[j], k[j + 1], k[j + 2 <= N ? j + 2 : N],
+                                                            jb, lastb, w[0][d], w[1][d], w[2][d], w[3][d]);
+                        int32_t code = 0;
+                        put_point<T, M, false>(t, own + j * sa, v[j], pred, code);
+                        if constexpr (M == COMPRESS) rc.code[j] = code;
                     }
                 }
-                int32_t code;
-                put_point<T, M, SINK>(t, own_slot + o, t.s[own_slot + o], pred, code);
-                if constexpr (M == COMPRESS && SINK == TO_GLOBAL) {
-                    if (own && (IN || (2 * j + 1) * U < ra)) t.qc_out[idx + j * idx_step] = code;
+                rc.slot = own;
+                rc.step = sa;
+            } else if constexpr (U == 2) {
+                const int ji = 1 + h, je = 3 * h, oi = ji * sa, oe = je * sa;
+                const T *w = ka + h * sa, w0 = w[0], w1 = w[sa], w2 = w[2 * sa], w3 = w[3 * sa];
+                const T i0 = p0[oi], i1 = p1[oi], i2 = p2[oi], i3 = p3[oi];
+                const T e0 = p0[oe], e1 = p1[oe], e2 = p2[oe], e3 = p3[oe];
+                const T vi = t.s[own + oi], ve = t.s[own + oe];
+                const T pi = pred_face2<T, N, IN>(left + oi, IN ? R_CUBIC : rank_of<N, IN>(ji, lasta), ji, lasta, w0, w1, w2,
+                                                  w3, jb, lastb, i0, i1, i2, i3);
+                const T pe = pred_face2<T, N, IN>(left + oe, IN ? R_QUAD : rank_of<N, IN>(je, lasta), je, lasta, w1,
+                                                  h == 0 ? w0 : w2, h == 0 ? w1 : w3, w2, jb, lastb, e0, e1, e2, e3);
+                int32_t ci = 0, ce = 0;
+                put_point<T, M, false>(t, own + oi, vi, pi, ci);
+                put_point<T, M, false>(t, own + oe, ve, pe, ce);
+                if constexpr (M == COMPRESS) {
+                    rc.code[0] = ci;
+                    rc.code[1] = ce;
                 }
-                if constexpr (M == COMPRESS && SINK == TO_REGS) rc->code[j] = code;
-            }
-            if constexpr (M == COMPRESS && SINK == TO_REGS) {
-                rc->slot = own ? own_slot : -1;
-                rc->step = sa;
+                rc.slot = own + oi;
+                rc.step = oe - oi;
+            } else {
+                const int o = h * sa;
+                const T w0 = ka[0], w1 = ka[sa], w2 = ka[(N == 2 ? 2 : 1) * sa];
+                const T b0 = p0[o], b1 = p1[o], b2 = p2[o], b3 = p3[o], v = t.s[own + o];
+                const T pred = pred_face2<T, N, IN>(left + o, IN ? R_QUAD : rank_of<N, IN>(h, lasta), h, lasta, w0,
+                                                    h == 0 ? w0 : w1, h == 0 ? w1 : w2, w2, jb, lastb, b0, b1, b2, b3);
+                put_point<T, M, false>(t, own + o, v, pred, rc.code[0]);
+                rc.slot = own + o;
             }
         }
     }
@@ -319,12 +446,13 @@ __device__ __forceinline__ void faces_stage(Tile<T, IN>& t, RegCodes* rc = nullp
 // CUBE points (three odd coordinates, InterpolationPredictor.cu:1671-1723):
 // the mean of the directions whose formula is the cubic; without one, x's
 // formula.
-template <typename T, int U, int M, int SINK, bool IN>
-__device__ __forceinline__ void cubes_stage(Tile<T, IN>& t) {
-    constexpr int N = 8 / U, L = level_of_unit<U>(), TOTAL = N * N * N;
+template <typename T, int U, int M, bool IN>
+__device__ __forceinline__ void cubes_stage(Tile<T, IN>& t, RegCodes<kPart<U>>& rc) {
+    constexpr int N = 8 / U, TOTAL = N * N * N;
+    constexpr bool LAST = U == 1;
     constexpr int SX = slot_step<U, 0>(), SY = slot_step<U, 1>(), SZ = slot_step<U, 2>();
     constexpr int HX = slot_half<U, 0>(), HY = slot_half<U, 1>(), HZ = slot_half<U, 2>();
-    const int l = lane_id();
+    const int l = lane_id(stage_wave<U, 2, true>());
 #pragma unroll
     for (int it = 0; it < (TOTAL + kThreads - 1) / kThreads; ++it) {
         const int p = l + it * kThreads;
@@ -336,116 +464,185 @@ __device__ __forceinline__ void cubes_stage(Tile<T, IN>& t) {
                           lastz = (int)((unsigned)(t.rz - 1) / (2 * U));
                 const int corner = i * SX + j * SY + k * SZ, own_slot = corner + HX + HY + HZ;
                 // x's taps: y and z odd, from the left neighbour
-                const int bx = corner + HY + HZ;
-                const T x0 = t.s[bx - (i > 0 ? SX : 0)], x1 = t.s[bx], x2 = t.s[bx + SX];
-                const T x3 = t.s[bx + (i < N - 1 ? 2 * SX : SX)];
+                const T* bx = t.s + corner + (HY + HZ);
+                const T own = t.s[own_slot];
+                const T x0 = bx[i > 0 ? -SX : 0], x1 = bx[0], x2 = bx[SX], x3 = bx[i < N - 1 ? 2 * SX : SX];
                 const Rank fx = rank_of<N, IN>(i, lastx);
                 T pred = x1;
-                if (N > 1 && fx == R_QUAD) pred = i == 0 ? quad_r(x1, x2, x3) : quad_l(x0, x1, x2);
-                if ((N == 1 || !IN) && fx == R_LIN) pred = lin(x1, x2);
+                if constexpr (N == 1) {
+                    if (IN || fx == R_LIN) pred = lin(x1, x2);
+                } else {
+                    const T qr = quad_r(x1, x2, x3), ql = quad_l(x0, x1, x2);
+                    if constexpr (!IN) {
+                        if (fx == R_LIN) pred = lin(x1, x2);
+                    }
+                    pred = IN || fx == R_QUAD ? (i == 0 ? qr : ql) : pred;
+                }
                 if constexpr (N > 2) {
-                    const int by = corner + HX + HZ, bz = corner + HX + HY;
-                    const int y0 = by - (j > 0 ? SY : 0), y3 = by + (j < N - 1 ? 2 * SY : SY);
-                    const int z0 = bz - (k > 0 ? SZ : 0), z3 = bz + (k < N - 1 ? 2 * SZ : SZ);
-                    const T px = cubic(x0, x1, x2, x3);
-                    const T py = cubic(t.s[y0], t.s[by], t.s[by + SY], t.s[y3]);
-                    const T pz = cubic(t.s[z0], t.s[bz], t.s[bz + SZ], t.s[z3]);
+                    const T *by = t.s + corner + (HX + HZ), *bz = t.s + corner + (HX + HY);
+                    const T y0 = by[j > 0 ? -SY : 0], y1 = by[0], y2 = by[SY], y3 = by[j < N - 1 ? 2 * SY : SY];
+                    const T z0 = bz[k > 0 ? -SZ : 0], z1 = bz[0], z2 = bz[SZ], z3 = bz[k < N - 1 ? 2 * SZ : SZ];
                     const bool cx = fx == R_CUBIC, cy = rank_of<N, IN>(j, lasty) == R_CUBIC,
                                cz = rank_of<N, IN>(k, lastz) == R_CUBIC;
                     // an absent direction adds 0 (a zero's sign cannot reach a
                     // value or code: each adds code * ebx2 to the prediction)
-                    const T sum = ((cx ? px : (T)0) + (cy ? py : (T)0)) + (cz ? pz : (T)0);
-                    const int n = (int)cx + (int)cy + (int)cz;
-                    if (n == 1) pred = sum;
-                    if (n == 2) pred = sum / (T)2;
-                    if (n == 3) pred = sum / (T)3;
+                    const T px = cx ? cubic(x0, x1, x2, x3) : (T)0;
+                    const T py = cy ? cubic(y0, y1, y2, y3) : (T)0;
+                    const T pz = cz ? cubic(z0, z1, z2, z3) : (T)0;
+                    const T sum = (px + py) + pz;
+                    const T half = sum / (T)2, third = third_of(sum);
+                    const bool all = cx && cy && cz, two = (cx && cy) || (cz && (cx || cy)), any = cx || cy || cz;
+                    pred = any ? sum : pred;
+                    pred = two ? half : pred;
+                    pred = all ? third : pred;
                 }
-                int32_t code;
-                put_point<T, M, SINK>(t, own_slot, t.s[own_slot], pred, code);
-                if constexpr (M == COMPRESS && SINK == TO_GLOBAL) t.qc_out[lm_at<L>(t, x, y, z)] = code;
+                int32_t code = 0;
+                put_point<T, M, LAST>(t, own_slot, own, pred, code);
+                if constexpr (M == COMPRESS && !LAST) {  // one point: every code its, step 0
+#pragma unroll
+                    for (int d = 0; d < kPart<U>; ++d) rc.code[d] = code;
+                    rc.slot = own_slot;
+                    rc.step = 0;
+                }
             }
         }
     }
     lds_barrier();
 }
 
-// Level 0's codes of the 16^3 tile, in their slots once the register-held
-// ones join them, written out row by row: lane (x, y) = (l mod 16, l / 16)
-// takes z = 0..15.  A row (y, z) with y or z odd holds every x (16 adjacent
-// codes), the others the odd x (8 adjacent codes); from z to z + 2 the index
-// advances by 2 lxy0 - lxy1.
-template <typename T, bool IN>
-__device__ __forceinline__ void level0_codes_out(Tile<T, IN>& t, const RegCodes& a, const RegCodes& b) {
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        if (a.slot >= 0) t.s[a.slot + k * a.step] = code_slot(a.code[k], T());
+// Level 0's codes of a tile in the level-major array, by column (x, y): at odd
+// z a row holds every x, at even z every x of an odd y and the odd x of an
+// even y; from z to z + 2 the index advances by 2 lxy0 - lxy1.  The tile's
+// part of an index is uniform (a scalar base that steps along z), the lane's
+// a 32-bit offset (nx is below 2^24 in an IN tile; elsewhere the lane's part
+// is added in 64 bits).
+template <typename E, bool IN>
+struct Columns0 {
+    using Off = std::conditional_t<IN, uint32_t, int64_t>;
+    E *even, *odd;  // z = 0 and z = 1
+    int64_t step;
+    Off off_even, off_odd;
+
+    template <typename T>
+    __device__ __forceinline__ Columns0(const Tile<T, IN>& t, E* q, int x, int y) {
+        const int64_t lx0 = t.g.lx[0], lx1 = t.g.lx[1], lxy0 = t.g.lxy[0], lxy1 = t.g.lxy[1];
+        step = 2 * lxy0 - lxy1;
+        const int64_t base = t.g.prefix[0] + t.oy * lx0 + (t.oz >> 1) * step;
+        even = q + (base - (t.oy >> 1) * lx1);
+        odd = q + (base + t.ox + lxy0 - lxy1);
+        const Off row = (Off)y * (Off)lx0;
+        off_odd = row + (Off)x;
+        off_even = row - (Off)((y + 1) >> 1) * (Off)lx1 + (Off)((y & 1) ? t.ox + x : (t.ox + x) >> 1);
     }
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        if (b.slot >= 0) t.s[b.slot + k * b.step] = code_slot(b.code[k], T());
-    }
-    lds_barrier();
-    const int lane = lane_id();
-    const int x = lane & 15, y = lane >> 4;
-    if (!(t.template in<0>(x) && t.template in<1>(y))) return;
-    const int64_t step = 2 * t.g.lxy[0] - t.g.lxy[1];
-    const T* src = t.s + tslot(x, y, 0);
-    int32_t* odd = t.qc_out + lm_at<0>(t, x, y, 1);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        if (t.template in<2>(2 * k + 1)) *odd = slot_code(src[(2 * k + 1) * kZP]);
+    __device__ __forceinline__ E& at_even() const { return *(E*)((char*)even + off_even * (Off)sizeof(E)); }
+    __device__ __forceinline__ E& at_odd() const { return *(E*)((char*)odd + off_odd * (Off)sizeof(E)); }
+    __device__ __forceinline__ void next() {
+        even += step;
         odd += step;
     }
-    if ((x | y) & 1) {
-        int32_t* even = t.qc_out + lm_at<0>(t, x, y, 0);
+};
+
+// The codes of the group's tiles, all in their slots, written out row by row.
+// Level 0: a row lane takes its column's z = 0..15 (rows of 16 or 8 adjacent
+// codes per tile).  Level 1: the group's points with even coordinates, in two
+// passes of 8 adjacent codes per tile and row; levels 2 and 3 in one.
+template <typename T, bool IN>
+__device__ __forceinline__ void codes_out(const Tile<T, IN>& m) {
+    constexpr int P = kGroup<T, COMPRESS>;
+    {
+        const RowLane<P> r;
+        if (m.template in<0>(r.X) && m.template in<1>(r.y)) {
+            const T* src = m.s + r.slot(r.y, 0);
+            Columns0<int32_t, IN> c(m, m.qc_out, r.X, r.y);
+            const bool on_even = (r.X | r.y) & 1;
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            if (t.template in<2>(2 * k)) *even = slot_code(src[2 * k * kZP]);
-            even += step;
+            for (int k = 0; k < 8; ++k) {
+                if (m.template in<2>(2 * k + 1)) c.at_odd() = slot_code(src[(2 * k + 1) * kZP]);
+                if (on_even && m.template in<2>(2 * k)) c.at_even() = slot_code(src[2 * k * kZP]);
+                c.next();
+            }
         }
     }
-}
-
-// The three stages of one level (InterpolationPredictor.cu:1940-2025).
-template <typename T, int U, int M, bool IN>
-__device__ __forceinline__ void level3(Tile<T, IN>& t, bool md, bool rev) {
-    constexpr bool EX = U == 1;
-    constexpr int S1 = U == 1 ? TO_REGS : TO_GLOBAL, S2 = U == 1 ? TO_SLOT : TO_GLOBAL;
-    RegCodes a, b;
-    if (md) {
-        lines3_stage<T, U, M, S1>(t, &a);
-        faces_stage<T, U, M, S1>(t, &b);
-        cubes_stage<T, U, M, S2>(t);
-    } else if (rev) {
-        line_stage<T, U, 0, false, false, false, M, S1>(t, &a);
-        line_stage<T, U, 1, true, false, false, M, S1>(t, &b);
-        line_stage<T, U, 2, true, true, EX, M, S2>(t);
-    } else {
-        line_stage<T, U, 2, false, false, false, M, S1>(t, &a);
-        line_stage<T, U, 1, false, true, false, M, S1>(t, &b);
-        line_stage<T, U, 0, true, true, EX, M, S2>(t);
-    }
-    if constexpr (M == COMPRESS && U == 1) level0_codes_out(t, a, b);
-}
-
-// The four levels of a tile, coarsest first.
-template <typename T, int M, bool IN>
-__device__ __forceinline__ void tile_levels(Tile<T, IN>& t, const LevelEb<T>& le, const uint8_t* flags8, int maxlevel) {
-    uint8_t fl[8];
+    const int v = thread_id();
 #pragma unroll
-    for (int i = 0; i < 8; ++i) fl[i] = flags8[i];
-    if (3 <= maxlevel) { t.eb_r = le.eb_r[3]; t.ebx2 = le.ebx2[3]; level3<T, 8, M>(t, fl[3], fl[7]); }
-    if (2 <= maxlevel) { t.eb_r = le.eb_r[2]; t.ebx2 = le.ebx2[2]; level3<T, 4, M>(t, fl[2], fl[6]); }
-    if (1 <= maxlevel) { t.eb_r = le.eb_r[1]; t.ebx2 = le.ebx2[1]; level3<T, 2, M>(t, fl[1], fl[5]); }
-    if (0 <= maxlevel) { t.eb_r = le.eb_r[0]; t.ebx2 = le.ebx2[0]; level3<T, 1, M>(t, fl[0], fl[4]); }
+    for (int it = 0; it < 2; ++it) {
+        const int X = 2 * (v & (8 * P - 1)), y = 2 * ((v / (8 * P)) & 7), z = 2 * (v / (64 * P) + 4 * it);
+        if (((X | y | z) & 2) && m.in3(X, y, z))
+            m.qc_out[lm_at<1>(m, X, y, z)] = slot_code(m.s[(X >> 4) * kTileLds + tslot(X & 15, y, z)]);
+    }
+    if (v < 64 * P) {
+        const int X = 4 * (v & (4 * P - 1)), y = 4 * ((v / (4 * P)) & 3), z = 4 * (v / (16 * P));
+        if (((X | y | z) & 4) && m.in3(X, y, z))
+            m.qc_out[lm_at<2>(m, X, y, z)] = slot_code(m.s[(X >> 4) * kTileLds + tslot(X & 15, y, z)]);
+    } else if (v < 64 * P + 8 * P) {
+        const int w = v - 64 * P, X = 8 * (w & (2 * P - 1)), y = 8 * ((w / (2 * P)) & 1), z = 8 * (w / (4 * P));
+        if (((X | y | z) & 8) && m.in3(X, y, z))
+            m.qc_out[lm_at<3>(m, X, y, z)] = slot_code(m.s[(X >> 4) * kTileLds + tslot(X & 15, y, z)]);
+    }
+}
+
+// The three stages of one level (InterpolationPredictor.cu:1940-2025); a, b:
+// the codes' registers.  At level 0 they hold the first two stages' codes.  At
+// levels 2 and 3 each stage has a wave of its own, and a holds them all; at
+// level 1 a and b hold the codes of disjoint lanes: stages 0 and 2 (a: wave 0;
+// waves 1-3), 1 (b: waves 2, 3), or in the multi-dimensional form 0 (a: waves
+// 0-2), 1 and 2 (b: waves 2, 3; wave 0).
+template <typename T, int U, int M, bool IN>
+__device__ __forceinline__ void level3(Tile<T, IN>& t, bool md, bool rev, RegCodes<kPart<U>>& a, RegCodes<kPart<U>>& b) {
+    if (md) {
+        lines3_stage<T, U, M>(t, a);
+        faces_stage<T, U, M>(t, U > 2 ? a : b);
+        cubes_stage<T, U, M>(t, U > 2 ? a : b);
+    } else if (rev) {
+        line_stage<T, U, 0, 0, false, false, M>(t, a);
+        line_stage<T, U, 1, 1, true, false, M>(t, U > 2 ? a : b);
+        line_stage<T, U, 2, 2, true, true, M>(t, a);
+    } else {
+        line_stage<T, U, 0, 2, false, false, M>(t, a);
+        line_stage<T, U, 1, 1, false, true, M>(t, U > 2 ? a : b);
+        line_stage<T, U, 2, 0, true, true, M>(t, a);
+    }
+}
+
+// The flags in two steps: every lane loads one byte before the tile's loads
+// are issued, and once those are in their slots the bytes become a scalar mask
+// (bit i: flags8[i] is set).  Flags kept in registers as loaded instead made
+// the compiler wait for every outstanding access (the codes already stored,
+// the previous values still on their way) at each level.
+__device__ __forceinline__ uint32_t flags_load(const uint8_t* flags8) { return flags8[threadIdx.x & 7]; }
+__device__ __forceinline__ uint32_t flags_mask(uint32_t byte) {
+    asm volatile("" : "+v"(byte));  // (the comparison stays here)
+    return (uint32_t)__ballot(byte != 0u) & 0xFFu;
+}
+
+// The four levels of a tile, coarsest first; compressing, every code ends up
+// in its point's slot.
+template <typename T, int M, bool IN>
+__device__ __forceinline__ void tile_levels(Tile<T, IN>& t, const LevelEb<T>& le, uint32_t flags, int maxlevel) {
+    RegCodes<1> c3, c2;
+    RegCodes<2> c1a, c1b;
+    RegCodes<8> a, b;
+    if (3 <= maxlevel) { t.eb_r = le.eb_r[3]; t.ebx2 = le.ebx2[3]; level3<T, 8, M>(t, flags & 8, flags & 128, c3, c3); }
+    if (2 <= maxlevel) { t.eb_r = le.eb_r[2]; t.ebx2 = le.ebx2[2]; level3<T, 4, M>(t, flags & 4, flags & 64, c2, c2); }
+    if (1 <= maxlevel) { t.eb_r = le.eb_r[1]; t.ebx2 = le.ebx2[1]; level3<T, 2, M>(t, flags & 2, flags & 32, c1a, c1b); }
+    if (0 <= maxlevel) { t.eb_r = le.eb_r[0]; t.ebx2 = le.ebx2[0]; level3<T, 1, M>(t, flags & 1, flags & 16, a, b); }
+    if constexpr (M == COMPRESS) {
+        join_slots(t.s, c3);
+        join_slots(t.s, c2);
+        join_slots(t.s, c1a);
+        join_slots(t.s, c1b);
+        join_slots(t.s, a);
+        join_slots(t.s, b);
+        lds_barrier();
+    }
 }
 
 // ------------------------------------------------------- tile and memory --
 // The 17^3 points of a tile are taken as 20 sets of at most one point per
-// lane: the column (x, y) = (l mod 16, l / 16) at z = 0..16, then the faces
-// y = 16 (lane (x, z)) and x = 16 (lane (y, z)) without their last rows, then
-// those rows: (x, 16, 16), (16, 16, z) and (16, y, 16).  Addresses advance by
-// one plane from point to point, so a column costs one addition per point.
+// lane: the rows y < 16 at z = 0..16, the rows y = 16 at z < 16 (both by the
+// group's row lanes), then by the tile's own lanes the face x = 16 (lane
+// (y, z) = (l mod 16, l / 16)) and the last rows (x, 16, 16), (16, 16, z) and
+// (16, y, 16).  Addresses of the first advance by a plane from point to point.
 // false: the lane has no point.
 __device__ __forceinline__ bool edge_point(int l, int& x, int& y, int& z) {
     x = l < 16 ? l : 16;
@@ -454,34 +651,51 @@ __device__ __forceinline__ bool edge_point(int l, int& x, int& y, int& z) {
     return l < 49;
 }
 
+// Column (x, y) of a tile of a field (base: the tile's first value), plane by
+// plane: a uniform base that steps by a plane and the lane's 32-bit offset
+// (nx is below 2^24 in an IN tile; elsewhere 64-bit).
+template <typename T, bool IN>
+struct Column {
+    using Off = std::conditional_t<IN, uint32_t, uint64_t>;
+    T* base;
+    uint32_t plane;
+    Off off;
+
+    __device__ __forceinline__ Column(T* b, uint32_t nx, uint32_t nxy, int x, int y)
+        : base(b), plane(nxy), off((Off)y * nx + (Off)x) {}
+    __device__ __forceinline__ T& at() const { return *(T*)((char*)base + off * (Off)sizeof(T)); }
+    __device__ __forceinline__ void next() { base += plane; }
+};
+
 // Tile plus halo into LDS: all global loads of a lane are issued before the
 // first LDS write so the tile costs one memory latency.  Points outside the
 // field are not read (no formula uses their slots).
 template <typename T, bool IN>
-__device__ __forceinline__ void tile_load(const Tile<T, IN>& t, const T* __restrict__ data) {
-    const int l = lane_id();
-    const int x = l & 15, y = l >> 4;
-    const int64_t nx = t.g.nx, nxy = nx * t.g.ny;
-    const T* base = data + (t.oz * nxy + t.oy * nx + t.ox);
+__device__ __forceinline__ void tile_load(const Tile<T, IN>& t, const Tile<T, IN>& m, const T* __restrict__ data) {
+    const uint32_t nx = (uint32_t)t.g.nx, nxy = nx * (uint32_t)t.g.ny;  // (fields have fewer than 2^31 values)
+    const T* base = data + ((uint64_t)m.oz * nxy + (uint64_t)m.oy * nx + m.ox);
     T v[17], fy = (T)0, fx = (T)0, e = (T)0;
-    int ex, ey, ez;
-    const bool edge = edge_point(l, ex, ey, ez);
-    const bool on = t.template in<0>(x) && t.template in<1>(y);
-    const T* p = base + (y * nx + x);
+    const RowLane<kGroup<T, COMPRESS>> r;
+    const bool on = m.template in<0>(r.X) && m.template in<1>(r.y);
+    Column<const T, IN> p(base, nx, nxy, r.X, r.y);
 #pragma unroll
     for (int z = 0; z < 17; ++z) {
         v[z] = (T)0;
-        if (on && t.template in<2>(z)) v[z] = *p;
-        p += nxy;
+        if (on && m.template in<2>(z)) v[z] = p.at();
+        p.next();
     }
-    if (t.in3(x, 16, y)) fy = base[y * nxy + 16 * nx + x];
-    if (t.in3(16, x, y)) fx = base[y * nxy + x * nx + 16];
-    if (edge && t.in3(ex, ey, ez)) e = base[ez * nxy + ey * nx + ex];
-    T* d = t.s + tslot(x, y, 0);
+    if (m.in3(r.X, 16, r.y)) fy = base[(uint64_t)r.y * nxy + (16 * (uint64_t)nx + r.X)];
+    const int l = lane_id(), y = l & 15, z = l >> 4;
+    int ex, ey, ez;
+    const bool edge = edge_point(l, ex, ey, ez);
+    base += t.ox - m.ox;
+    if (t.in3(16, y, z)) fx = base[(uint64_t)z * nxy + ((uint64_t)y * nx + 16)];
+    if (edge && t.in3(ex, ey, ez)) e = base[(uint64_t)ez * nxy + ((uint64_t)ey * nx + ex)];
+    T* d = m.s + r.slot(r.y, 0);
 #pragma unroll
-    for (int z = 0; z < 17; ++z) d[z * kZP] = v[z];
-    t.s[tslot(x, 16, y)] = fy;
-    t.s[tslot(16, x, y)] = fx;
+    for (int k = 0; k < 17; ++k) d[k * kZP] = v[k];
+    m.s[r.slot(16, r.y)] = fy;
+    t.s[tslot(16, y, z)] = fx;
     if (edge) t.s[tslot(ex, ey, ez)] = e;
 }
 
@@ -527,10 +741,9 @@ __device__ __forceinline__ bool coarse_point(int l, int& unit, int& i, int& j, i
 }
 
 template <typename T, bool IN, typename E>
-__device__ __forceinline__ void codes_load(const Tile<T, IN>& t, const E* __restrict__ q, int maxlevel,
+__device__ __forceinline__ void codes_load(const Tile<T, IN>& t, const Tile<T, IN>& m, const E* __restrict__ q, int maxlevel,
                                            const T* __restrict__ anchors, int bx, int by, int bz, TileCodes<T>& c) {
     const int l = lane_id();
-    const int x = l & 15, y = l >> 4;
     const bool l0 = maxlevel >= 0;
     c.v23 = 0;
     {
@@ -550,35 +763,31 @@ __device__ __forceinline__ void codes_load(const Tile<T, IN>& t, const E* __rest
         if (maxlevel >= 1 && p < 729 && ((i | j | k) & 1) && t.in3(2 * i, 2 * j, 2 * k))
             c.v1[it] = q[lm_at<1>(t, 2 * i, 2 * j, 2 * k)];
     }
-    const int64_t step = 2 * t.g.lxy[0] - t.g.lxy[1];
-    const bool on = l0 && t.template in<0>(x) && t.template in<1>(y), on_even = on && ((x | y) & 1);
-    const E* even = q + lm_at<0>(t, x, y, 0);
-    const E* odd = q + lm_at<0>(t, x, y, 1);
+    const RowLane<kGroup<T, DECOMPRESS>> r;
+    const bool on = l0 && m.template in<0>(r.X) && m.template in<1>(r.y), on_even = on && ((r.X | r.y) & 1);
+    Columns0<const E, IN> col(m, q, r.X, r.y);
 #pragma unroll
     for (int k = 0; k <= 8; ++k) {
         c.v0[2 * k] = 0;
-        if (on_even && t.template in<2>(2 * k)) c.v0[2 * k] = *even;
-        even += step;
+        if (on_even && m.template in<2>(2 * k)) c.v0[2 * k] = col.at_even();
         if (k < 8) {
             c.v0[2 * k + 1] = 0;
-            if (on && t.template in<2>(2 * k + 1)) c.v0[2 * k + 1] = *odd;
-            odd += step;
+            if (on && m.template in<2>(2 * k + 1)) c.v0[2 * k + 1] = col.at_odd();
         }
+        col.next();
     }
     c.fy = c.fx = c.e = 0;
-    if (l0 && ((x | y) & 1)) {  // z = y here, then y = x
-        if (t.in3(x, 16, y)) c.fy = q[lm_at<0>(t, x, 16, y)];
-        if (t.in3(16, x, y)) c.fx = q[lm_at<0>(t, 16, x, y)];
-    }
+    if (l0 && ((r.X | r.y) & 1) && m.in3(r.X, 16, r.y)) c.fy = q[lm_at<0>(m, r.X, 16, r.y)];
+    const int y = l & 15, z = l >> 4;
+    if (l0 && ((y | z) & 1) && t.in3(16, y, z)) c.fx = q[lm_at<0>(t, 16, y, z)];
     int ex, ey, ez;
     if (edge_point(l, ex, ey, ez) && l0 && ((ex | ey | ez) & 1) && t.in3(ex, ey, ez)) c.e = q[lm_at<0>(t, ex, ey, ez)];
     c.anc = anchor_load(t, anchors, bx, by, bz);
 }
 
 template <typename T, bool IN>
-__device__ __forceinline__ void codes_store(const Tile<T, IN>& t, const TileCodes<T>& c) {
+__device__ __forceinline__ void codes_store(const Tile<T, IN>& t, const Tile<T, IN>& m, const TileCodes<T>& c) {
     const int l = lane_id();
-    const int x = l & 15, y = l >> 4;
     {
         int u, i, j, k;
         if (coarse_point(l, u, i, j, k) && ((i | j | k) & 1)) t.s[tslot(u * i, u * j, u * k)] = code_slot(c.v23, T());
@@ -588,15 +797,17 @@ __device__ __forceinline__ void codes_store(const Tile<T, IN>& t, const TileCode
         const int p = l + it * kThreads, i = p % 9, j = (p / 9) % 9, k = p / 81;
         if (p < 729 && ((i | j | k) & 1)) t.s[tslot(2 * i, 2 * j, 2 * k)] = code_slot(c.v1[it], T());
     }
-    T* d = t.s + tslot(x, y, 0);
+    const RowLane<kGroup<T, DECOMPRESS>> r;
+    T* d = m.s + r.slot(r.y, 0);
 #pragma unroll
     for (int k = 0; k < 8; ++k) d[(2 * k + 1) * kZP] = code_slot(c.v0[2 * k + 1], T());
-    if ((x | y) & 1) {
+    if ((r.X | r.y) & 1) {
 #pragma unroll
         for (int k = 0; k <= 8; ++k) d[2 * k * kZP] = code_slot(c.v0[2 * k], T());
-        t.s[tslot(x, 16, y)] = code_slot(c.fy, T());
-        t.s[tslot(16, x, y)] = code_slot(c.fx, T());
+        m.s[r.slot(16, r.y)] = code_slot(c.fy, T());
     }
+    const int y = l & 15, z = l >> 4;
+    if ((y | z) & 1) t.s[tslot(16, y, z)] = code_slot(c.fx, T());
     int ex, ey, ez;
     if (edge_point(l, ex, ey, ez) && ((ex | ey | ez) & 1)) t.s[tslot(ex, ey, ez)] = code_slot(c.e, T());
     anchor_store(t, c.anc);
