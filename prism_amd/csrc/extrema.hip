@@ -17,21 +17,25 @@ __global__ void extrema_init_kernel(unsigned long long* keys) {
     keys[1] = 0ull;   // running max
 }
 
+// One workgroup of 16 waves per CU: as many loads in flight as four of 4
+// waves, and a quarter of the atomics on the keys, which all workgroups of a
+// field below about 50 MB reach at the same time (24 MB: 35 us with 1024
+// workgroups of 4 waves, most of it in up to 2048 atomics of 12 ns).
+constexpr int kExtThreads = 1024;
 template <typename T>
-__global__ __launch_bounds__(256) void extrema_kernel(const T* __restrict__ in, int64_t n,
-                                                      unsigned long long* __restrict__ keys) {
-    __shared__ double s_min[4], s_max[4];
-    constexpr int V = 16 / sizeof(T);
-    using Vec = typename std::conditional<sizeof(T) == 4, float4, double2>::type;
-    double mn = __builtin_inf(), mx = -__builtin_inf();
+__global__ __launch_bounds__(kExtThreads) void extrema_kernel(const T* __restrict__ in, int64_t n,
+                                                              unsigned long long* __restrict__ keys) {
+    MinMax<T> m;
+    using Vec = typename MinMax<T>::Vec;
+    constexpr int V = MinMax<T>::V;
     const int64_t nv = n / V;
     const Vec* vin = reinterpret_cast<const Vec*>(in);
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    // Each workgroup streams one contiguous chunk of whole 32 KiB batches;
-    // a batch puts kBatch independent 16-byte loads per lane in flight
-    // before any is reduced.
-    constexpr int kBatch = 8;
-    constexpr int64_t kSpan = (int64_t)kBatch * 256;  // vectors per batch
+    const int64_t stride = (int64_t)gridDim.x * kExtThreads;
+    // Each workgroup streams one contiguous chunk of whole 64 KiB batches; a
+    // batch puts kBatch independent 16-byte loads per lane in flight before
+    // any is reduced.
+    constexpr int kBatch = 4;
+    constexpr int64_t kSpan = (int64_t)kBatch * kExtThreads;  // vectors per batch
     const int64_t batches = nv / kSpan;
     const int64_t per = (batches + gridDim.x - 1) / gridDim.x;
     const int64_t b0 = blockIdx.x * per, b1 = b0 + per < batches ? b0 + per : batches;
@@ -39,49 +43,16 @@ __global__ __launch_bounds__(256) void extrema_kernel(const T* __restrict__ in, 
         const Vec* p = vin + bt * kSpan + threadIdx.x;
         Vec v[kBatch];
 #pragma unroll
-        for (int k = 0; k < kBatch; ++k) v[k] = p[k * 256];
+        for (int k = 0; k < kBatch; ++k) v[k] = p[k * kExtThreads];
 #pragma unroll
-        for (int k = 0; k < kBatch; ++k) {
-            const T* e = reinterpret_cast<const T*>(&v[k]);
-#pragma unroll
-            for (int j = 0; j < V; ++j) {
-                mn = fmin(mn, (double)e[j]);
-                mx = fmax(mx, (double)e[j]);
-            }
-        }
+        for (int k = 0; k < kBatch; ++k) m.take(v[k]);
     }
-    for (int64_t i = batches * kSpan + blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < nv; i += stride) {
-        const Vec v = vin[i];
-        const T* e = reinterpret_cast<const T*>(&v);
-#pragma unroll
-        for (int j = 0; j < V; ++j) {
-            mn = fmin(mn, (double)e[j]);
-            mx = fmax(mx, (double)e[j]);
-        }
-    }
-    for (int64_t i = nv * V + blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += stride) {
-        mn = fmin(mn, (double)in[i]);
-        mx = fmax(mx, (double)in[i]);
-    }
-    wave_minmax(mn, mx);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (lane == 0) {
-        s_min[wave] = mn;
-        s_max[wave] = mx;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int w = 1; w < 4; ++w) {
-            mn = fmin(mn, s_min[w]);
-            mx = fmax(mx, s_max[w]);
-        }
-        // atomics on one address from every workgroup serialise (about 12 ns
-        // each on MI355X); a workgroup that cannot improve the running value
-        // skips its atomic, and the running values settle after a few
-        const unsigned long long kmn = order_key(mn), kmx = order_key(mx);
-        if (kmn < __hip_atomic_load(keys, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(keys, kmn);
-        if (kmx > __hip_atomic_load(keys + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(keys + 1, kmx);
-    }
+    const int64_t at = blockIdx.x * (int64_t)kExtThreads + threadIdx.x;
+    for (int64_t i = batches * kSpan + at; i < nv; i += stride) m.take(vin[i]);
+    for (int64_t i = nv * V + at; i < n; i += stride) m.take(in[i]);
+    double mn = (double)m.mn, mx = (double)m.mx;
+    group_minmax<kExtThreads / 64>(mn, mx);
+    if (threadIdx.x == 0) join_keys(mn, mx, keys);
 }
 
 __global__ void extrema_finish_kernel(const unsigned long long* keys, double* out) {
@@ -102,14 +73,13 @@ extern "C" int pa_extrema(const void* d_data, int dtype, int64_t n, double* d_mi
     unsigned long long* keys = reinterpret_cast<unsigned long long*>(d_minmax + 2);
     hipLaunchKernelGGL(extrema_init_kernel, dim3(1), dim3(1), 0, st, keys);
     PA_LAUNCH_CHECK();
-    // 1024 workgroups (4 per CU) streaming contiguous ranges read faster on
-    // MI355X than 2048 or 4096 (78 us against 90 us for 302 MB)
-    const int64_t work = (n + 255) / 256;
-    const int blocks = (int)(work < 1024 ? work : 1024);
+    const int64_t work = (n + kExtThreads - 1) / kExtThreads;
+    const int blocks = (int)(work < device_cus() ? work : device_cus());
     if (dtype == PA_F32)
-        hipLaunchKernelGGL(extrema_kernel<float>, dim3(blocks), dim3(256), 0, st, (const float*)d_data, n, keys);
+        hipLaunchKernelGGL(extrema_kernel<float>, dim3(blocks), dim3(kExtThreads), 0, st, (const float*)d_data, n, keys);
     else
-        hipLaunchKernelGGL(extrema_kernel<double>, dim3(blocks), dim3(256), 0, st, (const double*)d_data, n, keys);
+        hipLaunchKernelGGL(extrema_kernel<double>, dim3(blocks), dim3(kExtThreads), 0, st, (const double*)d_data, n,
+                           keys);
     PA_LAUNCH_CHECK();
     hipLaunchKernelGGL(extrema_finish_kernel, dim3(1), dim3(1), 0, st, keys, d_minmax);
     PA_LAUNCH_CHECK();

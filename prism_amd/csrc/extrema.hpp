@@ -40,17 +40,50 @@ __device__ inline void wave_minmax(double& mn, double& mx) {
     mx = b;
 }
 
-// Workgroup b of the batch streams `span` 16-byte vectors of its field in
-// batches of 8 loads per lane (the field's tail elements go to its last
-// workgroup); the running keys of each field live in its own descriptor.
+// Running minimum and maximum of 16-byte vectors, in T (exact, as in double).
 template <typename T>
-__device__ inline void extrema_span(const T* in, int64_t n, int64_t wg, int64_t span, unsigned long long* keys) {
-    __shared__ double s_min[4], s_max[4];
-    constexpr int V = 16 / sizeof(T);
+struct MinMax {
+    static constexpr int V = 16 / sizeof(T);
     using Vec = typename std::conditional<sizeof(T) == 4, float4, double2>::type;
-    const int64_t nv = n / V;
+    T mn = (T)__builtin_inf(), mx = -(T)__builtin_inf();
+    __device__ __forceinline__ void take(T v) {
+        mn = sizeof(T) == 4 ? (T)fminf((float)mn, (float)v) : (T)fmin((double)mn, (double)v);
+        mx = sizeof(T) == 4 ? (T)fmaxf((float)mx, (float)v) : (T)fmax((double)mx, (double)v);
+    }
+    __device__ __forceinline__ void take(const Vec& v) {
+        const T* e = reinterpret_cast<const T*>(&v);
+#pragma unroll
+        for (int j = 0; j < V; ++j) take(e[j]);
+    }
+};
+
+// Min and max of a workgroup of WAVES waves; valid in thread 0.
+template <int WAVES>
+__device__ inline void group_minmax(double& mn, double& mx) {
+    __shared__ double s_min[WAVES], s_max[WAVES];
+    wave_minmax(mn, mx);
+    if ((threadIdx.x & 63) == 0) {
+        s_min[threadIdx.x >> 6] = mn;
+        s_max[threadIdx.x >> 6] = mx;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < WAVES; ++w) {
+            mn = fmin(mn, s_min[w]);
+            mx = fmax(mx, s_max[w]);
+        }
+    }
+}
+
+// Workgroup `wg` of a field streams `span` 16-byte vectors of it in batches
+// of 8 loads per lane (the tail elements go to the last one).  Its result is
+// valid in thread 0.
+template <typename T>
+__device__ inline void extrema_span(const T* in, int64_t n, int64_t wg, int64_t span, double& mn, double& mx) {
+    MinMax<T> m;
+    using Vec = typename MinMax<T>::Vec;
+    const int64_t nv = n / MinMax<T>::V;
     const Vec* vin = reinterpret_cast<const Vec*>(in);
-    double mn = __builtin_inf(), mx = -__builtin_inf();
     const int64_t v0 = wg * span;
     const int64_t v1 = v0 + span < nv ? v0 + span : nv;
     for (int64_t b = v0; b < v1; b += kExtBatch) {
@@ -63,38 +96,24 @@ __device__ inline void extrema_span(const T* in, int64_t n, int64_t wg, int64_t 
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
             const int64_t i = b + threadIdx.x + k * 256;
-            if (i < v1) {
-                const T* e = reinterpret_cast<const T*>(&v[k]);
-#pragma unroll
-                for (int j = 0; j < V; ++j) {
-                    mn = fmin(mn, (double)e[j]);
-                    mx = fmax(mx, (double)e[j]);
-                }
-            }
+            if (i < v1) m.take(v[k]);
         }
     }
     if (v0 + span >= nv) {  // last workgroup of the field: scalar tail
-        for (int64_t i = nv * V + threadIdx.x; i < n; i += 256) {
-            mn = fmin(mn, (double)in[i]);
-            mx = fmax(mx, (double)in[i]);
-        }
+        for (int64_t i = nv * MinMax<T>::V + threadIdx.x; i < n; i += 256) m.take(in[i]);
     }
-    wave_minmax(mn, mx);
-    if ((threadIdx.x & 63) == 0) {
-        s_min[threadIdx.x >> 6] = mn;
-        s_max[threadIdx.x >> 6] = mx;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int w = 1; w < 4; ++w) {
-            mn = fmin(mn, s_min[w]);
-            mx = fmax(mx, s_max[w]);
-        }
-        const unsigned long long kmn = order_key(mn), kmx = order_key(mx);
-        if (kmn < __hip_atomic_load(keys, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(keys, kmn);
-        if (kmx > __hip_atomic_load(keys + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(keys + 1, kmx);
-    }
+    mn = (double)m.mn;
+    mx = (double)m.mx;
+    group_minmax<4>(mn, mx);
 }
 
+// A workgroup's result joins the field's running keys.  Atomics on one address
+// from every workgroup serialise (about 12 ns each on MI355X); one that cannot
+// improve the running value skips its atomic.
+__device__ inline void join_keys(double mn, double mx, unsigned long long* keys) {
+    const unsigned long long kmn = order_key(mn), kmx = order_key(mx);
+    if (kmn < __hip_atomic_load(keys, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(keys, kmn);
+    if (kmx > __hip_atomic_load(keys + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(keys + 1, kmx);
+}
 
 }  // namespace pa

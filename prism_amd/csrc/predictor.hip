@@ -1330,7 +1330,7 @@ __global__ void tune_pick_kernel(const double* __restrict__ part, int nblocks, d
 // 384 x 384 x 256), too few to fill the GPU on their own.
 template <typename T>
 __global__ __launch_bounds__(kThreads) void extrema_tune_kernel(const T* __restrict__ data, int64_t n,
-                                                                unsigned long long* __restrict__ keys, int64_t span,
+                                                                double* __restrict__ ext_part, int64_t span,
                                                                 Geom g, int sx0, int sy0, int sz0, int nsx, int nsy,
                                                                 int nblocks, double* __restrict__ part) {
     __shared__ T tile[kTileVals];
@@ -1339,29 +1339,39 @@ __global__ __launch_bounds__(kThreads) void extrema_tune_kernel(const T* __restr
     if ((int)blockIdx.x < ntune)
         tune_block<T>(data, g, sx0, sy0, sz0, nsx, nsy, (int)blockIdx.x % nblocks, (int)blockIdx.x / nblocks, part,
                       tile, red);
-    else
-        extrema_span<T>(data, n, (int64_t)blockIdx.x - ntune, span, keys);
-}
-
-__global__ void extrema_keys_init_kernel(unsigned long long* keys) {
-    keys[0] = ~0ull;  // running min
-    keys[1] = 0ull;   // running max
+    else {
+        double mn, mx;
+        extrema_span<T>(data, n, (int64_t)blockIdx.x - ntune, span, mn, mx);
+        if (threadIdx.x == 0) {
+            double* p = ext_part + 2 * ((int)blockIdx.x - ntune);
+            p[0] = mn;
+            p[1] = mx;
+        }
+    }
 }
 
 __device__ int64_t fill_bounds(const double* minmax, double eb_in, int rel, int dtype, double alpha, double* e);
 
-// min / max from the keys, the tuner's pick (as tune_pick_kernel) and, with
-// `bounds`, the level bounds of a relative eb (as level_bounds_kernel)
-__global__ void extrema_tune_finish_kernel(const unsigned long long* __restrict__ keys, double* __restrict__ minmax,
-                                           const double* __restrict__ part, int nblocks, double* __restrict__ scores,
-                                           uint8_t* __restrict__ flags, double eb, int dtype, double alpha,
-                                           double* __restrict__ bounds) {
+// min / max from the extrema workgroups' results, the tuner's pick (as
+// tune_pick_kernel) and, with `bounds`, the level bounds of a relative eb (as
+// level_bounds_kernel)
+constexpr int kFinishThreads = 256;
+__global__ __launch_bounds__(kFinishThreads) void extrema_tune_finish_kernel(
+    const double* __restrict__ ext_part, int next, double* __restrict__ minmax, const double* __restrict__ part,
+    int nblocks, double* __restrict__ scores, uint8_t* __restrict__ flags, double eb, int dtype, double alpha,
+    double* __restrict__ bounds) {
     __shared__ double s[kPickLds];
     __shared__ double e[15];
+    double mn = __builtin_inf(), mx = -__builtin_inf();
+    for (int i = threadIdx.x; i < next; i += kFinishThreads) {
+        mn = fmin(mn, ext_part[2 * i]);
+        mx = fmax(mx, ext_part[2 * i + 1]);
+    }
+    group_minmax<kFinishThreads / 64>(mn, mx);
     pick_parallel(part, nblocks, scores, flags, s, e);
     if (threadIdx.x != 0) return;
-    minmax[0] = key_value(keys[0]);
-    minmax[1] = key_value(keys[1]);
+    minmax[0] = mn;
+    minmax[1] = mx;
     if (bounds) {
         bounds[14] = (double)fill_bounds(minmax, eb, true, dtype, alpha, bounds);
         bounds[15] = 0.0;
@@ -1500,8 +1510,10 @@ __global__ __launch_bounds__(kThreads) void batch_front_kernel(const BatchField*
         const BatchField& F = fields[f];
         unsigned long long* keys = reinterpret_cast<unsigned long long*>(F.minmax + 2);
         const int64_t wg = b - p_ext[f];
-        if (F.dtype == PA_F32) extrema_span<float>(static_cast<const float*>(F.data), F.L.n, wg, span, keys);
-        else extrema_span<double>(static_cast<const double*>(F.data), F.L.n, wg, span, keys);
+        double mn, mx;
+        if (F.dtype == PA_F32) extrema_span<float>(static_cast<const float*>(F.data), F.L.n, wg, span, mn, mx);
+        else extrema_span<double>(static_cast<const double*>(F.data), F.L.n, wg, span, mn, mx);
+        if (threadIdx.x == 0) join_keys(mn, mx, keys);
         return;
     }
     b -= n_ext;
@@ -1721,12 +1733,16 @@ bool valid_dtype(int d) { return d == PA_F32 || d == PA_F64; }
 
 using namespace pa;
 
+// extrema workgroups of pa_extrema_autotune at most, each with its result in
+// the workspace after the tuner's partial sums
+constexpr int kExtParts = 2048;
+
 extern "C" size_t pa_autotune_workspace(const pa_layout* L) {
     int s[3], n[3];
     if (!L || !tune_axis(L->nx, &s[0], &n[0]) || !tune_axis(L->ny, &s[1], &n[1]) ||
         !tune_axis(L->nz, &s[2], &n[2]))
         return 0;
-    return sizeof(double) * 15 * (size_t)n[0] * n[1] * n[2];
+    return sizeof(double) * (15 * (size_t)n[0] * n[1] * n[2] + 2 * kExtParts);
 }
 
 extern "C" int pa_autotune(const void* d_data, int dtype, const pa_layout* L, double* d_scores15,
@@ -1740,7 +1756,7 @@ extern "C" int pa_autotune(const void* d_data, int dtype, const pa_layout* L, do
         return PA_OK;
     }
     const int nblocks = n[0] * n[1] * n[2];
-    if (ws_bytes < pa_autotune_workspace(L) || !d_ws) return PA_ERR_WORKSPACE;
+    if (ws_bytes < sizeof(double) * 15 * (size_t)nblocks || !d_ws) return PA_ERR_WORKSPACE;
     double* part = static_cast<double*>(d_ws);
     Geom g = make_geom(L);
     dim3 grid(nblocks, 15);
@@ -1773,31 +1789,32 @@ extern "C" int pa_extrema_autotune(const void* d_data, int dtype, const pa_layou
     if (ws_bytes < pa_autotune_workspace(L) || !d_ws) return PA_ERR_WORKSPACE;
     hipStream_t st = as_stream(stream);
     double* part = static_cast<double*>(d_ws);
-    unsigned long long* keys = reinterpret_cast<unsigned long long*>(d_minmax + 2);  // after the result, as pa_extrema
-    hipLaunchKernelGGL(extrema_keys_init_kernel, dim3(1), dim3(1), 0, st, keys);
-    PA_LAUNCH_CHECK();
+    double* ext_part = part + 15 * (size_t)nblocks;
     // the tuner's LDS tile leaves three workgroups per CU; the extrema are cut
-    // into 8 workgroups per CU, queued behind the tuner blocks (measured
+    // into up to 8 workgroups per CU, queued behind the tuner blocks (measured
     // against 4 per CU and against exactly the slots the tuner leaves: the
-    // step was 1 % faster)
+    // step was 1 % faster), of at least one full batch of loads each.  Each
+    // leaves its result in the workspace: 2048 workgroups of a 64^3 field, a
+    // few vectors each, had spent 40 us on atomics of one pair of keys.
     const int ntune = 15 * nblocks;
     const int64_t nv = L->n / (16 / dtype);
     int64_t ext = 8 * (int64_t)device_cus();
+    if (ext > kExtParts) ext = kExtParts;
     int64_t span = (nv + ext - 1) / ext;
-    if (span < 1) span = 1;
+    if (span < kExtBatch) span = kExtBatch;
     ext = (nv + span - 1) / span;
     if (ext < 1) ext = 1;  // the last extrema workgroup also takes the scalar tail
     const unsigned grid = (unsigned)(ntune + ext);
     Geom g = make_geom(L);
     if (dtype == PA_F32)
         hipLaunchKernelGGL(extrema_tune_kernel<float>, dim3(grid), dim3(kThreads), 0, st, (const float*)d_data, L->n,
-                           keys, span, g, s[0], s[1], s[2], n[0], n[1], nblocks, part);
+                           ext_part, span, g, s[0], s[1], s[2], n[0], n[1], nblocks, part);
     else
         hipLaunchKernelGGL(extrema_tune_kernel<double>, dim3(grid), dim3(kThreads), 0, st, (const double*)d_data,
-                           L->n, keys, span, g, s[0], s[1], s[2], n[0], n[1], nblocks, part);
+                           L->n, ext_part, span, g, s[0], s[1], s[2], n[0], n[1], nblocks, part);
     PA_LAUNCH_CHECK();
-    hipLaunchKernelGGL(extrema_tune_finish_kernel, dim3(1), dim3(64), 0, st, keys, d_minmax, part, nblocks, d_scores15,
-                       d_flags8, rel_eb, dtype, alpha_of(rel_eb), d_bounds);
+    hipLaunchKernelGGL(extrema_tune_finish_kernel, dim3(1), dim3(kFinishThreads), 0, st, ext_part, (int)ext, d_minmax,
+                       part, nblocks, d_scores15, d_flags8, rel_eb, dtype, alpha_of(rel_eb), d_bounds);
     PA_LAUNCH_CHECK();
     return PA_OK;
 }
