@@ -171,11 +171,29 @@ int pa_spline_reconstruct_planes(const void* d_qc, const int32_t* d_src, const u
  * decoupled look-back over the chunks before it and writes its bytes
  * straight into the stream.  Workspace (8-byte aligned): an int32 error
  * word in an 8-byte slot (non-zero only if a chunk gave up waiting for the
- * sizes before it, which in-order dispatch rules out), then one 8-byte
- * status word per chunk. */
+ * sizes before it, which in-order dispatch rules out), one 8-byte status
+ * word per chunk, then room for the code magnitudes of the calls below. */
 size_t pa_encode_workspace(const pa_layout* L);
 int pa_lossless_encode(const uint8_t* d_bp, const pa_layout* L, uint8_t* d_out, uint64_t* d_cum,
                        uint64_t* d_outsize, void* d_ws, size_t ws_bytes, void* stream);
+
+/* The same compression without moving planes that hold no bit (no reference
+ * counterpart): most leading bit-planes of a field are zero.  In this order on
+ * one stream, with one encoder workspace throughout: pa_encode_prepare clears
+ * it; pa_spline_construct_live is pa_spline_construct_dev and leaves the
+ * codes' magnitudes in it; pa_bitshuffle_live is pa_bitshuffle but may leave
+ * bytes of planes that these magnitudes show to be zero unwritten;
+ * pa_lossless_encode_live is pa_lossless_encode on such planes and does not read
+ * those bytes.  The stream equals the other calls'.  pa_live_planes: whether
+ * these calls are the faster ones for a field (large 3-D ones). */
+int pa_live_planes(const pa_layout* L);
+int pa_encode_prepare(const pa_layout* L, void* d_ws, size_t ws_bytes, void* stream);
+int pa_spline_construct_live(const void* d_data, int dtype, const pa_layout* L, const double* d_bounds,
+                             const uint8_t* d_flags8, int32_t* d_qc, void* d_anchors, void* d_ews, void* stream);
+int pa_bitshuffle_live(const int32_t* d_qc, const pa_layout* L, int mode, uint8_t* d_bp, const void* d_ews,
+                       void* stream);
+int pa_lossless_encode_live(const uint8_t* d_bp, const pa_layout* L, uint8_t* d_out, uint64_t* d_cum,
+                            uint64_t* d_outsize, void* d_ws, size_t ws_bytes, void* stream);
 
 /* compress_merge (compressor.cu:139-151): pads the stream to 8 bytes and
  * appends flags, range, size table and anchors; d_total receives the final

@@ -103,6 +103,11 @@ SIGNATURES = {
     "pa_spline_reconstruct_planes": (I32, [P, P, P, P, P, P, P, I32, LP, D, D, P, P, P, P]),
     "pa_encode_workspace": (SZ, [LP]),
     "pa_lossless_encode": (I32, [P, LP, P, P, P, P, SZ, P]),
+    "pa_live_planes": (I32, [LP]),
+    "pa_encode_prepare": (I32, [LP, P, SZ, P]),
+    "pa_spline_construct_live": (I32, [P, I32, LP, P, P, P, P, P, P]),
+    "pa_bitshuffle_live": (I32, [P, LP, I32, P, P, P]),
+    "pa_lossless_encode_live": (I32, [P, LP, P, P, P, P, SZ, P]),
     "pa_compress_merge": (I32, [P, LP, I32, P, P, P, P, P, P, P]),
     "pa_decode_workspace": (SZ, [LP]),
     "pa_lossless_decode": (I32, [P, I64, LP, P, P, SZ, P]),

@@ -53,7 +53,7 @@ FieldSizes field_sizes(const BatchField& f) {
     z.qc = up((size_t)L.code_len * 4);
     z.anchors = up((size_t)L.n4 * f.dtype);
     z.bp = up((size_t)L.host_size);
-    z.encws = up(((size_t)L.nchunks + 1) * 8);
+    z.encws = up(pa::encws_words(L.nchunks) * 8);
     z.cum = up(128 * sizeof(uint64_t));
     z.outsize = up(sizeof(uint64_t));
     return z;
@@ -115,6 +115,12 @@ int count_launches(const pa::BatchDev& b) {
 int build_descriptors(const pa_batch_field* fields, int nf, const std::vector<int>& order, uint8_t* ws,
                       uint64_t* d_result, std::vector<BatchField>& out, const std::vector<BatchField>* ref) {
     out.resize(nf);
+    int64_t codes = 0;  // of the 3-D fields, whose launches are one after another
+    for (int i = 0; i < nf; ++i) {
+        pa_layout L;
+        if (pa_layout_init(&L, fields[i].nx, fields[i].ny, fields[i].nz) == PA_OK && pa::live_dims(&L))
+            codes += L.code_len;
+    }
     size_t off = 0;
     for (int k = 0; k < nf; ++k) {
         const int i = order[k];
@@ -147,6 +153,7 @@ int build_descriptors(const pa_batch_field* fields, int nf, const std::vector<in
         b += z.bp;
         f.encws = reinterpret_cast<uint64_t*>(b);
         b += z.encws;
+        f.live = codes >= pa::kLiveCodes && pa::live_dims(&f.L) ? pa::live_words(f.encws, f.L.nchunks) : nullptr;
         f.cum = reinterpret_cast<uint64_t*>(b);
         b += z.cum;
         f.outsize = reinterpret_cast<uint64_t*>(b);

@@ -52,7 +52,7 @@ __device__ __forceinline__ int block_level(const Levels& v, int blk, int* first)
 
 template <int MODE>
 __device__ __forceinline__ void shuffle_block(const int32_t* __restrict__ qc, const Levels& v, uint8_t* __restrict__ bp,
-                                              int blk, int nblk, int32_t* stage) {
+                                              const uint64_t* __restrict__ live, int blk, int nblk, int32_t* stage) {
     int first;
     const int lv = block_level(v, blk, &first);
     const int64_t g0 = (int64_t)(blk - first) * kGroupsPerBlock;
@@ -66,6 +66,14 @@ __device__ __forceinline__ void shuffle_block(const int32_t* __restrict__ qc, co
     for (int k = 0; k < kPer; ++k) {
         const int64_t r = c0 + threadIdx.x + k * kThreads;
         c[k] = r < real ? src[r] : 0;
+    }
+    // planes whose rows of this block lie in no chunk that reaches past the
+    // level's zero planes are left unwritten (lane k tests plane k)
+    uint32_t skip = 0;
+    if (live) {
+        const ZeroSpan z = zero_spans(live, v.base, v.stride);
+        const int64_t a = v.base[lv] + (int64_t)(threadIdx.x & 31) * v.stride[lv] + g0;
+        skip = (uint32_t)__ballot(a - kCS >= z.lo[lv] && a + kGroupsPerBlock + kCS <= z.hi[lv]);
     }
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
@@ -84,7 +92,8 @@ __device__ __forceinline__ void shuffle_block(const int32_t* __restrict__ qc, co
         transpose32(a);
         uint8_t* row = bp + v.base[lv] + g;
 #pragma unroll
-        for (int k = 0; k < 32; ++k) *reinterpret_cast<uint32_t*>(row + k * v.stride[lv]) = a[31 - k];
+        for (int k = 0; k < 32; ++k)
+            if (!((skip >> k) & 1u)) *reinterpret_cast<uint32_t*>(row + k * v.stride[lv]) = a[31 - k];
     }
     if (blk == nblk - 1) {  // bytes between the device and host layouts
         for (int64_t i = v.dev_size + 4 * threadIdx.x; i < v.host_size; i += 4 * kThreads)
@@ -94,9 +103,9 @@ __device__ __forceinline__ void shuffle_block(const int32_t* __restrict__ qc, co
 
 template <int MODE>
 __global__ __launch_bounds__(kThreads) void shuffle_kernel(const int32_t* __restrict__ qc, Levels v,
-                                                           uint8_t* __restrict__ bp) {
+                                                           uint8_t* __restrict__ bp, const uint64_t* __restrict__ live) {
     __shared__ int32_t stage[kThreads * kRow];
-    shuffle_block<MODE>(qc, v, bp, blockIdx.x, gridDim.x, stage);
+    shuffle_block<MODE>(qc, v, bp, live, blockIdx.x, gridDim.x, stage);
 }
 
 // one launch over the shuffle workgroups of every field of a batch
@@ -106,8 +115,8 @@ __global__ __launch_bounds__(kThreads) void batch_shuffle_kernel(const BatchFiel
     const int f = find_field(prefix, 0, nf, blockIdx.x);
     const BatchField& F = fields[f];
     const int blk = (int)(blockIdx.x - prefix[f]), nblk = (int)(prefix[f + 1] - prefix[f]);
-    if (F.mode == PA_MODE_NB) shuffle_block<PA_MODE_NB>(F.qc, F.lv, F.bp, blk, nblk, stage);
-    else shuffle_block<PA_MODE_SM>(F.qc, F.lv, F.bp, blk, nblk, stage);
+    if (F.mode == PA_MODE_NB) shuffle_block<PA_MODE_NB>(F.qc, F.lv, F.bp, F.live, blk, nblk, stage);
+    else shuffle_block<PA_MODE_SM>(F.qc, F.lv, F.bp, F.live, blk, nblk, stage);
 }
 
 // Inverse; WINDOW restricts each level to planes [begin[lr], end[lr]) (plus
@@ -288,16 +297,29 @@ __global__ __launch_bounds__(kThreads) void retr_unshuffle_kernel(const RetrJob*
 
 using namespace pa;
 
-extern "C" int pa_bitshuffle(const int32_t* d_qc, const pa_layout* L, int mode, uint8_t* d_bp, void* stream) {
+static int launch_shuffle(const int32_t* d_qc, const pa_layout* L, int mode, uint8_t* d_bp, const uint64_t* live,
+                          void* stream) {
     if (!L || !d_qc || !d_bp || (mode != PA_MODE_NB && mode != PA_MODE_SM)) return PA_ERR_ARG;
     Levels v = make_levels(L);
     hipStream_t st = as_stream(stream);
     if (mode == PA_MODE_NB)
-        hipLaunchKernelGGL(shuffle_kernel<PA_MODE_NB>, dim3(v.blk_start[4]), dim3(kThreads), 0, st, d_qc, v, d_bp);
+        hipLaunchKernelGGL(shuffle_kernel<PA_MODE_NB>, dim3(v.blk_start[4]), dim3(kThreads), 0, st, d_qc, v, d_bp, live);
     else
-        hipLaunchKernelGGL(shuffle_kernel<PA_MODE_SM>, dim3(v.blk_start[4]), dim3(kThreads), 0, st, d_qc, v, d_bp);
+        hipLaunchKernelGGL(shuffle_kernel<PA_MODE_SM>, dim3(v.blk_start[4]), dim3(kThreads), 0, st, d_qc, v, d_bp, live);
     PA_LAUNCH_CHECK();
     return PA_OK;
+}
+
+extern "C" int pa_bitshuffle(const int32_t* d_qc, const pa_layout* L, int mode, uint8_t* d_bp, void* stream) {
+    return launch_shuffle(d_qc, L, mode, d_bp, nullptr, stream);
+}
+
+extern "C" int pa_bitshuffle_live(const int32_t* d_qc, const pa_layout* L, int mode, uint8_t* d_bp, const void* d_ews,
+                                  void* stream) {
+    if (!L || !d_ews || ((uintptr_t)d_ews & 7) != 0) return PA_ERR_ARG;
+    const uint64_t* live =
+        live_dims(L) ? live_words(static_cast<uint64_t*>(const_cast<void*>(d_ews)), L->nchunks) : nullptr;
+    return launch_shuffle(d_qc, L, mode, d_bp, live, stream);
 }
 
 extern "C" int pa_inverse_bitshuffle(const uint8_t* d_bp, const pa_layout* L, int mode, int32_t* d_qc,

@@ -261,6 +261,7 @@ __device__ __forceinline__ bool re3_keep(uint32_t f2, int lane) {
 // Where an encoder writes: the stream, its cumulative size table and
 // length, the look-back status words and the error word.
 struct EncodeOut {
+    const uint64_t* live;  // code magnitudes (zero_spans), or null: every byte of the planes is there
     uint8_t* stream;
     uint64_t* cum;
     uint64_t* outsize;
@@ -290,6 +291,14 @@ __device__ __forceinline__ void encode_chunk(const uint8_t* __restrict__ bp, con
     const ChunkPos cp = chunk_pos(g, valid ? id : 0);
     const int osize = valid ? cp.osize : 0;
     const uint8_t* src = bp + cp.base;
+    // a chunk inside a level's zero planes is not read (nor was it written)
+    bool unread = false;
+    if (o.live) {
+        const ZeroSpan z = zero_spans(o.live, g.dbase, g.dstride);
+#pragma unroll
+        for (int lv = 0; lv < 4; ++lv) unread = unread || (cp.base >= z.lo[lv] && cp.base + cp.osize <= z.hi[lv]);
+    }
+    const int rsize = unread ? 0 : osize;  // bytes read
 
     // the whole chunk is requested before the first step (16 KiB per wave,
     // 64 registers per lane) so it costs one memory latency; it stays in
@@ -301,21 +310,27 @@ __device__ __forceinline__ void encode_chunk(const uint8_t* __restrict__ bp, con
         const int b = 16 * (64 * k + lane);
         lo8[k] = make_uint2(0u, 0u);
         hi8[k] = make_uint2(0u, 0u);
-        if (b < osize) {
+        if (b < rsize) {
             lo8[k] = *reinterpret_cast<const uint2*>(src + b);
-            if (b + 8 < osize) hi8[k] = *reinterpret_cast<const uint2*>(src + b + 8);
+            if (b + 8 < rsize) hi8[k] = *reinterpret_cast<const uint2*>(src + b + 8);
         }
     }
-    // zero-elimination bitmaps and the surviving-byte count
+    // zero-elimination bitmaps and the surviving-byte count (none of an
+    // all-zero chunk, whose bitmap nothing reads)
     int Z = 0;
+    uint32_t any = 0;
 #pragma unroll
-    for (int k = 0; k < kSteps; ++k) {
-        const uint32_t m = nz_bytes(lo8[k].x) | (nz_bytes(lo8[k].y) << 4) | (nz_bytes(hi8[k].x) << 8) |
-                           (nz_bytes(hi8[k].y) << 12);
-        W.b0[64 * k + lane] = (uint16_t)m;
-        const int c = __builtin_amdgcn_readlane(wave_incl_scan(__popc(m)), 63);  // the wave's total
-        if (lane == 0) W.zs[k] = c;
-        Z += c;
+    for (int k = 0; k < kSteps; ++k) any |= (lo8[k].x | lo8[k].y) | (hi8[k].x | hi8[k].y);
+    if (__ballot(any != 0)) {
+#pragma unroll
+        for (int k = 0; k < kSteps; ++k) {
+            const uint32_t m = nz_bytes(lo8[k].x) | (nz_bytes(lo8[k].y) << 4) | (nz_bytes(hi8[k].x) << 8) |
+                               (nz_bytes(hi8[k].y) << 12);
+            W.b0[64 * k + lane] = (uint16_t)m;
+            const int c = __builtin_amdgcn_readlane(wave_incl_scan(__popc(m)), 63);  // the wave's total
+            if (lane == 0) W.zs[k] = c;
+            Z += c;
+        }
     }
     bool fail = Z >= kAvail;
     wave_sync();
@@ -481,18 +496,20 @@ __global__ __launch_bounds__(64 * kW) void batch_encode_kernel(const BatchField*
     const int64_t gid0 = (int64_t)blockIdx.x * kW;
     const int f = find_field(prefix, 0, nf, gid0);
     const BatchField& F = fields[f];
-    const EncodeOut o{F.out, F.cum, F.outsize, F.encws + 1, reinterpret_cast<int32_t*>(F.encws)};
+    const EncodeOut o{F.live, F.out, F.cum, F.outsize, F.encws + 1, reinterpret_cast<int32_t*>(F.encws)};
     const int64_t id0 = gid0 - prefix[f];
     encode_chunk<kW>(F.bp, F.cg, o, id0, id0 / kW, slots[threadIdx.x >> 6], G);
 }
 
-// clears an encoder workspace: the error word, then the n status words
-__global__ void encode_clear_kernel(uint64_t* __restrict__ ws, int64_t n) {
+// clears an encoder workspace: the error word, then the n status words, and
+// the code magnitudes where they are in use
+__global__ void encode_clear_kernel(uint64_t* __restrict__ ws, int64_t n, int live) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i <= n) ws[i] = 0ull;
+    if (live && i < kLiveLines) live_words(ws, n)[i * kLiveStep] = 0ull;
 }
 
-// the same for every field of a batch (one thread per launch slot of a
+// the status words of every field of a batch (one thread per launch slot of a
 // chunk, plus one per field for its error word)
 __global__ void batch_encode_clear_kernel(const BatchField* __restrict__ fields, const int64_t* __restrict__ prefix,
                                           int nf, int64_t total) {
@@ -1043,30 +1060,61 @@ int pa::retr_decode(const RetrDev& r, hipStream_t st) {
     return PA_OK;
 }
 
-// the error word (an 8-byte slot), then the look-back status words (8 B per chunk)
+// the error word (an 8-byte slot), then the look-back status words (8 B per
+// chunk), then the code magnitudes
 extern "C" size_t pa_encode_workspace(const pa_layout* L) {
     if (!L) return 0;
-    return ((size_t)L->nchunks + 1) * 8;
+    return encws_words(L->nchunks) * 8;
+}
+
+static int encode_clear(const pa_layout* L, uint64_t* ws, int live, hipStream_t st) {
+    hipLaunchKernelGGL(encode_clear_kernel, dim3((unsigned)((L->nchunks + 1 + 255) / 256)), dim3(256), 0, st, ws,
+                       L->nchunks, live);
+    PA_LAUNCH_CHECK();
+    return PA_OK;
+}
+
+extern "C" int pa_live_planes(const pa_layout* L) { return L && live_dims(L) && L->code_len >= kLiveCodes; }
+
+extern "C" int pa_encode_prepare(const pa_layout* L, void* d_ws, size_t ws_bytes, void* stream) {
+    if (!L) return PA_ERR_ARG;
+    if (!d_ws || ws_bytes < pa_encode_workspace(L) || ((uintptr_t)d_ws & 7) != 0) return PA_ERR_WORKSPACE;
+    return encode_clear(L, static_cast<uint64_t*>(d_ws), 1, as_stream(stream));
 }
 
 // chunks per encoder workgroup (one per wave64)
 constexpr int kEncodeWaves = 4;
 
-extern "C" int pa_lossless_encode(const uint8_t* d_bp, const pa_layout* L, uint8_t* d_out, uint64_t* d_cum,
-                                  uint64_t* d_outsize, void* d_ws, size_t ws_bytes, void* stream) {
+// live: the planes come from pa_bitshuffle_live and the workspace from
+// pa_encode_prepare
+static int encode_common(const uint8_t* d_bp, const pa_layout* L, uint8_t* d_out, uint64_t* d_cum, uint64_t* d_outsize,
+                         void* d_ws, size_t ws_bytes, bool live, void* stream) {
     if (!L || !d_bp || !d_out || !d_cum || !d_outsize) return PA_ERR_ARG;
-    if (!d_ws || ws_bytes < pa_encode_workspace(L) || ((uintptr_t)d_ws & 7) != 0) return PA_ERR_WORKSPACE;
+    const size_t need = live ? pa_encode_workspace(L) : ((size_t)L->nchunks + 1) * 8;
+    if (!d_ws || ws_bytes < need || ((uintptr_t)d_ws & 7) != 0) return PA_ERR_WORKSPACE;
     hipStream_t st = as_stream(stream);
     ChunkGeom g = make_chunk_geom(L);
     uint64_t* ws = static_cast<uint64_t*>(d_ws);
-    hipLaunchKernelGGL(encode_clear_kernel, dim3((unsigned)((L->nchunks + 1 + 255) / 256)), dim3(256), 0, st, ws,
-                       L->nchunks);
-    PA_LAUNCH_CHECK();
-    EncodeOut o{d_out, d_cum, d_outsize, ws + 1, reinterpret_cast<int32_t*>(ws)};
+    if (!live) {  // (the words before the magnitudes: all that this form uses)
+        const int e = encode_clear(L, ws, 0, st);
+        if (e != PA_OK) return e;
+    }
+    const EncodeOut o{live && live_dims(L) ? live_words(ws, L->nchunks) : nullptr, d_out, d_cum, d_outsize, ws + 1,
+                      reinterpret_cast<int32_t*>(ws)};
     const unsigned eblocks = (unsigned)((L->nchunks + kEncodeWaves - 1) / kEncodeWaves);
     hipLaunchKernelGGL(encode_kernel<kEncodeWaves>, dim3(eblocks), dim3(64 * kEncodeWaves), 0, st, d_bp, g, o);
     PA_LAUNCH_CHECK();
     return PA_OK;
+}
+
+extern "C" int pa_lossless_encode(const uint8_t* d_bp, const pa_layout* L, uint8_t* d_out, uint64_t* d_cum,
+                                  uint64_t* d_outsize, void* d_ws, size_t ws_bytes, void* stream) {
+    return encode_common(d_bp, L, d_out, d_cum, d_outsize, d_ws, ws_bytes, false, stream);
+}
+
+extern "C" int pa_lossless_encode_live(const uint8_t* d_bp, const pa_layout* L, uint8_t* d_out, uint64_t* d_cum,
+                                       uint64_t* d_outsize, void* d_ws, size_t ws_bytes, void* stream) {
+    return encode_common(d_bp, L, d_out, d_cum, d_outsize, d_ws, ws_bytes, true, stream);
 }
 
 extern "C" int pa_compress_merge(uint8_t* d_out, const pa_layout* L, int dtype, const uint64_t* d_outsize,

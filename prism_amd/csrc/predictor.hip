@@ -454,6 +454,7 @@ struct SplineArgs {
     int gaps_on;  // (its workgroups share them out; disjoint from the codes)
     PlaneSrc ps;  // decompression: the round's bit-planes (ps.bp null: none)
     bool planes;  // resolved: the codes come from ps
+    uint64_t* live = nullptr;  // compression: where the codes' magnitudes go (live_words), or null
 };
 
 // Compression launches clear the code array's gaps alongside the tiles.
@@ -698,8 +699,12 @@ __device__ __forceinline__ void tile_run(const SplineArgs<T>& a, T* lds, int px,
     // loads return in issue order, so the code slots are filled while the
     // previous values (needed only at the output) are still in flight
     T prev[kOutIters];
+    uint64_t seen = 0;
     if constexpr (M == COMPRESS) {
+        seen = live_seen(a.live);
         tile_load(t, m, a.data);
+        seen = ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(seen >> 32)) << 32) |
+               __builtin_amdgcn_readfirstlane((uint32_t)seen);
         __syncthreads();
         if (lane_id() == 0 && bx < g.gx) a.anchors[bx + (int64_t)by * g.gx + (int64_t)bz * g.gx * g.gy] = t.s[0];
     } else {
@@ -728,7 +733,7 @@ __device__ __forceinline__ void tile_run(const SplineArgs<T>& a, T* lds, int px,
 
     tile_levels<T, M>(t, a.le, flags_mask(fl), maxlevel);
 
-    if constexpr (M == COMPRESS) codes_out(m);
+    if constexpr (M == COMPRESS) live_join(codes_out(m), seen, a.live);
     else tile_out(m, DELTA, (((uintptr_t)a.out | (uint64_t)g.nx * sizeof(T)) & 127) == 0, prev, a.out);
 }
 
@@ -1531,6 +1536,8 @@ __global__ __launch_bounds__(kThreads) void batch_front_kernel(const BatchField*
     const BatchField& F = fields[f];
     const int64_t k = i < n_chunk ? gid - p_chunk[f] : -1;  // status word k (-1: the error word)
     if (k < F.cg.nchunks) F.encws[1 + k] = 0ull;
+    if (k < 0 && F.live)  // with the error word: the code magnitudes
+        for (int w = 0; w < kLiveLines; ++w) F.live[w * kLiveStep] = 0ull;
 }
 
 // Per field, after the front launch: min and max from the extrema keys
@@ -1581,8 +1588,9 @@ __global__ __launch_bounds__((kGroupThreads<T, COMPRESS>)) __attribute__((amdgpu
     const int64_t gt = base + (xcd_order ? xcd * per + (xcd < extra ? xcd : extra) + b / kXcds : b);
     const int f = find_field(prefix, lo, hi, gt);
     const BatchField& F = fields[f];
-    const SplineArgs<T> a{static_cast<const T*>(F.data), F.g, load_level_ebs<T>(F.ebinfo), nullptr, nullptr, false,
-                          F.flags, nullptr, F.qc, nullptr, static_cast<T*>(F.anchors), nullptr, nullptr, nullptr};
+    SplineArgs<T> a{static_cast<const T*>(F.data), F.g, load_level_ebs<T>(F.ebinfo), nullptr, nullptr, false,
+                    F.flags, nullptr, F.qc, nullptr, static_cast<T*>(F.anchors), nullptr, nullptr, nullptr};
+    a.live = F.live;
     const Geom& g = a.g;
     const int64_t tix = gt - prefix[f];
     if (line_field(g)) {  // one unit per 256 lanes
@@ -1688,7 +1696,8 @@ template <typename T, int M>
 int launch_spline(const pa_layout* L, const T* data, double eb, double rel_eb, const uint8_t* flags8,
                   const int32_t* d_maxlevel, int32_t* qc_out, const int32_t* qc_in, T* anchors,
                   const T* anchors_in, const T* old, T* out, hipStream_t st, const double* le_dev = nullptr,
-                  const int32_t* narrow = nullptr, const Gaps* gaps = nullptr, const PlaneSrc* ps = nullptr) {
+                  const int32_t* narrow = nullptr, const Gaps* gaps = nullptr, const PlaneSrc* ps = nullptr,
+                  uint64_t* live = nullptr) {
     Geom g = make_geom(L);
     const int64_t ntiles = (int64_t)g.gx * g.gy * g.gz;
     if (ntiles > 0x7fffffff) return PA_ERR_ARG;
@@ -1700,6 +1709,7 @@ int launch_spline(const pa_layout* L, const T* data, double eb, double rel_eb, c
         args.gaps_on = 1;
     }
     if (ps) args.ps = *ps;
+    args.live = live;
     if (line_field(g))
         hipLaunchKernelGGL((line_kernel<T, M>), dim3((unsigned)((ntiles + kLineTiles - 1) / kLineTiles)),
                            dim3(kThreads), 0, st, args);
@@ -1844,18 +1854,31 @@ extern "C" int pa_level_bounds(const double* d_minmax, double eb, int dtype, dou
     return PA_OK;
 }
 
-extern "C" int pa_spline_construct_dev(const void* d_data, int dtype, const pa_layout* L, const double* d_bounds,
-                                       const uint8_t* d_flags8, int32_t* d_qc, void* d_anchors, void* stream) {
+static int construct_dev(const void* d_data, int dtype, const pa_layout* L, const double* d_bounds,
+                         const uint8_t* d_flags8, int32_t* d_qc, void* d_anchors, uint64_t* live, void* stream) {
     if (!L || !d_data || !d_bounds || !d_flags8 || !d_qc || !d_anchors || !valid_dtype(dtype)) return PA_ERR_ARG;
     hipStream_t st = as_stream(stream);
     const Gaps gaps = make_gaps(L);
     if (dtype == PA_F32)
         return launch_spline<float, COMPRESS>(L, (const float*)d_data, 0.0, 0.0, d_flags8, nullptr, d_qc, nullptr,
                                               (float*)d_anchors, nullptr, nullptr, nullptr, st, d_bounds, nullptr,
-                                              &gaps);
+                                              &gaps, nullptr, live);
     return launch_spline<double, COMPRESS>(L, (const double*)d_data, 0.0, 0.0, d_flags8, nullptr, d_qc, nullptr,
                                            (double*)d_anchors, nullptr, nullptr, nullptr, st, d_bounds, nullptr,
-                                           &gaps);
+                                           &gaps, nullptr, live);
+}
+
+extern "C" int pa_spline_construct_dev(const void* d_data, int dtype, const pa_layout* L, const double* d_bounds,
+                                       const uint8_t* d_flags8, int32_t* d_qc, void* d_anchors, void* stream) {
+    return construct_dev(d_data, dtype, L, d_bounds, d_flags8, d_qc, d_anchors, nullptr, stream);
+}
+
+extern "C" int pa_spline_construct_live(const void* d_data, int dtype, const pa_layout* L, const double* d_bounds,
+                                        const uint8_t* d_flags8, int32_t* d_qc, void* d_anchors, void* d_ews,
+                                        void* stream) {
+    if (!L || !d_ews || ((uintptr_t)d_ews & 7) != 0) return PA_ERR_ARG;
+    return construct_dev(d_data, dtype, L, d_bounds, d_flags8, d_qc, d_anchors,
+                         live_words(static_cast<uint64_t*>(d_ews), L->nchunks), stream);
 }
 
 extern "C" int pa_spline_reconstruct(const int32_t* d_qc, const void* d_anchors, int dtype, const pa_layout* L,

@@ -4,6 +4,8 @@
 // so the compressor and the decompressor reproduce identical values.
 #pragma once
 
+#include <rocprim/warp/warp_reduce.hpp>
+
 #include "common.hpp"
 
 namespace pa {
@@ -85,6 +87,55 @@ __device__ __forceinline__ int32_t quantize_val(T& v, T pred, T eb_r, T ebx2) {
     code = (T)qv;
     v = pred + code * ebx2;
     return qv;
+}
+
+// Range of the codes that a lane stores, 0 included: a code passes through and
+// is counted (two instructions for two codes: the compiler joins the
+// comparisons of a pair; an OR of the magnitudes took three a code, 8 % of the
+// tile kernels' instructions).
+struct CodeRange {
+    int32_t lo = 0, hi = 0;
+    __device__ __forceinline__ int32_t operator()(int32_t c) {
+        lo = min(lo, c);
+        hi = max(hi, c);
+        return c;
+    }
+    // the bits of the largest magnitudes c ^ (c >> 31)
+    __device__ __forceinline__ uint32_t mags() const { return (uint32_t)hi | (uint32_t)(lo ^ (lo >> 31)); }
+};
+struct Mags {
+    CodeRange fine, coarse;  // level 0's, the other levels'
+};
+
+// A wave's part in live_words: its XCD's word as it was when the wave began
+// (read with the wave's first loads), and its own magnitudes joined at the end.
+// The bits settle after a few workgroups, so nearly every wave finds them
+// there and ends without another access; the others read the word again
+// before they pay for an atomic.
+struct OrU32 {
+    __device__ uint32_t operator()(uint32_t a, uint32_t b) const { return a | b; }
+};
+__device__ __forceinline__ unsigned long long* live_word(uint64_t* live) {
+    return reinterpret_cast<unsigned long long*>(live) + (blockIdx.x % kLiveLines) * kLiveStep;
+}
+__device__ __forceinline__ uint64_t live_seen(uint64_t* live) {
+    return live ? __hip_atomic_load(live_word(live), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) : ~0ull;
+}
+__device__ __forceinline__ uint32_t wave_or(uint32_t v) {
+    using Reduce = rocprim::warp_reduce<uint32_t, 64>;  // (DPP: no LDS)
+    typename Reduce::storage_type storage;
+    uint32_t out;
+    Reduce().reduce(v, out, storage, OrU32());
+    return __builtin_amdgcn_readfirstlane(out);
+}
+__device__ __forceinline__ void live_join(const Mags& g, uint64_t seen, uint64_t* live) {
+    if (!live) return;
+    const uint32_t fine = g.fine.mags(), coarse = g.coarse.mags();
+    if (__ballot(((fine & ~(uint32_t)seen) | (coarse & ~(uint32_t)(seen >> 32))) != 0) == 0) return;
+    const uint64_t all = ((uint64_t)wave_or(coarse) << 32) | wave_or(fine);
+    if ((threadIdx.x & 63) != 0) return;
+    unsigned long long* w = live_word(live);
+    if (all & ~__hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicOr(w, (unsigned long long)all);
 }
 
 // In a decompressing tile a point's slot holds the bit pattern of its code

@@ -546,9 +546,11 @@ struct Columns0 {
 // Level 0: a row lane takes its column's z = 0..15 (rows of 16 or 8 adjacent
 // codes per tile).  Level 1: the group's points with even coordinates, in two
 // passes of 8 adjacent codes per tile and row; levels 2 and 3 in one.
+// Returns the magnitudes of the lane's codes (live_words).
 template <typename T, bool IN>
-__device__ __forceinline__ void codes_out(const Tile<T, IN>& m) {
+__device__ __forceinline__ Mags codes_out(const Tile<T, IN>& m) {
     constexpr int P = kGroup<T, COMPRESS>;
+    Mags g;
     {
         const RowLane<P> r;
         if (m.template in<0>(r.X) && m.template in<1>(r.y)) {
@@ -557,8 +559,8 @@ __device__ __forceinline__ void codes_out(const Tile<T, IN>& m) {
             const bool on_even = (r.X | r.y) & 1;
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
-                if (m.template in<2>(2 * k + 1)) c.at_odd() = slot_code(src[(2 * k + 1) * kZP]);
-                if (on_even && m.template in<2>(2 * k)) c.at_even() = slot_code(src[2 * k * kZP]);
+                if (m.template in<2>(2 * k + 1)) c.at_odd() = g.fine(slot_code(src[(2 * k + 1) * kZP]));
+                if (on_even && m.template in<2>(2 * k)) c.at_even() = g.fine(slot_code(src[2 * k * kZP]));
                 c.next();
             }
         }
@@ -568,17 +570,18 @@ __device__ __forceinline__ void codes_out(const Tile<T, IN>& m) {
     for (int it = 0; it < 2; ++it) {
         const int X = 2 * (v & (8 * P - 1)), y = 2 * ((v / (8 * P)) & 7), z = 2 * (v / (64 * P) + 4 * it);
         if (((X | y | z) & 2) && m.in3(X, y, z))
-            m.qc_out[lm_at<1>(m, X, y, z)] = slot_code(m.s[(X >> 4) * kTileLds + tslot(X & 15, y, z)]);
+            m.qc_out[lm_at<1>(m, X, y, z)] = g.coarse(slot_code(m.s[(X >> 4) * kTileLds + tslot(X & 15, y, z)]));
     }
     if (v < 64 * P) {
         const int X = 4 * (v & (4 * P - 1)), y = 4 * ((v / (4 * P)) & 3), z = 4 * (v / (16 * P));
         if (((X | y | z) & 4) && m.in3(X, y, z))
-            m.qc_out[lm_at<2>(m, X, y, z)] = slot_code(m.s[(X >> 4) * kTileLds + tslot(X & 15, y, z)]);
+            m.qc_out[lm_at<2>(m, X, y, z)] = g.coarse(slot_code(m.s[(X >> 4) * kTileLds + tslot(X & 15, y, z)]));
     } else if (v < 64 * P + 8 * P) {
         const int w = v - 64 * P, X = 8 * (w & (2 * P - 1)), y = 8 * ((w / (2 * P)) & 1), z = 8 * (w / (4 * P));
         if (((X | y | z) & 8) && m.in3(X, y, z))
-            m.qc_out[lm_at<3>(m, X, y, z)] = slot_code(m.s[(X >> 4) * kTileLds + tslot(X & 15, y, z)]);
+            m.qc_out[lm_at<3>(m, X, y, z)] = g.coarse(slot_code(m.s[(X >> 4) * kTileLds + tslot(X & 15, y, z)]));
     }
+    return g;
 }
 
 // The three stages of one level (InterpolationPredictor.cu:1940-2025); a, b:

@@ -206,6 +206,11 @@ def compress(data: torch.Tensor, eb: float, rel: bool = True, progressive: bool 
     p_bounds, p_ews, p_mm, p_scores, p_flags, p_cum, p_sizes, p_tws = (
         V(sp), V(sp + 128), V(sp + e), V(sp + e + 32), V(sp + e + 152), V(sp + e + 160), V(sp + e + 1184),
         V(sp + e + 1216))
+    # planes that hold no bit are neither written nor read where that pays, but
+    # where the planes are handed out
+    live = not return_parts and bool(lib().pa_live_planes(C.byref(L)))
+    if live:
+        check(lib().pa_encode_prepare(C.byref(L), p_ews, ews_bytes, st), "pa_encode_prepare")
     if rel:  # extrema, auto-tuning and the level bounds share one launch sequence
         with tm("extrema"):
             check(lib().pa_extrema_autotune(_p(data), dt, C.byref(L), p_mm, float(eb), p_bounds, p_scores, p_flags,
@@ -217,17 +222,24 @@ def compress(data: torch.Tensor, eb: float, rel: bool = True, progressive: bool 
     qc = torch.empty(L.code_len, dtype=torch.int32, device=dev)
     anchors = torch.empty(L.n4, dtype=data.dtype, device=dev)
     with tm("predict"):
-        check(lib().pa_spline_construct_dev(_p(data), dt, C.byref(L), p_bounds, p_flags, _p(qc), _p(anchors), st),
-              "pa_spline_construct_dev")
+        if live:
+            check(lib().pa_spline_construct_live(_p(data), dt, C.byref(L), p_bounds, p_flags, _p(qc), _p(anchors), p_ews,
+                                                 st), "pa_spline_construct_live")
+        else:
+            check(lib().pa_spline_construct_dev(_p(data), dt, C.byref(L), p_bounds, p_flags, _p(qc), _p(anchors), st),
+                  "pa_spline_construct_dev")
     bp = _empty(L.host_size)
     mode = PA_MODE_NB if progressive else PA_MODE_SM
     with tm("shuffle"):
-        check(lib().pa_bitshuffle(_p(qc), C.byref(L), mode, _p(bp), st), "pa_bitshuffle")
+        if live:
+            check(lib().pa_bitshuffle_live(_p(qc), C.byref(L), mode, _p(bp), p_ews, st), "pa_bitshuffle_live")
+        else:
+            check(lib().pa_bitshuffle(_p(qc), C.byref(L), mode, _p(bp), st), "pa_bitshuffle")
     bound = lib().pa_compress_bound(C.byref(L), dt)
     out = _empty(bound)
+    encode = lib().pa_lossless_encode_live if live else lib().pa_lossless_encode
     with tm("encode"):
-        check(lib().pa_lossless_encode(_p(bp), C.byref(L), _p(out), p_cum, p_sizes, p_ews, ews_bytes, st),
-              "pa_lossless_encode")
+        check(encode(_p(bp), C.byref(L), _p(out), p_cum, p_sizes, p_ews, ews_bytes, st), "pa_lossless_encode")
     with tm("merge"):  # the stream length goes to bounds[15] (int64 bits)
         check(lib().pa_compress_merge(_p(out), C.byref(L), dt, p_sizes, p_flags, V(sp + 8), p_cum, _p(anchors),
                                       V(sp + 120), st), "pa_compress_merge")
