@@ -59,9 +59,10 @@ def _empty(nbytes: int, dtype=torch.uint8):
 _TLS = threading.local()
 
 
-def _host_read(t: torch.Tensor) -> np.ndarray:
-    """Copies a small device tensor to the host through a pinned per-thread
-    buffer and waits for the current stream; returns a fresh numpy copy."""
+def _host_copy(t: torch.Tensor) -> torch.Tensor:
+    """Queues the copy of a small device tensor to the pinned buffer of this
+    thread; the values are there once the caller has waited for it, until the
+    thread's next copy."""
     nb = t.numel() * t.element_size()
     buf = getattr(_TLS, "pinned", None)
     if buf is None or buf.numel() < nb:
@@ -69,6 +70,13 @@ def _host_read(t: torch.Tensor) -> np.ndarray:
         _TLS.pinned = buf
     h = buf[:nb].view(t.dtype)
     h.copy_(t.reshape(-1), non_blocking=True)
+    return h
+
+
+def _host_read(t: torch.Tensor) -> np.ndarray:
+    """Copies a small device tensor to the host and waits for the current
+    stream; returns a fresh numpy copy."""
+    h = _host_copy(t)
     torch.cuda.current_stream().synchronize()
     return h.numpy().copy()
 
@@ -359,17 +367,23 @@ class BatchCompressor:
         mode) raises, or gives None when not `strict`."""
         if self._done is not None:
             self._done.synchronize()
-        r = self._res_host.view(-1, 4)
+        # the result table as host numbers and the streams as one split of the
+        # buffer (stream, gap, stream, ...): single elements and slices of
+        # tensors took 6 us a field
+        r = self._res_host.numpy().reshape(-1, 4)
+        totals, statuses, ranges = r[:, 0].tolist(), r[:, 1].tolist(), r[:, 2].copy().view(np.float64).tolist()
+        bad = [i for i, status in enumerate(statuses) if status != 0]
+        if bad and strict:
+            raise _lib.PrismError(f"batch field {bad[0]}: non-positive error bound (constant field in REL mode?)")
+        sizes = []
+        for off, nxt, total, status in zip(self.offs, self.offs[1:] + [self.outbuf.numel()], totals, statuses):
+            total = total if status == 0 else 0
+            sizes += [total, nxt - off - total]
         out = []
-        for i in range(self.nf):
-            total, status = int(r[i, 0]), int(r[i, 1])
-            if status != 0:
-                if strict:
-                    raise _lib.PrismError(f"batch field {i}: non-positive error bound (constant field in REL mode?)")
+        for i, (s, rng) in enumerate(zip(self.outbuf.split(sizes)[::2], ranges)):
+            if statuses[i] != 0:
                 out.append(None)
                 continue
-            rng = float(r[i, 2:3].view(torch.float64).item())
-            s = self.outbuf[self.offs[i]:self.offs[i] + total]
             out.append(Compressed(stream=s, shape=self.shapes[i], dtype=self.dtypes[i], eb_input=float(self._ebs[i]),
                                   rel=self.rel, progressive=self.progressive, range=rng if self.rel else 1.0))
         return out
@@ -428,9 +442,11 @@ def decompress(c: Compressed, check_stream: bool = True) -> torch.Tensor:
     dt = DTYPES[c.dtype]
     st = _stream()
     t0, flags, cum, anchors = _trailer(c, L)
-    rng = stream_range(c)
-    eb_abs = c.eb_input * rng if c.rel else c.eb_input
-    rel_eb = c.eb_input if c.rel else 0.0
+    # the range is copied ahead of the decoder and waited for behind its
+    # launches, which do not need it
+    rng = _host_copy(c.stream[t0 + 8:t0 + 16].view(torch.float64))
+    copied = torch.cuda.Event()
+    copied.record()
     bp = _empty(L.host_size)
     ws = _empty(lib().pa_decode_workspace(C.byref(L)))
     check(lib().pa_lossless_decode(_p(c.stream), c.nbytes, C.byref(L), _p(bp), _p(ws), ws.numel(), st), "pa_lossless_decode")
@@ -438,6 +454,9 @@ def decompress(c: Compressed, check_stream: bool = True) -> torch.Tensor:
     mode = PA_MODE_NB if c.progressive else PA_MODE_SM
     check(lib().pa_inverse_bitshuffle(_p(bp), C.byref(L), mode, _p(qc), st), "pa_inverse_bitshuffle")
     out = torch.empty((nz, ny, nx), dtype=c.dtype, device=c.stream.device)
+    copied.synchronize()
+    eb_abs = c.eb_input * float(rng[0]) if c.rel else c.eb_input
+    rel_eb = c.eb_input if c.rel else 0.0
     check(lib().pa_spline_reconstruct(_p(qc), _p(anchors), dt, C.byref(L), eb_abs, rel_eb, _p(flags), None,
                                       _p(out), st), "pa_spline_reconstruct")
     if check_stream:
@@ -465,11 +484,12 @@ class Retriever:
         self.range = c.range if c.range is not None else stream_range(c)
         self.eb_abs = c.eb_input * self.range if c.rel else c.eb_input
         self.rel_eb = c.eb_input if c.rel else 0.0
-        # state (begin[4] end[4] maxlevel narrow, int32[16]) and the byte
-        # counter (int64) in one zero-filled block; views on demand
-        self._small = torch.zeros(18, dtype=torch.int32, device=dev)
-        # the strategy search's best key and arrival count (zero before first use)
-        self.sws = torch.zeros(lib().pa_strategy_workspace(), dtype=torch.uint8, device=dev)
+        # state (begin[4] end[4] maxlevel narrow, int32[16]), the byte counter
+        # (int64) and, from byte 128, the strategy search's best key and arrival
+        # count in one zero-filled block (one allocation and launch a field)
+        sws_bytes = lib().pa_strategy_workspace()
+        self._small = torch.zeros(32 + (sws_bytes + 3) // 4, dtype=torch.int32, device=dev)
+        self.sws = self._small[32:].view(torch.uint8)[:sws_bytes]
         self._bufs = None  # bit-planes, codes and decoder workspace, allocated on first use
         self.out = None
         self.rounds = 0
@@ -487,28 +507,34 @@ class Retriever:
                        anchors=V(sb + self.t0 + 1040), flags=V(sb + self.t0), L=C.byref(self.L))
 
     def _buffers(self):
-        """(bp, qc, dws), allocated at first use: the first round's strategy
-        search is already queued by then."""
+        """The bit-planes, codes and decoder workspace, allocated at first use
+        (the first round's strategy search is already queued by then) as one
+        block; returns their addresses."""
         if self._bufs is None:
-            dev = self._small.device
-            bp = _empty(self.L.host_size)
-            qc = torch.empty(self.L.code_len, dtype=torch.int32, device=dev)
-            dws = _empty(lib().pa_decode_workspace(C.byref(self.L)))
-            self._bufs = (bp, qc, dws)
-            self._a.update(bp=_p(bp), qc=_p(qc), dws=_p(dws))
-        return self._bufs
+            up = lambda n: (n + 511) // 512 * 512
+            self._qc_at = up(self.L.host_size)
+            self._dws_at = self._qc_at + up(4 * self.L.code_len)
+            self._dws_bytes = lib().pa_decode_workspace(C.byref(self.L))
+            self._bufs = torch.empty(self._dws_at + self._dws_bytes, dtype=torch.uint8, device=self._small.device)
+            p = self._bufs.data_ptr()
+            self._at = (p, p + self._qc_at, p + self._dws_at)
+            self._a.update(zip(("bp", "qc", "dws"), map(C.c_void_p, self._at)))
+        return self._at
 
     @property
     def bp(self):
-        return self._buffers()[0]
+        self._buffers()
+        return self._bufs[:self.L.host_size]
 
     @property
     def qc(self):
-        return self._buffers()[1]
+        self._buffers()
+        return self._bufs[self._qc_at:self._qc_at + 4 * self.L.code_len].view(torch.int32)
 
     @property
     def dws(self):
-        return self._buffers()[2]
+        self._buffers()
+        return self._bufs[self._dws_at:]
 
     # views of the device state and of the trailer
     @property
@@ -554,7 +580,7 @@ class Retriever:
         the field reports it."""
         if self._bufs is None:
             return 0
-        return _decoder_error(self._bufs[2])
+        return _decoder_error(self.dws)
 
     def check(self) -> None:
         """Raises PrismError if a round of this field met a malformed chunk."""
@@ -575,10 +601,10 @@ class Retriever:
         with tm("strategy"):
             check(lb.pa_find_strategy(a["cum"], a["begin"], a["end"], a["maxlevel"], self.eb_abs, target_abs,
                                       a["sws"], self.sws.numel(), st), "pa_find_strategy")
-        dws = self._buffers()[2]
+        self._buffers()
         with tm("decode"):
             check(lb.pa_lossless_decode_window(a["stream"], self.c.nbytes, a["L"], a["begin"], a["end"], a["bp"],
-                                               a["bytes_read"], int(self.rounds > 0), a["dws"], dws.numel(), st),
+                                               a["bytes_read"], int(self.rounds > 0), a["dws"], self._dws_bytes, st),
                   "pa_lossless_decode_window")
         with tm("unshuffle"):
             # no codes written when the reconstruction reads the planes itself
@@ -604,8 +630,8 @@ class Retriever:
         desc.eb, desc.rel_eb = self.eb_abs, self.rel_eb
         desc.target = target * self.range if c.rel else target
         sp = self._small.data_ptr()
-        desc.state, desc.bp, desc.qc = sp, self.bp.data_ptr(), self.qc.data_ptr()
-        desc.dws, desc.bytes_read = self.dws.data_ptr(), sp + 64
+        desc.state, desc.bytes_read = sp, sp + 64
+        desc.bp, desc.qc, desc.dws = self._buffers()
         desc.round = self.rounds
         desc.old = self.out.data_ptr() if self.out is not None else None
         desc.out = out.data_ptr()
@@ -658,7 +684,7 @@ def retrieve_batch(items, pinned: bool = False) -> RetrievalBatch:
     outs = []
     for k, (r, target) in enumerate(items):
         nx, ny, nz = r.c.shape
-        new = torch.empty((nz, ny, nx), dtype=r.c.dtype, device=r.qc.device)
+        new = torch.empty((nz, ny, nx), dtype=r.c.dtype, device=r.c.stream.device)
         r.job(float(target), new, arr[k])
         outs.append(new)
     ws = _empty(lib().pa_retrieve_workspace(nj))
