@@ -79,56 +79,113 @@ __device__ __forceinline__ int block_scan(int v, int* lds, int* total) {
 }
 
 
-// 4-bit mask of the non-zero bytes of w
+// a byte 1 for each non-zero byte of w, 0 for the others
+__device__ __forceinline__ uint32_t nz_ones(uint32_t w) {
+    return ((((w & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | w) >> 7) & 0x01010101u;
+}
+// 4-bit mask of the non-zero bytes of w, 8-bit mask of those of w0, w1 (byte
+// products gather the bits in one instruction a word)
 __device__ __forceinline__ uint32_t nz_bytes(uint32_t w) {
-    const uint32_t h = (((w & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | w) & 0x80808080u;
-    return ((h >> 7) & 1u) | ((h >> 14) & 2u) | ((h >> 21) & 4u) | ((h >> 28) & 8u);
+    return __builtin_amdgcn_udot4(nz_ones(w), 0x08040201u, 0u, false);
+}
+__device__ __forceinline__ uint32_t nz_bytes2(uint32_t w0, uint32_t w1) {
+    return __builtin_amdgcn_udot4(nz_ones(w1), 0x80402010u, nz_bytes(w0), false);
 }
 
 // keep the ordering of LDS accesses of one wave across phases
 __device__ __forceinline__ void wave_sync() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); __builtin_amdgcn_wave_barrier(); }
 
-// LDS of one wave: the zero-elimination bitmap, one step's bytes and the
-// repetition-elimination bytes with the footer.  The surviving bytes go to
-// the stream step by step, so a wave needs 5.5 KiB of LDS (an encoded chunk
-// held whole would need 16 KiB and cap the encoder at two waves per SIMD).
+// LDS of one wave: the zero-elimination bitmap and a ring that the encoded
+// bytes pass through (with 6 KiB a wave the registers, not the LDS, set the
+// waves on a CU; an encoded chunk held whole would need 16 KiB).
+constexpr int kRing = 4096, kFlush = 1024;            // bytes; the ring is emptied from kFlush on
 constexpr int kTailBytes = 2048 + 256 + 32 + 4 + 2;  // RE1 + RE2 + RE3 kept bytes, B3, size
+static_assert(kFlush + 1024 + 16 <= kRing && kFlush + 16 + kTailBytes <= kRing, "a step or the tail fits behind what waits");
 struct __align__(16) WaveSlot {
     uint16_t b0[kCS / 16];  // zero-elimination bitmap: 2 bytes per 16-byte segment
-    // a step's bytes: the zero-eliminated form keeps the (< 4) bytes carried
-    // from the previous step's last partial word in front of its surviving
-    // bytes; a raw chunk puts the previous step's last word at 12..16 and
-    // the step's 1 KiB from byte 16 (plus one word of slack)
-    uint8_t step[16 + 1024 + 16];
-    // the RE bytes, B3 and footer from byte 4, after up to 4 bytes that
-    // carry the last partial word of the zero-eliminated bytes (plus slack
-    // for the funnel reads of the last word)
-    uint8_t tail[(4 + kTailBytes + 8 + 15) / 16 * 16];
-    int zs[16];  // surviving bytes per step
+    uint32_t ring[kRing / 4];
 };
-static_assert(sizeof(WaveSlot) % 16 == 0, "slots must keep 16-byte alignment");
 
-// Writes the 4-byte-aligned global words dst[0..nw) from the LDS byte
-// sequence at src + d0 + 4i (any byte offset: funnel-shifted from two
-// aligned LDS words), but only the bytes whose offset from dst lies in
-// [lo, hi): a word shared with a neighbouring chunk is written byte by
-// byte, so the two chunks' waves never overwrite each other's bytes.
-__device__ __forceinline__ void store_funnel(const uint8_t* src, int d0, uint32_t* dst, int nw, int lo, int hi,
-                                             int lane) {
-    const uint32_t* s = reinterpret_cast<const uint32_t*>(src);
-    for (int i = lane; i < nw; i += 64) {
-        const int d = d0 + 4 * i;
-        const uint32_t v = __builtin_amdgcn_alignbyte(s[(d >> 2) + 1], s[d >> 2], d & 3);
-        const int x = 4 * i;
-        if (x >= lo && x + 4 <= hi) {
-            dst[i] = v;
-        } else {
-            uint8_t* a = reinterpret_cast<uint8_t*>(dst + i);
+// The encoded bytes on their way to the stream.  Byte x of the ring's running
+// count is byte x & 15 of 16-byte unit x >> 4 of the stream, counted from the
+// aligned address below the payload's first byte, so whole units leave as one
+// aligned 16-byte store a lane, whatever the payload's alignment, and only the
+// first and last unit, shared with the neighbouring chunks, byte by byte.
+// Bytes join the ring by LDS ORs (units are cleared as they leave): a lane's
+// up to 16 bytes meet its neighbours' inside one word.
+struct ByteRing {
+    uint32_t* ring;
+    uint8_t* dst;  // the aligned address
+    int q;         // payload's first byte
+    int x, done;   // running count; units that have left
+
+    __device__ __forceinline__ ByteRing(uint32_t* ring_, uint8_t* payload, int lane) : ring(ring_) {
+        q = (int)((uintptr_t)payload & 15);
+        dst = payload - q;
+        x = q;
+        done = 0;
 #pragma unroll
-            for (int b = 0; b < 4; ++b)
-                if (x + b >= lo && x + b < hi) a[b] = (uint8_t)(v >> (8 * b));
-        }
+        for (int i = 0; i < kRing / 1024; ++i) unit(64 * i + lane) = make_uint4(0u, 0u, 0u, 0u);
+        wave_sync();
     }
+    __device__ __forceinline__ uint4& unit(int u) { return reinterpret_cast<uint4*>(ring)[u & (kRing / 16 - 1)]; }
+    __device__ __forceinline__ void word(int w, uint32_t v) {
+        __hip_atomic_fetch_or(ring + (w & (kRing / 4 - 1)), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+    }
+    // n <= 16 bytes lo, hi (zero past them) of this lane, at running count at
+    __device__ __forceinline__ void put(int at, int n, uint64_t lo, uint64_t hi) {
+        const int b = 8 * (at & 3), w = at >> 2, span = n > 0 ? (at & 3) + n : 0;
+        const uint64_t u = lo << b, v = (hi << b) | ((lo >> 1) >> (63 - b));
+        if (span > 0) word(w, (uint32_t)u);
+        if (span > 4) word(w + 1, (uint32_t)(u >> 32));
+        if (span > 8) word(w + 2, (uint32_t)v);
+        if (span > 12) word(w + 3, (uint32_t)(v >> 32));
+        if (span > 16) word(w + 4, (uint32_t)((hi >> 1) >> (63 - b)));
+    }
+    // bytes [lo, hi) of unit u, one a lane
+    __device__ __forceinline__ void part(int u, int lo, int hi, int lane) {
+        if (lane >= lo && lane < hi) dst[16 * u + lane] = reinterpret_cast<const uint8_t*>(&unit(u))[lane];
+    }
+    // the whole units
+    __device__ __forceinline__ void flush(int lane) {
+        wave_sync();
+        const int end = x >> 4;
+        if (done == 0 && q != 0 && end > 0) {
+            part(0, q, 16, lane);
+            if (lane == 0) unit(0) = make_uint4(0u, 0u, 0u, 0u);
+            done = 1;
+        }
+        for (int u = done + lane; u < end; u += 64) {
+            reinterpret_cast<uint4*>(dst)[u] = unit(u);
+            unit(u) = make_uint4(0u, 0u, 0u, 0u);
+        }
+        done = end;
+        wave_sync();
+    }
+    __device__ __forceinline__ void finish(int lane) {
+        flush(lane);
+        part(done, done == 0 ? q : 0, x & 15, lane);
+    }
+};
+
+// The bytes of up to four words whose bits in `keep` are set, packed (sel: for
+// each 4-bit mask, the byte selector that packs its bytes).
+__device__ __forceinline__ uint64_t pack8(uint32_t w0, uint32_t w1, uint32_t keep, const uint32_t* sel) {
+    const uint32_t a = __builtin_amdgcn_perm(0u, w0, sel[keep & 15u]), b = __builtin_amdgcn_perm(0u, w1, sel[(keep >> 4) & 15u]);
+    return a | ((uint64_t)b << (8 * __popc(keep & 15u)));
+}
+__device__ __forceinline__ void put16(ByteRing& r, int at, const uint32_t (&w)[4], uint32_t keep, const uint32_t* sel) {
+    const uint64_t a = pack8(w[0], w[1], keep, sel), b = pack8(w[2], w[3], keep >> 8, sel);
+    const int h = 4 * __popc(keep & 255u);  // half the bits of a (shifts by 64 in two halves)
+    r.put(at, __popc(keep & 0xFFFFu), a | ((b << h) << h), (b >> (32 - h)) >> (32 - h));
+}
+__device__ __forceinline__ uint32_t pack_selector(uint32_t keep) {
+    uint32_t s = 0, n = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i)
+        if ((keep >> i) & 1u) s |= i << (8 * n++);
+    for (; n < 4; ++n) s |= 0x0Cu << (8 * n);  // (a zero byte)
+    return s;
 }
 
 // ---- decoupled look-back over the encoder's workgroups in index order ----
@@ -273,6 +330,7 @@ struct EncodeOut {
 struct GroupLds {
     int csize[8];
     int64_t off;
+    uint32_t sel[16];  // pack_selector
 };
 
 // One chunk per wave64, kW chunks per workgroup (chunks id0 .. id0 + kW - 1,
@@ -282,6 +340,17 @@ struct GroupLds {
 // compressed sizes, the workgroup's look-back for its payload offset, then
 // the bytes straight to their place in the stream (zbpc.cu:155-263).  Every
 // wave of the workgroup calls it (a wave past the last chunk has size 0).
+//
+// A chunk's latency bounds it: one wave works on it from its load to its last
+// byte, and the chunks before it hold its offset.  So a step costs few
+// dependent instructions: masks by byte dot products, two steps' counts in one
+// wave scan, kept in registers for the write; bytes packed word by word through
+// byte selectors and ORed into a ring that leaves as aligned 16-byte stores
+// (single byte writes, a carried word and funnel-shifted 4-byte stores a step took
+// 2000 cycles each); a raw chunk goes from its registers to any alignment.
+// Four waves a SIMD (128 registers).  Microseconds before -> after: 64^3
+// float32 25.4 -> 15.6, 2048^2 float64 28 -> 17, 7 M codes 1-D 29 -> 20,
+// 19 M codes 77 -> 63, 512^3 float32 177 -> 152.
 template <int kW>
 __device__ __forceinline__ void encode_chunk(const uint8_t* __restrict__ bp, const ChunkGeom& g, const EncodeOut& o,
                                              int64_t id0, int64_t w, WaveSlot& W, GroupLds& G) {
@@ -290,6 +359,7 @@ __device__ __forceinline__ void encode_chunk(const uint8_t* __restrict__ bp, con
     const bool valid = id < g.nchunks;
     const ChunkPos cp = chunk_pos(g, valid ? id : 0);
     const int osize = valid ? cp.osize : 0;
+    if (threadIdx.x < 16) G.sel[threadIdx.x] = pack_selector(threadIdx.x);
     const uint8_t* src = bp + cp.base;
     // a chunk inside a level's zero planes is not read (nor was it written)
     bool unread = false;
@@ -317,19 +387,24 @@ __device__ __forceinline__ void encode_chunk(const uint8_t* __restrict__ bp, con
     }
     // zero-elimination bitmaps and the surviving-byte count (none of an
     // all-zero chunk, whose bitmap nothing reads)
+    // The mask and the counts of two steps share a register each: 16 steps' masks
+    // and prefix counts (below 2^11) stay in 16 registers until the bytes leave.
     int Z = 0;
-    uint32_t any = 0;
+    uint32_t any = 0, mask[kSteps / 2] = {}, upto[kSteps / 2] = {};
 #pragma unroll
     for (int k = 0; k < kSteps; ++k) any |= (lo8[k].x | lo8[k].y) | (hi8[k].x | hi8[k].y);
     if (__ballot(any != 0)) {
 #pragma unroll
         for (int k = 0; k < kSteps; ++k) {
-            const uint32_t m = nz_bytes(lo8[k].x) | (nz_bytes(lo8[k].y) << 4) | (nz_bytes(hi8[k].x) << 8) |
-                               (nz_bytes(hi8[k].y) << 12);
+            const uint32_t m = nz_bytes2(lo8[k].x, lo8[k].y) | (nz_bytes2(hi8[k].x, hi8[k].y) << 8);
             W.b0[64 * k + lane] = (uint16_t)m;
-            const int c = __builtin_amdgcn_readlane(wave_incl_scan(__popc(m)), 63);  // the wave's total
-            if (lane == 0) W.zs[k] = c;
-            Z += c;
+            mask[k / 2] |= m << (16 * (k & 1));
+        }
+#pragma unroll
+        for (int k = 0; k < kSteps / 2; ++k) {
+            upto[k] = (uint32_t)wave_incl_scan(__popc(mask[k] & 0xFFFFu) | (__popc(mask[k] >> 16) << 16));
+            const uint32_t t = __builtin_amdgcn_readlane(upto[k], 63);  // the wave's totals
+            Z += (t & 0xFFFFu) + (t >> 16);
         }
     }
     bool fail = Z >= kAvail;
@@ -382,103 +457,68 @@ __device__ __forceinline__ void encode_chunk(const uint8_t* __restrict__ bp, con
     }
     uint8_t* P = o.stream + 8 + 2 * g.nchunks + off;  // first byte of the payload
 
-    if (raw) {
-        // step k: the previous step's last word at step[12..16), the step's
-        // 1 KiB from step[16]; global word i of the step starts at chunk
-        // position 1024k + 4i - q (q = misalignment of P), LDS byte
-        // 16 + 4i - q
-        const int q = (int)((uintptr_t)P & 3);
-        uint32_t* dst = reinterpret_cast<uint32_t*>(P - q);
-#pragma unroll
-        for (int k = 0; k < kSteps; ++k) {
-            if (1024 * k >= osize) break;  // wave-uniform
-            const uint32_t prev_last = k > 0 ? __shfl(hi8[k - 1].y, 63, 64) : 0u;
-            reinterpret_cast<uint4*>(W.step + 16)[lane] = make_uint4(lo8[k].x, lo8[k].y, hi8[k].x, hi8[k].y);
-            if (lane == 0) reinterpret_cast<uint32_t*>(W.step)[3] = prev_last;
-            wave_sync();
-            const int rest = osize - 1024 * k;  // chunk bytes from this step on
-            // words whose last byte lies in this step (the final word of the
-            // chunk, when it ends past a word boundary, goes with the last step)
-            const int nw = rest > 1024 ? 256 : (rest + q + 3) >> 2;
-            store_funnel(W.step, 16 - q, dst + 256 * k, nw, q - 1024 * k, q + osize - 1024 * k, lane);
-            wave_sync();  // the next step reuses the buffer
-        }
+    if (Z == 0 && !raw) {  // the footer alone
+        if (lane < 2) P[lane] = (uint8_t)(osize >> (8 * lane));
         return;
     }
-    // zero-eliminated bytes, step by step from the registers the bitmap
-    // pass filled (the loop is unrolled so they stay in registers): a step's
-    // bytes follow the r < 4 bytes carried from the previous step's last
-    // partial word (r = alignment of the step's first byte in the stream),
-    // whole words go out, the last partial word is carried on
-    int zpos = 0;
-    if (Z != 0) {
+    if (raw) {  // straight from the registers, 16 bytes a lane at any alignment
 #pragma unroll
         for (int k = 0; k < kSteps; ++k) {
+            const int b = 16 * (64 * k + lane);
+            if (1024 * k >= osize) break;  // wave-uniform
             const uint32_t w[4] = {lo8[k].x, lo8[k].y, hi8[k].x, hi8[k].y};
-            const int zs = W.zs[k];
-            if (zs == 0) continue;  // wave-uniform
-            const int r = (int)((uintptr_t)(P + zpos) & 3);
-            const uint32_t m = W.b0[64 * k + lane];
-            const int cnt = __popc(m);
-            int pos = r + wave_incl_scan(cnt) - cnt;
-#pragma unroll
-            for (int i = 0; i < 16; ++i)
-                if ((m >> i) & 1u) W.step[pos++] = (uint8_t)(w[i >> 2] >> (8 * (i & 3)));
-            wave_sync();
-            const int nfull = (r + zs) >> 2;
-            store_funnel(W.step, 0, reinterpret_cast<uint32_t*>(P + zpos - r), nfull, r - zpos, r + csize - zpos, lane);
-            wave_sync();  // the stores have read the buffer
-            if (lane == 0) reinterpret_cast<uint32_t*>(W.step)[0] = reinterpret_cast<const uint32_t*>(W.step)[nfull];
-            wave_sync();  // the next step reuses the buffer
-            zpos += zs;
+            if (b + 16 <= osize) __builtin_memcpy(P + b, w, 16);
+            else if (b < osize) reinterpret_cast<uint4*>(W.ring)[0] = make_uint4(w[0], w[1], w[2], w[3]);
         }
+        wave_sync();
+        const int rest = osize & 15;  // the chunk's last bytes, one a lane
+        if (lane < rest) P[osize - rest + lane] = reinterpret_cast<const uint8_t*>(W.ring)[lane];
+        return;
     }
-    // the RE bytes at tail[4 + (chunk position - Z)], B3 and the footer,
-    // after the carried bytes (stream positions Z - rt .. Z - 1); then every
-    // word from the aligned P + Z - rt to the end
-    const int rt = (int)((uintptr_t)(P + Z) & 3);
-    if (lane < rt) W.tail[4 - rt + lane] = W.step[lane];
-    int pos = 4;
-    if (Z != 0) {
-        {  // round 1: B0 byte 32 lane + i is kept where bit i of f1 is set
-            const int cnt = __popc(f1);
-            int p = pos + wave_incl_scan(cnt) - cnt;
-            const uint4* b0v = reinterpret_cast<const uint4*>(W.b0) + 2 * lane;
-            const uint4 q0 = b0v[0], q1 = b0v[1];
-            const uint32_t v[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
+    // zero-eliminated bytes, step by step from the registers the bitmap pass
+    // filled (the loop is unrolled so they stay in registers)
+    ByteRing r(W.ring, P, lane);
 #pragma unroll
-            for (int i = 0; i < 32; ++i)
-                if ((f1 >> i) & 1u) W.tail[p++] = (uint8_t)(v[i >> 2] >> (8 * (i & 3)));
-            pos += __builtin_amdgcn_readlane(wave_incl_scan(cnt), 63);
-        }
-        {  // round 2: B1 byte 4 lane + i (byte i of f1) where bit i of f2 is set
-            const int cnt = __popc(f2);
-            int p = pos + wave_incl_scan(cnt) - cnt;
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                if ((f2 >> i) & 1u) W.tail[p++] = (uint8_t)(f1 >> (8 * i));
-            pos += __builtin_amdgcn_readlane(wave_incl_scan(cnt), 63);
-        }
-        {  // round 3: the B2 bytes where B3 is set
-            const uint32_t b2 = re2_byte(f2, lane);
-            if (lane < 32 && ((b3 >> lane) & 1u)) W.tail[pos + __popc(b3 & ((1u << lane) - 1u))] = (uint8_t)b2;
-            pos += __popc(b3);
-        }
-        if (lane < 4) W.tail[pos + lane] = (uint8_t)(b3 >> (8 * lane));
-        pos += 4;
+    for (int k = 0; k < kSteps; ++k) {
+        const int sh = 16 * (k & 1);
+        const int zs = (__builtin_amdgcn_readlane(upto[k / 2], 63) >> sh) & 0xFFFF;
+        if (zs == 0) continue;  // wave-uniform
+        const uint32_t w[4] = {lo8[k].x, lo8[k].y, hi8[k].x, hi8[k].y};
+        const uint32_t m = (mask[k / 2] >> sh) & 0xFFFFu;
+        put16(r, r.x + (int)((upto[k / 2] >> sh) & 0xFFFFu) - __popc(m), w, m, G.sel);
+        r.x += zs;
+        if (r.x - 16 * r.done >= kFlush) r.flush(lane);
     }
-    if (lane == 0) {
-        W.tail[pos] = (uint8_t)(osize & 0xFF);
-        W.tail[pos + 1] = (uint8_t)((osize >> 8) & 0xFF);
+    // the kept bytes of the three repetition-elimination rounds, B3, the footer
+    {  // round 1: B0 byte 32 lane + i is kept where bit i of f1 is set
+        const int cnt = __popc(f1), upto1 = wave_incl_scan(cnt), lower = __popc(f1 & 0xFFFFu);
+        const uint4* b0v = reinterpret_cast<const uint4*>(W.b0) + 2 * lane;
+        const uint4 q0 = b0v[0], q1 = b0v[1];
+        const uint32_t v0[4] = {q0.x, q0.y, q0.z, q0.w}, v1[4] = {q1.x, q1.y, q1.z, q1.w};
+        const int at = r.x + upto1 - cnt;
+        put16(r, at, v0, f1 & 0xFFFFu, G.sel);
+        put16(r, at + lower, v1, f1 >> 16, G.sel);
+        r.x += __builtin_amdgcn_readlane(upto1, 63);
     }
-    wave_sync();
-    store_funnel(W.tail, 4 - rt, reinterpret_cast<uint32_t*>(P + Z - rt), (rt + csize - Z + 3) >> 2, rt - Z,
-                 rt + csize - Z, lane);
+    {  // round 2: B1 byte 4 lane + i (byte i of f1) where bit i of f2 is set
+        const int cnt = __popc(f2), upto2 = wave_incl_scan(cnt);
+        r.put(r.x + upto2 - cnt, cnt, __builtin_amdgcn_perm(0u, f1, G.sel[f2 & 15u]), 0ull);
+        r.x += __builtin_amdgcn_readlane(upto2, 63);
+    }
+    {  // round 3: the B2 bytes where B3 is set
+        const uint32_t b2 = re2_byte(f2, lane);
+        const bool keep = lane < 32 && ((b3 >> lane) & 1u);
+        r.put(r.x + __popc(b3 & ((1u << (lane & 31)) - 1u)), keep ? 1 : 0, b2, 0ull);
+        r.x += __popc(b3);
+    }
+    r.put(r.x, lane == 0 ? 6 : 0, b3 | ((uint64_t)(osize & 0xFFFF) << 32), 0ull);
+    r.x += 6;
+    r.finish(lane);
 }
 
 // one chunk per wave, kW chunks per workgroup
 template <int kW>
-__global__ __launch_bounds__(64 * kW) void encode_kernel(const uint8_t* __restrict__ bp, ChunkGeom g, EncodeOut o) {
+__global__ __launch_bounds__(64 * kW) __attribute__((amdgpu_waves_per_eu(4))) void encode_kernel(const uint8_t* __restrict__ bp, ChunkGeom g, EncodeOut o) {
     __shared__ WaveSlot slots[kW];
     __shared__ GroupLds G;
     encode_chunk<kW>(bp, g, o, (int64_t)blockIdx.x * kW, blockIdx.x, slots[threadIdx.x >> 6], G);
@@ -489,7 +529,7 @@ __global__ __launch_bounds__(64 * kW) void encode_kernel(const uint8_t* __restri
 // prefix entry), so a workgroup never spans two fields, and they are
 // dispatched in id order
 template <int kW>
-__global__ __launch_bounds__(64 * kW) void batch_encode_kernel(const BatchField* __restrict__ fields,
+__global__ __launch_bounds__(64 * kW) __attribute__((amdgpu_waves_per_eu(4))) void batch_encode_kernel(const BatchField* __restrict__ fields,
                                                                const int64_t* __restrict__ prefix, int nf) {
     __shared__ WaveSlot slots[kW];
     __shared__ GroupLds G;
