@@ -1,8 +1,9 @@
 // predictor.hip -- multi-level cubic-spline prediction on gfx950.
 //
-// One workgroup (256 lanes = 4 wave64) per 16^3 tile.  The tile and its
-// +1 halo (17^3 values of T) live in LDS; each of the 4 levels (unit 8,4,2,1)
-// runs three stages, and every stage is a compile-time shape so the
+// 3-D fields: one workgroup (256 lanes = 4 wave64) per 16^3 tile, or per pair
+// of tiles, with the +1 halo in LDS (tile3.hpp).  2-D fields: one wave per
+// 16^2 tile; 1-D fields: one lane per 16 points.  Each of the 4 levels (unit
+// 8,4,2,1) runs three stages, and every stage is a compile-time shape so the
 // point <-> lane mapping uses constant divisors only.  Points of one stage
 // read only points of earlier stages, so a stage is one parallel sweep
 // followed by one barrier.  Arithmetic is in T (FP64 for double fields),
@@ -470,7 +471,7 @@ __device__ __forceinline__ void clear_gaps(const SplineArgs<T>& a) {
 // the decoded bit-planes instead of a code hand-off: the inverse shuffle
 // (bitplane.cu:645-667) folded into the reconstruction's code load
 // (InterpolationPredictor.cu:2209-2239).  Lane l takes rows l and 256 + l of
-// the tile's 404 code rows, in the row table's order.  A row's codes are
+// the tile's 404 code rows, level 0's first.  A row's codes are
 // adjacent in its level's segment, so on each plane of the window they lie
 // in at most 3 adjacent bytes (17 codes from any bit offset): one 8-byte
 // load from the 4-byte aligned address below them, a funnel shift, and the
@@ -526,8 +527,7 @@ __device__ __forceinline__ void plane_row_load(const Tile<T, IN>& t, const Plane
     for (int q = 0; q < kPlaneWindow; ++q) r.w[q] = 0u;
     if (r.np == 0) return;
     // the run's first code, relative to the level's segment (32-bit: the
-    // code array is shorter than 2^31); the row base computed here, so the
-    // loads need no row table
+    // code array is shorter than 2^31)
     const uint32_t start = (uint32_t)row_base<L>(t.g, t.oy + U * j, t.oz + U * k) +
                            (uint32_t)(r.full ? t.ox >> L : t.ox >> (L + 1));
     const uint32_t rel = start - (uint32_t)t.g.prefix[L];
