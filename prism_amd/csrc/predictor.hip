@@ -662,14 +662,28 @@ __device__ __forceinline__ void tile_out(const Tile<T, IN>& m, bool delta, bool 
     const uint32_t nx = (uint32_t)m.g.nx, nxy = nx * (uint32_t)m.g.ny;
     const T* src = m.s + r.slot(r.y, 0);
     Column<T, IN> dst(out + ((uint64_t)m.oz * nxy + (uint64_t)m.oy * nx + m.ox), nx, nxy, r.X, r.y);
+    // the compiler would join the two forms' stores and drop the hint: the
+    // empty statements keep them apart
+    if (lines) {
+        asm volatile("");
 #pragma unroll
-    for (int z = 0; z < kOutIters; ++z) {
-        if (m.template in<2>(z)) {
-            const T s = src[z * kZP], v = delta ? s + prev[z] : s;
-            if (lines) __builtin_nontemporal_store(v, &dst.at());
-            else dst.at() = v;
+        for (int z = 0; z < kOutIters; ++z) {
+            if (m.template in<2>(z)) {
+                const T s = src[z * kZP];
+                __builtin_nontemporal_store(delta ? s + prev[z] : s, &dst.at());
+            }
+            dst.next();
         }
-        dst.next();
+        asm volatile("");
+    } else {
+#pragma unroll
+        for (int z = 0; z < kOutIters; ++z) {
+            if (m.template in<2>(z)) {
+                const T s = src[z * kZP];
+                dst.at() = delta ? s + prev[z] : s;
+            }
+            dst.next();
+        }
     }
 }
 
