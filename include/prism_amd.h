@@ -68,7 +68,9 @@ int pa_extrema(const void* d_data, int dtype, int64_t n, double* d_minmax, void*
 /* Auto-tuning part of spline_construct (InterpolationPredictor.cu:2273-2355,
  * kernel auto_tuning_interpolation 880-967).  Scores the 15 candidates with a
  * fixed-order sum and picks flags on the device.  d_scores15 (double[15]) may
- * be NULL. */
+ * be NULL.  The workspace (8-byte aligned) holds 15 doubles for each 16^3
+ * sample block, which both tuning calls accept, and room for the extrema
+ * results of pa_extrema_autotune (two doubles each for 2048 workgroups). */
 size_t pa_autotune_workspace(const pa_layout* L);
 int pa_autotune(const void* d_data, int dtype, const pa_layout* L, double* d_scores15,
                 uint8_t* d_flags8, void* d_ws, size_t ws_bytes, void* stream);
@@ -79,7 +81,9 @@ int pa_autotune(const void* d_data, int dtype, const pa_layout* L, double* d_sco
  * prediction), run side by side in one launch, and with d_bounds non-NULL
  * pa_level_bounds(d_minmax, rel_eb, dtype, d_bounds) after them: the same
  * d_minmax, scores, flags and bounds as the separate calls.  d_data must be
- * 16-byte aligned; the workspace is pa_autotune's. */
+ * 16-byte aligned; the workspace is pa_autotune's (with the tuner's sums
+ * alone the extrema meet at two words in d_minmax[2..3]: the same results,
+ * in more time). */
 int pa_extrema_autotune(const void* d_data, int dtype, const pa_layout* L, double* d_minmax, double rel_eb,
                         double* d_bounds, double* d_scores15, uint8_t* d_flags8, void* d_ws, size_t ws_bytes,
                         void* stream);

@@ -1349,7 +1349,8 @@ __global__ void tune_pick_kernel(const double* __restrict__ part, int nblocks, d
 // 384 x 384 x 256), too few to fill the GPU on their own.
 template <typename T>
 __global__ __launch_bounds__(kThreads) void extrema_tune_kernel(const T* __restrict__ data, int64_t n,
-                                                                double* __restrict__ ext_part, int64_t span,
+                                                                double* __restrict__ ext_part,
+                                                                unsigned long long* __restrict__ keys, int64_t span,
                                                                 Geom g, int sx0, int sy0, int sz0, int nsx, int nsy,
                                                                 int nblocks, double* __restrict__ part) {
     __shared__ T tile[kTileVals];
@@ -1361,7 +1362,10 @@ __global__ __launch_bounds__(kThreads) void extrema_tune_kernel(const T* __restr
     else {
         double mn, mx;
         extrema_span<T>(data, n, (int64_t)blockIdx.x - ntune, span, mn, mx);
-        if (threadIdx.x == 0) {
+        if (threadIdx.x != 0) return;
+        if (keys) {
+            join_keys(mn, mx, keys);
+        } else {
             double* p = ext_part + 2 * ((int)blockIdx.x - ntune);
             p[0] = mn;
             p[1] = mx;
@@ -1369,15 +1373,20 @@ __global__ __launch_bounds__(kThreads) void extrema_tune_kernel(const T* __restr
     }
 }
 
+__global__ void extrema_keys_init_kernel(unsigned long long* keys) {
+    keys[0] = ~0ull;  // running min
+    keys[1] = 0ull;   // running max
+}
+
 __device__ int64_t fill_bounds(const double* minmax, double eb_in, int rel, int dtype, double alpha, double* e);
 
-// min / max from the extrema workgroups' results, the tuner's pick (as
-// tune_pick_kernel) and, with `bounds`, the level bounds of a relative eb (as
+// min / max from the extrema workgroups' results (or the keys that they met
+// at), the tuner's pick (as tune_pick_kernel) and, with `bounds`, the level bounds of a relative eb (as
 // level_bounds_kernel)
 constexpr int kFinishThreads = 256;
 __global__ __launch_bounds__(kFinishThreads) void extrema_tune_finish_kernel(
-    const double* __restrict__ ext_part, int next, double* __restrict__ minmax, const double* __restrict__ part,
-    int nblocks, double* __restrict__ scores, uint8_t* __restrict__ flags, double eb, int dtype, double alpha,
+    const double* __restrict__ ext_part, int next, const unsigned long long* __restrict__ keys,
+    double* __restrict__ minmax, const double* __restrict__ part, int nblocks, double* __restrict__ scores, uint8_t* __restrict__ flags, double eb, int dtype, double alpha,
     double* __restrict__ bounds) {
     __shared__ double s[kPickLds];
     __shared__ double e[15];
@@ -1389,8 +1398,8 @@ __global__ __launch_bounds__(kFinishThreads) void extrema_tune_finish_kernel(
     group_minmax<kFinishThreads / 64>(mn, mx);
     pick_parallel(part, nblocks, scores, flags, s, e);
     if (threadIdx.x != 0) return;
-    minmax[0] = mn;
-    minmax[1] = mx;
+    minmax[0] = keys ? key_value(keys[0]) : mn;
+    minmax[1] = keys ? key_value(keys[1]) : mx;
     if (bounds) {
         bounds[14] = (double)fill_bounds(minmax, eb, true, dtype, alpha, bounds);
         bounds[15] = 0.0;
@@ -1760,13 +1769,14 @@ using namespace pa;
 // extrema workgroups of pa_extrema_autotune at most, each with its result in
 // the workspace after the tuner's partial sums
 constexpr int kExtParts = 2048;
+static size_t tune_part_bytes(int nblocks) { return sizeof(double) * 15 * (size_t)nblocks; }
 
 extern "C" size_t pa_autotune_workspace(const pa_layout* L) {
     int s[3], n[3];
     if (!L || !tune_axis(L->nx, &s[0], &n[0]) || !tune_axis(L->ny, &s[1], &n[1]) ||
         !tune_axis(L->nz, &s[2], &n[2]))
         return 0;
-    return sizeof(double) * (15 * (size_t)n[0] * n[1] * n[2] + 2 * kExtParts);
+    return tune_part_bytes(n[0] * n[1] * n[2]) + sizeof(double) * 2 * kExtParts;
 }
 
 extern "C" int pa_autotune(const void* d_data, int dtype, const pa_layout* L, double* d_scores15,
@@ -1780,7 +1790,7 @@ extern "C" int pa_autotune(const void* d_data, int dtype, const pa_layout* L, do
         return PA_OK;
     }
     const int nblocks = n[0] * n[1] * n[2];
-    if (ws_bytes < sizeof(double) * 15 * (size_t)nblocks || !d_ws) return PA_ERR_WORKSPACE;
+    if (ws_bytes < tune_part_bytes(nblocks) || !d_ws) return PA_ERR_WORKSPACE;
     double* part = static_cast<double*>(d_ws);
     Geom g = make_geom(L);
     dim3 grid(nblocks, 15);
@@ -1810,10 +1820,18 @@ extern "C" int pa_extrema_autotune(const void* d_data, int dtype, const pa_layou
         return e;
     }
     const int nblocks = n[0] * n[1] * n[2];
-    if (ws_bytes < pa_autotune_workspace(L) || !d_ws) return PA_ERR_WORKSPACE;
+    if (ws_bytes < tune_part_bytes(nblocks) || !d_ws) return PA_ERR_WORKSPACE;
     hipStream_t st = as_stream(stream);
     double* part = static_cast<double*>(d_ws);
     double* ext_part = part + 15 * (size_t)nblocks;
+    // a workspace that holds the tuner's sums alone is enough as well: the
+    // extrema workgroups then meet at the two keys behind the result
+    unsigned long long* keys = nullptr;
+    if (ws_bytes < pa_autotune_workspace(L)) {
+        keys = reinterpret_cast<unsigned long long*>(d_minmax + 2);
+        hipLaunchKernelGGL(extrema_keys_init_kernel, dim3(1), dim3(1), 0, st, keys);
+        PA_LAUNCH_CHECK();
+    }
     // the tuner's LDS tile leaves three workgroups per CU; the extrema are cut
     // into up to 8 workgroups per CU, queued behind the tuner blocks (measured
     // against 4 per CU and against exactly the slots the tuner leaves: the
@@ -1832,13 +1850,13 @@ extern "C" int pa_extrema_autotune(const void* d_data, int dtype, const pa_layou
     Geom g = make_geom(L);
     if (dtype == PA_F32)
         hipLaunchKernelGGL(extrema_tune_kernel<float>, dim3(grid), dim3(kThreads), 0, st, (const float*)d_data, L->n,
-                           ext_part, span, g, s[0], s[1], s[2], n[0], n[1], nblocks, part);
+                           ext_part, keys, span, g, s[0], s[1], s[2], n[0], n[1], nblocks, part);
     else
         hipLaunchKernelGGL(extrema_tune_kernel<double>, dim3(grid), dim3(kThreads), 0, st, (const double*)d_data,
-                           L->n, ext_part, span, g, s[0], s[1], s[2], n[0], n[1], nblocks, part);
+                           L->n, ext_part, keys, span, g, s[0], s[1], s[2], n[0], n[1], nblocks, part);
     PA_LAUNCH_CHECK();
-    hipLaunchKernelGGL(extrema_tune_finish_kernel, dim3(1), dim3(kFinishThreads), 0, st, ext_part, (int)ext, d_minmax,
-                       part, nblocks, d_scores15, d_flags8, rel_eb, dtype, alpha_of(rel_eb), d_bounds);
+    hipLaunchKernelGGL(extrema_tune_finish_kernel, dim3(1), dim3(kFinishThreads), 0, st, ext_part, (int)ext, keys,
+                       d_minmax, part, nblocks, d_scores15, d_flags8, rel_eb, dtype, alpha_of(rel_eb), d_bounds);
     PA_LAUNCH_CHECK();
     return PA_OK;
 }
