@@ -183,8 +183,8 @@ int pa_lossless_encode(const uint8_t* d_bp, const pa_layout* L, uint8_t* d_out, 
 
 /* The same compression without moving planes that hold no bit (no reference
  * counterpart): most leading bit-planes of a field are zero.  In this order on
- * one stream, with one encoder workspace throughout: pa_encode_prepare clears
- * it; pa_spline_construct_live is pa_spline_construct_dev and leaves the
+ * one stream, with one encoder workspace (pa_encode_workspace bytes, checked
+ * by every call) throughout: pa_encode_prepare clears it; pa_spline_construct_live is pa_spline_construct_dev and leaves the
  * codes' magnitudes in it; pa_bitshuffle_live is pa_bitshuffle but may leave
  * bytes of planes that these magnitudes show to be zero unwritten;
  * pa_lossless_encode_live is pa_lossless_encode on such planes and does not read
@@ -193,9 +193,10 @@ int pa_lossless_encode(const uint8_t* d_bp, const pa_layout* L, uint8_t* d_out, 
 int pa_live_planes(const pa_layout* L);
 int pa_encode_prepare(const pa_layout* L, void* d_ws, size_t ws_bytes, void* stream);
 int pa_spline_construct_live(const void* d_data, int dtype, const pa_layout* L, const double* d_bounds,
-                             const uint8_t* d_flags8, int32_t* d_qc, void* d_anchors, void* d_ews, void* stream);
+                             const uint8_t* d_flags8, int32_t* d_qc, void* d_anchors, void* d_ews,
+                             size_t ews_bytes, void* stream);
 int pa_bitshuffle_live(const int32_t* d_qc, const pa_layout* L, int mode, uint8_t* d_bp, const void* d_ews,
-                       void* stream);
+                       size_t ews_bytes, void* stream);
 int pa_lossless_encode_live(const uint8_t* d_bp, const pa_layout* L, uint8_t* d_out, uint64_t* d_cum,
                             uint64_t* d_outsize, void* d_ws, size_t ws_bytes, void* stream);
 

@@ -105,8 +105,8 @@ SIGNATURES = {
     "pa_lossless_encode": (I32, [P, LP, P, P, P, P, SZ, P]),
     "pa_live_planes": (I32, [LP]),
     "pa_encode_prepare": (I32, [LP, P, SZ, P]),
-    "pa_spline_construct_live": (I32, [P, I32, LP, P, P, P, P, P, P]),
-    "pa_bitshuffle_live": (I32, [P, LP, I32, P, P, P]),
+    "pa_spline_construct_live": (I32, [P, I32, LP, P, P, P, P, P, SZ, P]),
+    "pa_bitshuffle_live": (I32, [P, LP, I32, P, P, SZ, P]),
     "pa_lossless_encode_live": (I32, [P, LP, P, P, P, P, SZ, P]),
     "pa_compress_merge": (I32, [P, LP, I32, P, P, P, P, P, P, P]),
     "pa_decode_workspace": (SZ, [LP]),

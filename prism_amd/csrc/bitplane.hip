@@ -315,10 +315,10 @@ extern "C" int pa_bitshuffle(const int32_t* d_qc, const pa_layout* L, int mode, 
 }
 
 extern "C" int pa_bitshuffle_live(const int32_t* d_qc, const pa_layout* L, int mode, uint8_t* d_bp, const void* d_ews,
-                                  void* stream) {
-    if (!L || !d_ews || ((uintptr_t)d_ews & 7) != 0) return PA_ERR_ARG;
-    const uint64_t* live =
-        live_dims(L) ? live_words(static_cast<uint64_t*>(const_cast<void*>(d_ews)), L->nchunks) : nullptr;
+                                  size_t ews_bytes, void* stream) {
+    if (!L) return PA_ERR_ARG;
+    if (!encws_holds(L, d_ews, ews_bytes)) return PA_ERR_WORKSPACE;
+    const uint64_t* live = live_dims(L) ? live_words(static_cast<const uint64_t*>(d_ews), L->nchunks) : nullptr;
     return launch_shuffle(d_qc, L, mode, d_bp, live, stream);
 }
 

@@ -1118,7 +1118,7 @@ extern "C" int pa_live_planes(const pa_layout* L) { return L && live_dims(L) && 
 
 extern "C" int pa_encode_prepare(const pa_layout* L, void* d_ws, size_t ws_bytes, void* stream) {
     if (!L) return PA_ERR_ARG;
-    if (!d_ws || ws_bytes < pa_encode_workspace(L) || ((uintptr_t)d_ws & 7) != 0) return PA_ERR_WORKSPACE;
+    if (!encws_holds(L, d_ws, ws_bytes)) return PA_ERR_WORKSPACE;
     return encode_clear(L, static_cast<uint64_t*>(d_ws), 1, as_stream(stream));
 }
 

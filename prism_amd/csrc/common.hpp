@@ -138,9 +138,15 @@ __host__ __device__ inline Levels make_levels(const pa_layout* L) {
 // write them and the encoder does not read them, but for the chunks that
 // reach past them.
 constexpr int kLiveLines = 8, kLiveStep = 16;  // 64-bit words
-__host__ __device__ inline uint64_t* live_words(uint64_t* encws, int64_t nchunks) { return encws + 1 + nchunks; }
+template <typename W>  // uint64_t, const or not
+__host__ __device__ inline W* live_words(W* encws, int64_t nchunks) {
+    return encws + 1 + nchunks;
+}
 __host__ __device__ inline size_t encws_words(int64_t nchunks) {
     return 1 + (size_t)nchunks + (size_t)(kLiveLines - 1) * kLiveStep + 1;
+}
+inline bool encws_holds(const pa_layout* L, const void* ws, size_t bytes) {
+    return ws && bytes >= encws_words(L->nchunks) * 8 && ((uintptr_t)ws & 7) == 0;
 }
 
 // Only the 3-D predictor leaves magnitudes, and they are worth its time (4 % of

@@ -1907,8 +1907,9 @@ extern "C" int pa_spline_construct_dev(const void* d_data, int dtype, const pa_l
 
 extern "C" int pa_spline_construct_live(const void* d_data, int dtype, const pa_layout* L, const double* d_bounds,
                                         const uint8_t* d_flags8, int32_t* d_qc, void* d_anchors, void* d_ews,
-                                        void* stream) {
-    if (!L || !d_ews || ((uintptr_t)d_ews & 7) != 0) return PA_ERR_ARG;
+                                        size_t ews_bytes, void* stream) {
+    if (!L) return PA_ERR_ARG;
+    if (!encws_holds(L, d_ews, ews_bytes)) return PA_ERR_WORKSPACE;
     return construct_dev(d_data, dtype, L, d_bounds, d_flags8, d_qc, d_anchors,
                          live_words(static_cast<uint64_t*>(d_ews), L->nchunks), stream);
 }

@@ -232,7 +232,7 @@ def compress(data: torch.Tensor, eb: float, rel: bool = True, progressive: bool 
     with tm("predict"):
         if live:
             check(lib().pa_spline_construct_live(_p(data), dt, C.byref(L), p_bounds, p_flags, _p(qc), _p(anchors), p_ews,
-                                                 st), "pa_spline_construct_live")
+                                                 ews_bytes, st), "pa_spline_construct_live")
         else:
             check(lib().pa_spline_construct_dev(_p(data), dt, C.byref(L), p_bounds, p_flags, _p(qc), _p(anchors), st),
                   "pa_spline_construct_dev")
@@ -240,7 +240,7 @@ def compress(data: torch.Tensor, eb: float, rel: bool = True, progressive: bool 
     mode = PA_MODE_NB if progressive else PA_MODE_SM
     with tm("shuffle"):
         if live:
-            check(lib().pa_bitshuffle_live(_p(qc), C.byref(L), mode, _p(bp), p_ews, st), "pa_bitshuffle_live")
+            check(lib().pa_bitshuffle_live(_p(qc), C.byref(L), mode, _p(bp), p_ews, ews_bytes, st), "pa_bitshuffle_live")
         else:
             check(lib().pa_bitshuffle(_p(qc), C.byref(L), mode, _p(bp), st), "pa_bitshuffle")
     bound = lib().pa_compress_bound(C.byref(L), dt)

@@ -69,3 +69,22 @@ def test_short_tuner_workspaces_are_refused():
     for ws, nbytes in ((p, need - 1), (p, 0), (None, need)):
         assert _lib.lib().pa_extrema_autotune(p, 8, C.byref(L), p, 1e-3, p, p, p, ws, nbytes, None) == _lib.PA_ERR_WORKSPACE
         assert _lib.lib().pa_autotune(p, 8, C.byref(L), p, p, ws, nbytes, None) == _lib.PA_ERR_WORKSPACE
+
+
+def test_short_encoder_workspaces_are_refused():
+    """By every call of the compression that leaves zero planes out; the plain
+    encoder needs the words before the code magnitudes alone."""
+    from prism_amd import _lib, pipeline as pl
+    lb = _lib.lib()
+    for L in (pl.layout(130, 97, 141), pl.layout(300, 400, 1)):
+        host = (C.c_double * 64)()  # never reached
+        p = C.c_void_p((C.addressof(host) + 15) // 16 * 16)
+        need, plain = lb.pa_encode_workspace(C.byref(L)), 8 * (1 + L.nchunks)
+        assert need > plain
+        for ws, nbytes in ((p, need - 1), (p, plain), (p, 0), (None, need), (C.c_void_p(p.value + 4), need)):
+            calls = (lb.pa_encode_prepare(C.byref(L), ws, nbytes, None),
+                     lb.pa_spline_construct_live(p, 8, C.byref(L), p, p, p, p, ws, nbytes, None),
+                     lb.pa_bitshuffle_live(p, C.byref(L), 0, p, ws, nbytes, None),
+                     lb.pa_lossless_encode_live(p, C.byref(L), p, p, p, ws, nbytes, None))
+            assert calls == (_lib.PA_ERR_WORKSPACE,) * 4, (nbytes, calls)
+        assert lb.pa_lossless_encode(p, C.byref(L), p, p, p, p, plain - 1, None) == _lib.PA_ERR_WORKSPACE
