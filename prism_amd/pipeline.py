@@ -436,25 +436,33 @@ def decompress(c: Compressed, check_stream: bool = True) -> torch.Tensor:
     (compressor.cu:153-164).  With `check_stream` (default) the call waits
     for the device and raises PrismError when the decoder found the stream
     malformed (a size-table entry pointing outside the stream: the chunks it
-    names decode to zeros); without it nothing is synchronised."""
+    names decode to zeros).  Without it a call under an absolute bound waits
+    for nothing, and one under a relative bound for the work that is on the
+    stream before it, with which the stream's value range arrives."""
     nx, ny, nz = c.shape
     L = layout(nx, ny, nz)
     dt = DTYPES[c.dtype]
     st = _stream()
     t0, flags, cum, anchors = _trailer(c, L)
-    # the range is copied ahead of the decoder and waited for behind its
-    # launches, which do not need it
-    rng = _host_copy(c.stream[t0 + 8:t0 + 16].view(torch.float64))
-    copied = torch.cuda.Event()
-    copied.record()
-    bp = _empty(L.host_size)
-    ws = _empty(lib().pa_decode_workspace(C.byref(L)))
-    check(lib().pa_lossless_decode(_p(c.stream), c.nbytes, C.byref(L), _p(bp), _p(ws), ws.numel(), st), "pa_lossless_decode")
-    qc = torch.empty(L.code_len, dtype=torch.int32, device=c.stream.device)
-    mode = PA_MODE_NB if c.progressive else PA_MODE_SM
-    check(lib().pa_inverse_bitshuffle(_p(bp), C.byref(L), mode, _p(qc), st), "pa_inverse_bitshuffle")
-    out = torch.empty((nz, ny, nx), dtype=c.dtype, device=c.stream.device)
-    copied.synchronize()
+    # a relative bound's range is copied ahead of the decoder and waited for
+    # behind its launches, which do not need it; also where one of them raises:
+    # no copy to the thread's buffer is left on its way
+    copied = torch.cuda.Event() if c.rel else None
+    if c.rel:
+        rng = _host_copy(c.stream[t0 + 8:t0 + 16].view(torch.float64))
+        copied.record()
+    try:
+        bp = _empty(L.host_size)
+        ws = _empty(lib().pa_decode_workspace(C.byref(L)))
+        check(lib().pa_lossless_decode(_p(c.stream), c.nbytes, C.byref(L), _p(bp), _p(ws), ws.numel(), st),
+              "pa_lossless_decode")
+        qc = torch.empty(L.code_len, dtype=torch.int32, device=c.stream.device)
+        mode = PA_MODE_NB if c.progressive else PA_MODE_SM
+        check(lib().pa_inverse_bitshuffle(_p(bp), C.byref(L), mode, _p(qc), st), "pa_inverse_bitshuffle")
+        out = torch.empty((nz, ny, nx), dtype=c.dtype, device=c.stream.device)
+    finally:
+        if c.rel:
+            copied.synchronize()
     eb_abs = c.eb_input * float(rng[0]) if c.rel else c.eb_input
     rel_eb = c.eb_input if c.rel else 0.0
     check(lib().pa_spline_reconstruct(_p(qc), _p(anchors), dt, C.byref(L), eb_abs, rel_eb, _p(flags), None,
