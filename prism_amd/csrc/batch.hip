@@ -480,13 +480,14 @@ extern "C" int pa_retrieve_batch(const pa_retrieve_job* jobs, int nj, void* h_ta
     int64_t* p_unit = p_unshuf + (nj + 1);
     unsigned long long* keys = reinterpret_cast<unsigned long long*>(ws + tb.total);
     int64_t* p_chunk = reinterpret_cast<int64_t*>(ws + tb.total + retr_keys_bytes(nj));
-    // float32 jobs first
-    int k = 0, nj32 = 0;
+    // float32 jobs first: those whose tiles are paired, then the others
+    int k = 0, nj32 = 0, njpair = 0;
     int64_t max_chunks = 0;
     p_unshuf[0] = p_unit[0] = 0;
-    for (int pass = 0; pass < 2; ++pass)
+    for (int pass = 0; pass < 3; ++pass)
         for (int i = 0; i < nj; ++i) {
-            if ((jobs[i].dtype == PA_F32) != (pass == 0)) continue;
+            const bool f32 = jobs[i].dtype == PA_F32;
+            if (pass != (f32 ? pa::retr_lone_tiles(PA_F32, jobs[i].nx, jobs[i].nz) : 2)) continue;
             RetrJob& j = hj[k];
             const int st = retr_describe(jobs[i], j);
             if (st != PA_OK) return st;
@@ -494,19 +495,22 @@ extern "C" int pa_retrieve_batch(const pa_retrieve_job* jobs, int nj, void* h_ta
             p_unshuf[k + 1] = p_unshuf[k] + pa::retr_unshuf_blocks(&j.L);
             p_unit[k + 1] = p_unit[k] + pa::retr_tile_units(&j.L, j.dtype);
             max_chunks += j.L.nchunks;
-            nj32 += pass == 0;
+            nj32 += pass < 2;
+            njpair += pass == 0;
             ++k;
         }
     pa::RetrDev r;
     r.jobs = reinterpret_cast<const RetrJob*>(ws);
     r.nj = nj;
     r.nj32 = nj32;
+    r.njpair = njpair;
     r.p_unshuf = reinterpret_cast<const int64_t*>(ws + tb.jobs);
     r.p_unit = r.p_unshuf + (nj + 1);
     r.p_chunk = p_chunk;
     r.n_unshuf = p_unshuf[nj];
     r.n_unit = p_unit[nj];
     r.n_unit32 = p_unit[nj32];
+    r.n_unitpair = p_unit[njpair];
     r.max_chunks = max_chunks;
     if (r.n_unshuf > 0x7fffffff || r.n_unit > 0x7fffffff) return PA_ERR_ARG;
     hipStream_t hs = pa::as_stream(stream);

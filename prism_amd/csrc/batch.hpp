@@ -39,19 +39,21 @@ int64_t batch_gap_blocks(const BatchField& f);
 int64_t batch_shuf_blocks(const pa_layout* L);
 int64_t batch_tile_units(const pa_layout* L, int dtype);  // spline workgroups
 int64_t retr_tile_units(const pa_layout* L, int dtype);   // reconstruction workgroups
+bool retr_lone_tiles(int dtype, int64_t nx, int64_t nz);  // float32 tiles taken one by one
 int64_t batch_merge_blocks(const pa_layout* L, int dtype);
 // host-side preparation of a descriptor (layout filled): tuner sampling,
 // alpha, code gaps
 void batch_predict_setup(BatchField& f);
 
-// A batch of retrieval rounds: jobs [0, nj32) hold float32 fields.
+// A batch of retrieval rounds: jobs [0, nj32) hold float32 fields, those from
+// njpair on with lone tiles.
 struct RetrDev {
     const RetrJob* jobs;
-    int nj, nj32;
+    int nj, nj32, njpair;
     const int64_t* p_unshuf;  // inverse-shuffle workgroups
-    const int64_t* p_unit;    // reconstruction workgroups (float32: twice the spline's)
+    const int64_t* p_unit;    // reconstruction workgroups (float32: of two tiles, but for lone ones)
     int64_t* p_chunk;         // selected chunks (device-computed exclusive prefix, nj + 1)
-    int64_t n_unshuf, n_unit, n_unit32, max_chunks;
+    int64_t n_unshuf, n_unit, n_unit32, n_unitpair, max_chunks;
 };
 
 int retr_strategy(const RetrDev& r, hipStream_t st);     // strategy.hip

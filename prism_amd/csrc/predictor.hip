@@ -635,9 +635,9 @@ __device__ __forceinline__ void plane_codes_store(const Tile<T, IN>& t, const Pl
 // The previous reconstruction of the group (delta form): a row lane's column,
 // z = 0..15.
 constexpr int kOutIters = 16;
-template <typename T, bool IN>
+template <int P, typename T, bool IN>
 __device__ __forceinline__ void prev_load(const Tile<T, IN>& m, const T* old, T (&prev)[kOutIters]) {
-    const RowLane<kGroup<T, DECOMPRESS>> r;
+    const RowLane<P> r;
     const bool on = m.template in<0>(r.X) && m.template in<1>(r.y);
     const uint32_t nx = (uint32_t)m.g.nx, nxy = nx * (uint32_t)m.g.ny;
     Column<const T, IN> src(old + ((uint64_t)m.oz * nxy + (uint64_t)m.oy * nx + m.ox), nx, nxy, r.X, r.y);
@@ -654,10 +654,10 @@ __device__ __forceinline__ void prev_load(const Tile<T, IN>& m, const T* old, T 
 // whole cache lines (`lines`), without a place in the caches (384 x 384 x 256
 // float64 rounds 144 against 153 us).  A line written in two parts is
 // combined in the L2 instead (301 x 257 x 385 float64: 125 against 179 us).
-template <typename T, bool IN>
+template <int P, typename T, bool IN>
 __device__ __forceinline__ void tile_out(const Tile<T, IN>& m, bool delta, bool lines, const T (&prev)[kOutIters],
                                          T* out) {
-    const RowLane<kGroup<T, DECOMPRESS>> r;
+    const RowLane<P> r;
     if (!(m.template in<0>(r.X) && m.template in<1>(r.y))) return;
     const uint32_t nx = (uint32_t)m.g.nx, nxy = nx * (uint32_t)m.g.ny;
     const T* src = m.s + r.slot(r.y, 0);
@@ -697,10 +697,9 @@ enum CodeSrc { CODES_32, CODES_16, CODES_PLANES };
 // DELTA: a delta round (a.old given), a compile-time fact so that the
 // previous values' loads are unconditional in interior tiles and the code
 // slots wait for the code loads alone
-template <typename T, int M, bool IN, int CS = CODES_32, bool DELTA = false>
+template <typename T, int M, int P, bool IN, int CS = CODES_32, bool DELTA = false>
 __device__ __forceinline__ void tile_run(const SplineArgs<T>& a, T* lds, int px, int by, int bz) {
     const Geom& g = a.g;
-    constexpr int P = kGroup<T, M>;
     // this wave's tile, and the group taken as one tile of 16 P + 1 columns
     const int h = P == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / kThreads), bx = px * P + h;
     Tile<T, IN> t = make_tile<T, IN>(g, lds + h * kTileLds, bx, by, bz, a.qc_out);
@@ -729,18 +728,18 @@ __device__ __forceinline__ void tile_run(const SplineArgs<T>& a, T* lds, int px,
         if constexpr (CS == CODES_PLANES) {
             PlaneCodes<T> c;
             plane_codes_load(t, a.ps, maxlevel, a.anchors_in, bx, by, bz, c);
-            if constexpr (DELTA) prev_load(m, a.old, prev);
+            if constexpr (DELTA) prev_load<P>(m, a.old, prev);
             __builtin_amdgcn_s_setprio(0);
             plane_codes_store(t, c);
         } else {
             TileCodes<T> c;
             if constexpr (CS == CODES_16)
-                codes_load(t, m, reinterpret_cast<const int16_t*>(a.qc_in), maxlevel, a.anchors_in, bx, by, bz, c);
+                codes_load<P>(t, m, reinterpret_cast<const int16_t*>(a.qc_in), maxlevel, a.anchors_in, bx, by, bz, c);
             else
-                codes_load(t, m, a.qc_in, maxlevel, a.anchors_in, bx, by, bz, c);
-            if constexpr (DELTA) prev_load(m, a.old, prev);
+                codes_load<P>(t, m, a.qc_in, maxlevel, a.anchors_in, bx, by, bz, c);
+            if constexpr (DELTA) prev_load<P>(m, a.old, prev);
             __builtin_amdgcn_s_setprio(0);
-            codes_store(t, m, c);
+            codes_store<P>(t, m, c);
         }
         __syncthreads();
     }
@@ -748,14 +747,14 @@ __device__ __forceinline__ void tile_run(const SplineArgs<T>& a, T* lds, int px,
     tile_levels<T, M>(t, a.le, flags_mask(fl), maxlevel);
 
     if constexpr (M == COMPRESS) live_join(codes_out(m), seen, a.live);
-    else tile_out(m, DELTA, (((uintptr_t)a.out | (uint64_t)g.nx * sizeof(T)) & 127) == 0, prev, a.out);
+    else tile_out<P>(m, DELTA, (((uintptr_t)a.out | (uint64_t)g.nx * sizeof(T)) & 127) == 0, prev, a.out);
 }
 
 // a decompressing tile of either form: delta (a.old given) or anchored
-template <typename T, bool IN, int CS>
+template <typename T, int P, bool IN, int CS>
 __device__ __forceinline__ void tile_run_dec(const SplineArgs<T>& a, T* lds, int px, int by, int bz) {
-    if (a.old) tile_run<T, DECOMPRESS, IN, CS, true>(a, lds, px, by, bz);
-    else tile_run<T, DECOMPRESS, IN, CS, false>(a, lds, px, by, bz);
+    if (a.old) tile_run<T, DECOMPRESS, P, IN, CS, true>(a, lds, px, by, bz);
+    else tile_run<T, DECOMPRESS, P, IN, CS, false>(a, lds, px, by, bz);
 }
 
 // ------------------------------------------------------------ 2-D fields --
@@ -1179,38 +1178,38 @@ constexpr int kTileWaves = sizeof(T) == 4 ? 6 : 4;
 // plus old for the delta form).  Tiles away from the far faces of the field
 // (all 17^3 points inside) run a variant whose boundary tests are resolved
 // at compile time.
-template <typename T, int M>
-__global__ __launch_bounds__((kGroupThreads<T, M>)) __attribute__((amdgpu_waves_per_eu(kTileWaves<T>))) void spline_kernel(SplineArgs<T> a) {
-    __shared__ T tile[kGroup<T, M> * kTileLds];
+template <typename T, int M, int P>
+__global__ __launch_bounds__(P * kThreads) __attribute__((amdgpu_waves_per_eu(kTileWaves<T>))) void spline_kernel(SplineArgs<T> a) {
+    __shared__ T tile[P * kTileLds];
     clear_gaps<T, M>(a);
     // XCD-aware tile order: workgroups are dealt round-robin to the 8 XCDs,
     // so workgroup b runs on XCD b mod 8; each XCD takes a contiguous range
     // of tiles (x fastest) and the cache lines that neighbouring tiles share
     // (halo rows and columns, level-major code runs) meet in one L2.
     const Geom& g = a.g;
-    const int64_t ntiles = (int64_t)groups_x<kGroup<T, M>>(g) * g.gy * g.gz;
+    const int64_t ntiles = (int64_t)groups_x<P>(g) * g.gy * g.gz;
     const int64_t b = blockIdx.x, xcd = b % kXcds, per = ntiles / kXcds, extra = ntiles % kXcds;
     const int64_t tix = xcd * per + (xcd < extra ? xcd : extra) + b / kXcds;
-    const int gpx = groups_x<kGroup<T, M>>(g);
+    const int gpx = groups_x<P>(g);
     const int px = (int)(tix % gpx), by = (int)((tix / gpx) % g.gy), bz = (int)(tix / ((int64_t)gpx * g.gy));
-    const bool interior = interior_group<kGroup<T, M>>(g, px, by, bz);
+    const bool interior = interior_group<P>(g, px, by, bz);
     const SplineArgs<T> r = resolve(a);
     if constexpr (M == DECOMPRESS) {
         if (r.planes) {
-            if (interior) tile_run_dec<T, true, CODES_PLANES>(r, tile, px, by, bz);
-            else tile_run_dec<T, false, CODES_PLANES>(r, tile, px, by, bz);
+            if (interior) tile_run_dec<T, P, true, CODES_PLANES>(r, tile, px, by, bz);
+            else tile_run_dec<T, P, false, CODES_PLANES>(r, tile, px, by, bz);
             return;
         }
         if (r.q16) {
-            if (interior) tile_run_dec<T, true, CODES_16>(r, tile, px, by, bz);
-            else tile_run_dec<T, false, CODES_16>(r, tile, px, by, bz);
+            if (interior) tile_run_dec<T, P, true, CODES_16>(r, tile, px, by, bz);
+            else tile_run_dec<T, P, false, CODES_16>(r, tile, px, by, bz);
             return;
         }
-        if (interior) tile_run_dec<T, true, CODES_32>(r, tile, px, by, bz);
-        else tile_run_dec<T, false, CODES_32>(r, tile, px, by, bz);
+        if (interior) tile_run_dec<T, P, true, CODES_32>(r, tile, px, by, bz);
+        else tile_run_dec<T, P, false, CODES_32>(r, tile, px, by, bz);
     } else {
-        if (interior) tile_run<T, M, true>(r, tile, px, by, bz);
-        else tile_run<T, M, false>(r, tile, px, by, bz);
+        if (interior) tile_run<T, M, P, true>(r, tile, px, by, bz);
+        else tile_run<T, M, P, false>(r, tile, px, by, bz);
     }
 }
 
@@ -1603,7 +1602,7 @@ __global__ void batch_keys_init_kernel(BatchField* fields, int nf) {
 // order of spline_kernel taken over the concatenated list of work units: a
 // tile, 4 tiles of a 2-D field or 256 tiles of a 1-D field.
 template <typename T>
-__global__ __launch_bounds__((kGroupThreads<T, COMPRESS>)) __attribute__((amdgpu_waves_per_eu(kTileWaves<T>))) void batch_spline_kernel(
+__global__ __launch_bounds__((kGroup<T, COMPRESS> * kThreads)) __attribute__((amdgpu_waves_per_eu(kTileWaves<T>))) void batch_spline_kernel(
     const BatchField* __restrict__ fields, const int64_t* __restrict__ prefix, int lo, int hi, int64_t base,
     int64_t ntiles, int xcd_order) {
     __shared__ T tile[kGroup<T, COMPRESS> * kTileLds];
@@ -1628,18 +1627,18 @@ __global__ __launch_bounds__((kGroupThreads<T, COMPRESS>)) __attribute__((amdgpu
     const int gpx = groups_x<kGroup<T, COMPRESS>>(g);
     const int px = (int)(tix % gpx), by = (int)((tix / gpx) % g.gy), bz = (int)(tix / ((int64_t)gpx * g.gy));
     const bool interior = interior_group<kGroup<T, COMPRESS>>(g, px, by, bz);
-    if (interior) tile_run<T, COMPRESS, true>(a, tile, px, by, bz);
-    else tile_run<T, COMPRESS, false>(a, tile, px, by, bz);
+    if (interior) tile_run<T, COMPRESS, kGroup<T, COMPRESS>, true>(a, tile, px, by, bz);
+    else tile_run<T, COMPRESS, kGroup<T, COMPRESS>, false>(a, tile, px, by, bz);
 }
 
 // Reconstruction units of a batch of retrieval rounds, jobs [lo, hi) (one
 // dtype): the anchored form on a field's first round, the delta form on old
 // after that; levels above the round's maxlevel are skipped.
-template <typename T>
-__global__ __launch_bounds__((kGroupThreads<T, DECOMPRESS>)) __attribute__((amdgpu_waves_per_eu(kTileWaves<T>))) void retr_spline_kernel(
+template <typename T, int P>
+__global__ __launch_bounds__(P * kThreads) __attribute__((amdgpu_waves_per_eu(kTileWaves<T>))) void retr_spline_kernel(
     const RetrJob* __restrict__ jobs, const int64_t* __restrict__ prefix, int lo, int hi, int64_t base,
     int64_t nunits) {
-    __shared__ T tile[kGroup<T, DECOMPRESS> * kTileLds];
+    __shared__ T tile[P * kTileLds];
     const int64_t b = blockIdx.x, xcd = b % kXcds, per = nunits / kXcds, extra = nunits % kXcds;
     const int64_t gt = base + xcd * per + (xcd < extra ? xcd : extra) + b / kXcds;
     const int j = find_field(prefix, lo, hi, gt);
@@ -1670,28 +1669,28 @@ __global__ __launch_bounds__((kGroupThreads<T, DECOMPRESS>)) __attribute__((amdg
     const int64_t tix = gt - prefix[j];
     if (line_field(g)) {  // one unit per 256 lanes
         const int h = threadIdx.x / kThreads;
-        line_tiles<T, DECOMPRESS>(a, tile + h * kLineSlots, tix * kGroup<T, DECOMPRESS> + h);
+        line_tiles<T, DECOMPRESS>(a, tile + h * kLineSlots, tix * P + h);
         return;
     }
     if (plane_field(g)) {
         plane_tiles<T, DECOMPRESS>(a, tile, tix);
         return;
     }
-    const int gpx = groups_x<kGroup<T, DECOMPRESS>>(g);
+    const int gpx = groups_x<P>(g);
     const int px = (int)(tix % gpx), by = (int)((tix / gpx) % g.gy), bz = (int)(tix / ((int64_t)gpx * g.gy));
-    const bool interior = interior_group<kGroup<T, DECOMPRESS>>(g, px, by, bz);
+    const bool interior = interior_group<P>(g, px, by, bz);
     if (a.planes) {
-        if (interior) tile_run_dec<T, true, CODES_PLANES>(a, tile, px, by, bz);
-        else tile_run_dec<T, false, CODES_PLANES>(a, tile, px, by, bz);
+        if (interior) tile_run_dec<T, P, true, CODES_PLANES>(a, tile, px, by, bz);
+        else tile_run_dec<T, P, false, CODES_PLANES>(a, tile, px, by, bz);
         return;
     }
     if (a.q16) {
-        if (interior) tile_run_dec<T, true, CODES_16>(a, tile, px, by, bz);
-        else tile_run_dec<T, false, CODES_16>(a, tile, px, by, bz);
+        if (interior) tile_run_dec<T, P, true, CODES_16>(a, tile, px, by, bz);
+        else tile_run_dec<T, P, false, CODES_16>(a, tile, px, by, bz);
         return;
     }
-    if (interior) tile_run_dec<T, true, CODES_32>(a, tile, px, by, bz);
-    else tile_run_dec<T, false, CODES_32>(a, tile, px, by, bz);
+    if (interior) tile_run_dec<T, P, true, CODES_32>(a, tile, px, by, bz);
+    else tile_run_dec<T, P, false, CODES_32>(a, tile, px, by, bz);
 }
 
 // ------------------------------------------------------------- host side --
@@ -1739,9 +1738,12 @@ int launch_spline(const pa_layout* L, const T* data, double eb, double rel_eb, c
     else if (plane_field(g))
         hipLaunchKernelGGL((plane_kernel<T, M>), dim3((unsigned)((ntiles + kPlaneWaves - 1) / kPlaneWaves)),
                            dim3(kThreads), 0, st, args);
+    else if (lone_tiles<T, M>(g.nx, g.nz))
+        hipLaunchKernelGGL((spline_kernel<T, M, 1>), dim3((unsigned)ntiles), dim3(kThreads), 0, st, args);
     else
-        hipLaunchKernelGGL((spline_kernel<T, M>), dim3((unsigned)(groups_x<kGroup<T, M>>(g) * ((int64_t)g.gy * g.gz))),
-                           dim3(kGroupThreads<T, M>), 0, st, args);
+        hipLaunchKernelGGL((spline_kernel<T, M, kGroup<T, M>>),
+                           dim3((unsigned)(groups_x<kGroup<T, M>>(g) * ((int64_t)g.gy * g.gz))),
+                           dim3(kGroup<T, M> * kThreads), 0, st, args);
     PA_LAUNCH_CHECK();
     return PA_OK;
 }
@@ -2043,7 +2045,7 @@ int pa::batch_keys_init(const BatchDev& b, hipStream_t st) {
 
 int pa::batch_spline(const BatchDev& b, hipStream_t st) {
     if (b.n_tile32 > 0) {
-        hipLaunchKernelGGL(batch_spline_kernel<float>, dim3((unsigned)b.n_tile32), dim3(kGroupThreads<float, COMPRESS>), 0, st, b.fields,
+        hipLaunchKernelGGL(batch_spline_kernel<float>, dim3((unsigned)b.n_tile32), dim3(kGroup<float, COMPRESS> * kThreads), 0, st, b.fields,
                            b.p_tile, 0, b.nf32, (int64_t)0, b.n_tile32, b.xcd_order);
         PA_LAUNCH_CHECK();
     }
@@ -2069,8 +2071,13 @@ int64_t pa::batch_tile_units(const pa_layout* L, int dtype) {
     return dtype == PA_F32 ? spline_units<kGroup<float, COMPRESS>>(L) : spline_units<kGroup<double, COMPRESS>>(L);
 }
 
+bool pa::retr_lone_tiles(int dtype, int64_t nx, int64_t nz) {
+    return dtype == PA_F32 && lone_tiles<float, DECOMPRESS>(nx, nz);
+}
+
 int64_t pa::retr_tile_units(const pa_layout* L, int dtype) {
-    return dtype == PA_F32 ? spline_units<kGroup<float, DECOMPRESS>>(L) : spline_units<kGroup<double, DECOMPRESS>>(L);
+    static_assert(kGroup<double, DECOMPRESS> == 1, "float64 tiles are taken one by one");
+    return dtype == PA_F32 && !retr_lone_tiles(dtype, L->nx, L->nz) ? spline_units<kGroup<float, DECOMPRESS>>(L) : spline_units<1>(L);
 }
 
 void pa::retr_level_ebs(RetrJob& j, double eb, double rel_eb) {
@@ -2084,16 +2091,19 @@ void pa::retr_level_ebs(RetrJob& j, double eb, double rel_eb) {
     }
 }
 
-int pa::retr_reconstruct(const RetrDev& r, hipStream_t st) {
-    if (r.n_unit32 > 0) {
-        hipLaunchKernelGGL(retr_spline_kernel<float>, dim3((unsigned)r.n_unit32), dim3(kGroupThreads<float, DECOMPRESS>), 0, st, r.jobs,
-                           r.p_unit, 0, r.nj32, (int64_t)0, r.n_unit32);
-        PA_LAUNCH_CHECK();
-    }
-    if (r.n_unit - r.n_unit32 > 0) {
-        hipLaunchKernelGGL(retr_spline_kernel<double>, dim3((unsigned)(r.n_unit - r.n_unit32)), dim3(kThreads), 0, st,
-                           r.jobs, r.p_unit, r.nj32, r.nj, r.n_unit32, r.n_unit - r.n_unit32);
-        PA_LAUNCH_CHECK();
-    }
+// the units of jobs [lo, hi), P tiles each
+template <typename T, int P>
+static int retr_launch(const RetrDev& r, int lo, int hi, int64_t base, int64_t nunits, hipStream_t st) {
+    if (nunits <= 0) return PA_OK;
+    hipLaunchKernelGGL((retr_spline_kernel<T, P>), dim3((unsigned)nunits), dim3(P * kThreads), 0, st, r.jobs, r.p_unit, lo,
+                       hi, base, nunits);
+    PA_LAUNCH_CHECK();
     return PA_OK;
+}
+
+int pa::retr_reconstruct(const RetrDev& r, hipStream_t st) {
+    int e = retr_launch<float, kGroup<float, DECOMPRESS>>(r, 0, r.njpair, 0, r.n_unitpair, st);
+    if (e == PA_OK) e = retr_launch<float, 1>(r, r.njpair, r.nj32, r.n_unitpair, r.n_unit32 - r.n_unitpair, st);
+    if (e == PA_OK) e = retr_launch<double, 1>(r, r.nj32, r.nj, r.n_unit32, r.n_unit - r.n_unit32, st);
+    return e;
 }

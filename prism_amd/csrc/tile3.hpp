@@ -52,8 +52,15 @@ constexpr int slot_half() {
 // against 372 us: half as many waves meet at each of its 13 barriers).
 template <typename T, int M>
 constexpr int kGroup = sizeof(T) == 4 && M == DECOMPRESS ? 2 : 1;
+
+// A field of one tile along x has no tiles to pair, and its tiles are taken one by
+// one.  (With the second half of every workgroup idle instead, decompressing
+// 4 x 4096 x 4096 float32 values took 1122 us, 16 x 2048 x 2048 448; 671 and 338
+// one by one.)
 template <typename T, int M>
-constexpr int kGroupThreads = kGroup<T, M> * kThreads;
+inline bool lone_tiles(int64_t nx, int64_t nz) {
+    return kGroup<T, M> > 1 && nx <= 16 && nz > 1;
+}
 
 // IN: not the last tile along any axis, all 17^3 points inside the field
 // (every stencil then is decided at compile time), and rows short enough for
@@ -743,7 +750,7 @@ __device__ __forceinline__ bool coarse_point(int l, int& unit, int& i, int& j, i
     return m < (l3 ? 27 : 125);
 }
 
-template <typename T, bool IN, typename E>
+template <int P, typename T, bool IN, typename E>
 __device__ __forceinline__ void codes_load(const Tile<T, IN>& t, const Tile<T, IN>& m, const E* __restrict__ q, int maxlevel,
                                            const T* __restrict__ anchors, int bx, int by, int bz, TileCodes<T>& c) {
     const int l = lane_id();
@@ -766,7 +773,7 @@ __device__ __forceinline__ void codes_load(const Tile<T, IN>& t, const Tile<T, I
         if (maxlevel >= 1 && p < 729 && ((i | j | k) & 1) && t.in3(2 * i, 2 * j, 2 * k))
             c.v1[it] = q[lm_at<1>(t, 2 * i, 2 * j, 2 * k)];
     }
-    const RowLane<kGroup<T, DECOMPRESS>> r;
+    const RowLane<P> r;
     const bool on = l0 && m.template in<0>(r.X) && m.template in<1>(r.y), on_even = on && ((r.X | r.y) & 1);
     Columns0<const E, IN> col(m, q, r.X, r.y);
 #pragma unroll
@@ -788,7 +795,7 @@ __device__ __forceinline__ void codes_load(const Tile<T, IN>& t, const Tile<T, I
     c.anc = anchor_load(t, anchors, bx, by, bz);
 }
 
-template <typename T, bool IN>
+template <int P, typename T, bool IN>
 __device__ __forceinline__ void codes_store(const Tile<T, IN>& t, const Tile<T, IN>& m, const TileCodes<T>& c) {
     const int l = lane_id();
     {
@@ -800,7 +807,7 @@ __device__ __forceinline__ void codes_store(const Tile<T, IN>& t, const Tile<T, 
         const int p = l + it * kThreads, i = p % 9, j = (p / 9) % 9, k = p / 81;
         if (p < 729 && ((i | j | k) & 1)) t.s[tslot(2 * i, 2 * j, 2 * k)] = code_slot(c.v1[it], T());
     }
-    const RowLane<kGroup<T, DECOMPRESS>> r;
+    const RowLane<P> r;
     T* d = m.s + r.slot(r.y, 0);
 #pragma unroll
     for (int k = 0; k < 8; ++k) d[(2 * k + 1) * kZP] = code_slot(c.v0[2 * k + 1], T());
