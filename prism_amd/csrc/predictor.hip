@@ -651,11 +651,20 @@ __device__ __forceinline__ void prev_load(const Tile<T, IN>& m, const T* old, T 
 
 // The reconstructed group (plus the previous one in the delta form) to `out`.
 // It is written once and read only by a later round: where a group's rows are
-// whole cache lines (`lines`), without a place in the caches (384 x 384 x 256
+// whole cache lines (`nt`), without a place in the caches (384 x 384 x 256
 // float64 rounds 144 against 153 us).  A line written in two parts is
-// combined in the L2 instead (301 x 257 x 385 float64: 125 against 179 us).
+// combined in the L2 instead (301 x 257 x 385 float64: 125 against 179 us).  In
+// the anchored form rows of whole 32-byte sectors are enough: decompressing 1000 x
+// 4000 x 17 values takes 575 us, 652 through the caches (float64), and 461, 515
+// (float32); 1000 x 1000 x 64 451, 502 and 384, 410; 500 x 500 x 300 float64 572,
+// 569.  Delta rounds of such rows do not gain (that field's three rounds with
+// every store past the caches: 1548 us, 1389 without).
+template <bool DELTA>
+__device__ __forceinline__ bool bypass(const void* out, int64_t row_bytes) {
+    return (((uintptr_t)out | (uint64_t)row_bytes) & (DELTA ? 127 : 31)) == 0;
+}
 template <int P, typename T, bool IN>
-__device__ __forceinline__ void tile_out(const Tile<T, IN>& m, bool delta, bool lines, const T (&prev)[kOutIters],
+__device__ __forceinline__ void tile_out(const Tile<T, IN>& m, bool delta, bool nt, const T (&prev)[kOutIters],
                                          T* out) {
     const RowLane<P> r;
     if (!(m.template in<0>(r.X) && m.template in<1>(r.y))) return;
@@ -664,7 +673,7 @@ __device__ __forceinline__ void tile_out(const Tile<T, IN>& m, bool delta, bool 
     Column<T, IN> dst(out + ((uint64_t)m.oz * nxy + (uint64_t)m.oy * nx + m.ox), nx, nxy, r.X, r.y);
     // the compiler would join the two forms' stores and drop the hint: the
     // empty statements keep them apart
-    if (lines) {
+    if (nt) {
         asm volatile("");
 #pragma unroll
         for (int z = 0; z < kOutIters; ++z) {
@@ -747,7 +756,7 @@ __device__ __forceinline__ void tile_run(const SplineArgs<T>& a, T* lds, int px,
     tile_levels<T, M>(t, a.le, flags_mask(fl), maxlevel);
 
     if constexpr (M == COMPRESS) live_join(codes_out(m), seen, a.live);
-    else tile_out<P>(m, DELTA, (((uintptr_t)a.out | (uint64_t)g.nx * sizeof(T)) & 127) == 0, prev, a.out);
+    else tile_out<P>(m, DELTA, bypass<DELTA>(a.out, (int64_t)g.nx * sizeof(T)), prev, a.out);
 }
 
 // a decompressing tile of either form: delta (a.old given) or anchored
