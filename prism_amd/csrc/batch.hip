@@ -482,7 +482,7 @@ extern "C" int pa_retrieve_batch(const pa_retrieve_job* jobs, int nj, void* h_ta
     int64_t* p_chunk = reinterpret_cast<int64_t*>(ws + tb.total + retr_keys_bytes(nj));
     // float32 jobs first: those whose tiles are paired, then the others
     int k = 0, nj32 = 0, njpair = 0;
-    int64_t max_chunks = 0;
+    int64_t max_chunks = 0, out_bytes = 0;
     p_unshuf[0] = p_unit[0] = 0;
     for (int pass = 0; pass < 3; ++pass)
         for (int i = 0; i < nj; ++i) {
@@ -495,6 +495,7 @@ extern "C" int pa_retrieve_batch(const pa_retrieve_job* jobs, int nj, void* h_ta
             p_unshuf[k + 1] = p_unshuf[k] + pa::retr_unshuf_blocks(&j.L);
             p_unit[k + 1] = p_unit[k] + pa::retr_tile_units(&j.L, j.dtype);
             max_chunks += j.L.nchunks;
+            out_bytes += j.L.n * j.dtype;
             nj32 += pass < 2;
             njpair += pass == 0;
             ++k;
@@ -512,6 +513,7 @@ extern "C" int pa_retrieve_batch(const pa_retrieve_job* jobs, int nj, void* h_ta
     r.n_unit32 = p_unit[nj32];
     r.n_unitpair = p_unit[njpair];
     r.max_chunks = max_chunks;
+    r.out_bytes = out_bytes;
     if (r.n_unshuf > 0x7fffffff || r.n_unit > 0x7fffffff) return PA_ERR_ARG;
     hipStream_t hs = pa::as_stream(stream);
     if (h_table) {

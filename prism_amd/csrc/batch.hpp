@@ -54,6 +54,7 @@ struct RetrDev {
     const int64_t* p_unit;    // reconstruction workgroups (float32: of two tiles, but for lone ones)
     int64_t* p_chunk;         // selected chunks (device-computed exclusive prefix, nj + 1)
     int64_t n_unshuf, n_unit, n_unit32, n_unitpair, max_chunks;
+    int64_t out_bytes;        // of all jobs' reconstructions
 };
 
 int retr_strategy(const RetrDev& r, hipStream_t st);     // strategy.hip

@@ -455,6 +455,7 @@ struct SplineArgs {
     int gaps_on;  // (its workgroups share them out; disjoint from the codes)
     PlaneSrc ps;  // decompression: the round's bit-planes (ps.bp null: none)
     bool planes;  // resolved: the codes come from ps
+    bool cached = false;  // decompression: the launch's output goes through the caches (kCachedOut)
     uint64_t* live = nullptr;  // compression: where the codes' magnitudes go (live_words), or null
 };
 
@@ -767,6 +768,16 @@ __device__ __forceinline__ void tile_run_dec(const SplineArgs<T>& a, T* lds, int
 }
 
 // ------------------------------------------------------------ 2-D fields --
+// Bytes of a launch's reconstructions up to which 2-D fields are written through
+// the caches: a delta round then finds the previous reconstruction there, as 256
+// MB hold both.  A delta round in microseconds, through the caches / past them:
+// 2048^2 float32 24.3 / 25.8, float64 27.8 / 29.4; 4096^2 float32 (67 MB) 78.3 /
+// 83.0; 3000^2 float64 (72 MB) 53.4 / 56.4; but 4096^2 float64 (134 MB) 99.5 /
+// 95.7, 6000^2 float32 (144 MB) 177.9 / 174.7, float64 206 / 201.  An anchored round
+// alone is faster past them (4096^2 float32 73.3 / 71.9), by less than it costs
+// the next one (three rounds 403 / 417).
+constexpr int64_t kCachedOut = (int64_t)100 << 20;
+
 // A field with nz = 1 (and ny > 1) holds only the plane z = 0 of each tile.
 // Of the stages only these have points inside it: YELLOW / YELLOW_R
 // (y-lines), HOLLOW / HOLLOW_R (x-lines), and in the multi-dimensional form
@@ -843,11 +854,12 @@ __device__ __forceinline__ int plane_point_level(int x, int y) {
     return __builtin_ctz(m) > 4 ? 4 : __builtin_ctz(m);
 }
 
-template <typename T, int M>
+// (P: 256 lanes of the workgroup)
+template <typename T, int M, int P>
 __device__ __forceinline__ void plane_tiles(const SplineArgs<T>& a, T* lds, int64_t unit) {
     const Geom& g = a.g;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int64_t tile = unit * (blockDim.x >> 6) + wave;
+    const int64_t tile = unit * (P * kPlaneWaves) + wave;
     if (tile >= (int64_t)g.gx * g.gy) return;  // no workgroup barrier follows
     const int bx = (int)(tile % g.gx), by = (int)(tile / g.gx);
     Ctx<T> t;
@@ -924,15 +936,31 @@ __device__ __forceinline__ void plane_tiles(const SplineArgs<T>& a, T* lds, int6
     if (1 <= maxlevel) { t.eb_r = le.eb_r[1]; t.ebx2 = le.ebx2[1]; plane_level<T, 2, M>(t, lane, fl[1], fl[5]); }
     if (0 <= maxlevel) { t.eb_r = le.eb_r[0]; t.ebx2 = le.ebx2[0]; plane_level<T, 1, M>(t, lane, fl[0], fl[4]); }
     if constexpr (M == DECOMPRESS) {
+        T v[4];
+        bool in[4];
+        int64_t at[4];
 #pragma unroll
         for (int it = 0; it < 4; ++it) {  // the 16 x 16 own points: lane -> x = lane mod 16, y = lane / 16 + 4 it
             const int x = lane & 15, y = (lane >> 4) + 4 * it;
             const int gx = t.ox + x, gy = t.oy + y;
-            if (gx < g.nx && gy < g.ny) {
-                const int64_t o = (int64_t)gx + (int64_t)gy * g.nx;
-                const T v = t.s[sidx(x, y, 0)];
-                a.out[o] = a.old ? v + a.old[o] : v;  // (lines written in parts: combined in the L2)
-            }
+            in[it] = gx < g.nx && gy < g.ny;
+            at[it] = (int64_t)gx + (int64_t)gy * g.nx;
+            v[it] = t.s[sidx(x, y, 0)];
+            if (a.old && in[it]) v[it] += a.old[at[it]];
+        }
+        // past the caches, but where the next round finds `old` there (the two forms
+        // kept apart as in tile_out)
+        if (a.cached) {
+            asm volatile("");
+#pragma unroll
+            for (int it = 0; it < 4; ++it)
+                if (in[it]) a.out[at[it]] = v[it];
+        } else {
+            asm volatile("");
+#pragma unroll
+            for (int it = 0; it < 4; ++it)
+                if (in[it]) __builtin_nontemporal_store(v[it], &a.out[at[it]]);
+            asm volatile("");
         }
     }
 }
@@ -953,7 +981,7 @@ template <typename T, int M>
 __global__ __launch_bounds__(kThreads) void plane_kernel(SplineArgs<T> a) {
     __shared__ T lds[kPlaneWaves * kPlaneVals];
     clear_gaps<T, M>(a);
-    plane_tiles<T, M>(resolve(a), lds, blockIdx.x);
+    plane_tiles<T, M, 1>(resolve(a), lds, blockIdx.x);
 }
 
 __host__ __device__ inline bool plane_field(const Geom& g) { return g.nz == 1 && g.ny > 1; }
@@ -1630,7 +1658,7 @@ __global__ __launch_bounds__((kGroup<T, COMPRESS> * kThreads)) __attribute__((am
         return;
     }
     if (plane_field(g)) {
-        plane_tiles<T, COMPRESS>(a, tile, tix);
+        plane_tiles<T, COMPRESS, kGroup<T, COMPRESS>>(a, tile, tix);
         return;
     }
     const int gpx = groups_x<kGroup<T, COMPRESS>>(g);
@@ -1646,7 +1674,7 @@ __global__ __launch_bounds__((kGroup<T, COMPRESS> * kThreads)) __attribute__((am
 template <typename T, int P>
 __global__ __launch_bounds__(P * kThreads) __attribute__((amdgpu_waves_per_eu(kTileWaves<T>))) void retr_spline_kernel(
     const RetrJob* __restrict__ jobs, const int64_t* __restrict__ prefix, int lo, int hi, int64_t base,
-    int64_t nunits) {
+    int64_t nunits, bool cached) {
     __shared__ T tile[P * kTileLds];
     const int64_t b = blockIdx.x, xcd = b % kXcds, per = nunits / kXcds, extra = nunits % kXcds;
     const int64_t gt = base + xcd * per + (xcd < extra ? xcd : extra) + b / kXcds;
@@ -1663,6 +1691,7 @@ __global__ __launch_bounds__(P * kThreads) __attribute__((amdgpu_waves_per_eu(kT
     SplineArgs<T> a{nullptr, J.g, le, nullptr, nullptr, src == 1, J.flags, J.state + 8, nullptr, J.qc, nullptr,
                     J.first ? static_cast<const T*>(J.anchors) : nullptr,
                     J.first ? nullptr : static_cast<const T*>(J.old), static_cast<T*>(J.out)};
+    a.cached = cached;
     if (src == 2) {
         a.ps.bp = J.bp;
         a.ps.begin = J.state + 10;  // each level's first live plane
@@ -1682,7 +1711,7 @@ __global__ __launch_bounds__(P * kThreads) __attribute__((amdgpu_waves_per_eu(kT
         return;
     }
     if (plane_field(g)) {
-        plane_tiles<T, DECOMPRESS>(a, tile, tix);
+        plane_tiles<T, DECOMPRESS, P>(a, tile, tix);
         return;
     }
     const int gpx = groups_x<P>(g);
@@ -1741,6 +1770,7 @@ int launch_spline(const pa_layout* L, const T* data, double eb, double rel_eb, c
     }
     if (ps) args.ps = *ps;
     args.live = live;
+    args.cached = L->n * (int64_t)sizeof(T) <= kCachedOut;
     if (line_field(g))
         hipLaunchKernelGGL((line_kernel<T, M>), dim3((unsigned)((ntiles + kLineTiles - 1) / kLineTiles)),
                            dim3(kThreads), 0, st, args);
@@ -2105,7 +2135,7 @@ template <typename T, int P>
 static int retr_launch(const RetrDev& r, int lo, int hi, int64_t base, int64_t nunits, hipStream_t st) {
     if (nunits <= 0) return PA_OK;
     hipLaunchKernelGGL((retr_spline_kernel<T, P>), dim3((unsigned)nunits), dim3(P * kThreads), 0, st, r.jobs, r.p_unit, lo,
-                       hi, base, nunits);
+                       hi, base, nunits, r.out_bytes <= kCachedOut);
     PA_LAUNCH_CHECK();
     return PA_OK;
 }
