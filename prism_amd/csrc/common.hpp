@@ -165,9 +165,10 @@ struct ZeroSpan {
     int64_t lo[4], hi[4];  // per level: bytes [lo, hi) of the bit-planes are zero (empty: lo >= hi)
 };
 
-// Leading planes of magnitudes below 2^b: their negabinary forms take at most
-// b + 2 digits (the digits of the largest and the smallest value of d digits are
-// every other one), their sign-magnitude forms b.
+// Leading planes of codes c whose c ^ (c >> 31) is below 2^b, that is of codes from
+// -2^b to 2^b - 1: their negabinary forms take at most b + 2 digits (the digits of
+// the largest and the smallest value of d digits are every other one), their
+// sign-magnitude forms b + 1 (2^b itself is the magnitude of -2^b).
 __device__ __forceinline__ int zero_planes(uint32_t mags) {
     const int b = 32 - __clz((int)mags);  // (__clz(0) = 32)
     return b + 2 < 32 ? 32 - (b + 2) : 0;
