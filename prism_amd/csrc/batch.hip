@@ -178,7 +178,7 @@ int upload(pa_batch_plan* p, hipStream_t st) {
                                         f.rel ? pa::batch_ext_blocks(&f.L, f.dtype, pa::kExtChoices[3]) : 0,
                                         f.tnblocks,
                                         pa::batch_gap_blocks(f),
-                                        pa::batch_tile_units(&f.L, f.dtype),
+                                        pa::batch_tile_units(&f.L),
                                         pa::batch_shuf_blocks(&f.L),
                                         (f.L.nchunks + 7) / 8 * 8,  // encoder launch slots: whole workgroups
                                         pa::batch_merge_blocks(&f.L, f.dtype)};

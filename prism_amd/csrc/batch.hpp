@@ -37,7 +37,7 @@ constexpr int kEncodeChoices[3] = {2, 4, 8};   // encode_waves candidates
 int64_t batch_ext_blocks(const pa_layout* L, int dtype, int ext_batches);
 int64_t batch_gap_blocks(const BatchField& f);
 int64_t batch_shuf_blocks(const pa_layout* L);
-int64_t batch_tile_units(const pa_layout* L, int dtype);  // spline workgroups
+int64_t batch_tile_units(const pa_layout* L);             // spline workgroups
 int64_t retr_tile_units(const pa_layout* L, int dtype);   // reconstruction workgroups
 bool retr_lone_tiles(int dtype, int64_t nx, int64_t nz);  // float32 tiles taken one by one
 int64_t batch_merge_blocks(const pa_layout* L, int dtype);

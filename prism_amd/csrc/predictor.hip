@@ -725,7 +725,7 @@ __device__ __forceinline__ void tile_run(const SplineArgs<T>& a, T* lds, int px,
     uint64_t seen = 0;
     if constexpr (M == COMPRESS) {
         seen = live_seen(a.live);
-        tile_load(t, m, a.data);
+        tile_load(t, a.data);
         seen = ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(seen >> 32)) << 32) |
                __builtin_amdgcn_readfirstlane((uint32_t)seen);
         __syncthreads();
@@ -756,7 +756,7 @@ __device__ __forceinline__ void tile_run(const SplineArgs<T>& a, T* lds, int px,
 
     tile_levels<T, M>(t, a.le, flags_mask(fl), maxlevel);
 
-    if constexpr (M == COMPRESS) live_join(codes_out(m), seen, a.live);
+    if constexpr (M == COMPRESS) live_join(codes_out(t), seen, a.live);
     else tile_out<P>(m, DELTA, bypass<DELTA>(a.out, (int64_t)g.nx * sizeof(T)), prev, a.out);
 }
 
@@ -1309,23 +1309,8 @@ __global__ __launch_bounds__(kThreads) void tune_kernel(const T* __restrict__ da
     tune_block<T>(data, g, sx0, sy0, sz0, nsx, nsy, blockIdx.x, blockIdx.y, part, tile, red);
 }
 
-// Sum over sample blocks in block order, then the host's pick rule
-// (InterpolationPredictor.cu:2306-2355) on the device.
-__device__ void pick_rule(const double* e, uint8_t* __restrict__ flags);
-
-__device__ void pick_flags(const double* __restrict__ part, int nblocks, double* __restrict__ scores,
-                           uint8_t* __restrict__ flags) {
-    double e[15];
-    for (int c = 0; c < 15; ++c) {
-        double s = 0.0;
-        for (int b = 0; b < nblocks; ++b) s += part[(int64_t)b * 15 + c];
-        e[c] = s;
-        if (scores) scores[c] = s;
-    }
-    pick_rule(e, flags);
-}
-
-// The pick rule on the 15 candidate sums.
+// The host's pick rule (InterpolationPredictor.cu:2306-2355) on the 15 candidate
+// sums.
 __device__ void pick_rule(const double* e, uint8_t* __restrict__ flags) {
     uint8_t f[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     double best;
@@ -1348,8 +1333,8 @@ __device__ void pick_rule(const double* e, uint8_t* __restrict__ flags) {
 
 // The partial sums go through LDS first (one cooperative load instead of a
 // chain of dependent global loads in the one thread that adds them in order).
-// Lane c < 15 then adds candidate c's sums in block order (the order of
-// pick_flags), and lane 0 applies the rule.
+// Lane c < 15 then adds candidate c's sums in block order, and lane 0 applies the
+// rule.
 constexpr int kPickLds = 2048;
 __device__ __forceinline__ void pick_parallel(const double* __restrict__ part, int nblocks, double* __restrict__ scores,
                                               uint8_t* __restrict__ flags, double* s, double* e) {
@@ -1639,10 +1624,10 @@ __global__ void batch_keys_init_kernel(BatchField* fields, int nf) {
 // order of spline_kernel taken over the concatenated list of work units: a
 // tile, 4 tiles of a 2-D field or 256 tiles of a 1-D field.
 template <typename T>
-__global__ __launch_bounds__((kGroup<T, COMPRESS> * kThreads)) __attribute__((amdgpu_waves_per_eu(kTileWaves<T>))) void batch_spline_kernel(
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kTileWaves<T>))) void batch_spline_kernel(
     const BatchField* __restrict__ fields, const int64_t* __restrict__ prefix, int lo, int hi, int64_t base,
     int64_t ntiles, int xcd_order) {
-    __shared__ T tile[kGroup<T, COMPRESS> * kTileLds];
+    __shared__ T tile[kTileLds];
     const int64_t b = blockIdx.x, xcd = b % kXcds, per = ntiles / kXcds, extra = ntiles % kXcds;
     const int64_t gt = base + (xcd_order ? xcd * per + (xcd < extra ? xcd : extra) + b / kXcds : b);
     const int f = find_field(prefix, lo, hi, gt);
@@ -1652,20 +1637,17 @@ __global__ __launch_bounds__((kGroup<T, COMPRESS> * kThreads)) __attribute__((am
     a.live = F.live;
     const Geom& g = a.g;
     const int64_t tix = gt - prefix[f];
-    if (line_field(g)) {  // one unit per 256 lanes
-        const int h = threadIdx.x / kThreads;
-        line_tiles<T, COMPRESS>(a, tile + h * kLineSlots, tix * kGroup<T, COMPRESS> + h);
+    if (line_field(g)) {
+        line_tiles<T, COMPRESS>(a, tile, tix);
         return;
     }
     if (plane_field(g)) {
-        plane_tiles<T, COMPRESS, kGroup<T, COMPRESS>>(a, tile, tix);
+        plane_tiles<T, COMPRESS, 1>(a, tile, tix);
         return;
     }
-    const int gpx = groups_x<kGroup<T, COMPRESS>>(g);
-    const int px = (int)(tix % gpx), by = (int)((tix / gpx) % g.gy), bz = (int)(tix / ((int64_t)gpx * g.gy));
-    const bool interior = interior_group<kGroup<T, COMPRESS>>(g, px, by, bz);
-    if (interior) tile_run<T, COMPRESS, kGroup<T, COMPRESS>, true>(a, tile, px, by, bz);
-    else tile_run<T, COMPRESS, kGroup<T, COMPRESS>, false>(a, tile, px, by, bz);
+    const int bx = (int)(tix % g.gx), by = (int)((tix / g.gx) % g.gy), bz = (int)(tix / ((int64_t)g.gx * g.gy));
+    if (interior_group<1>(g, bx, by, bz)) tile_run<T, COMPRESS, 1, true>(a, tile, bx, by, bz);
+    else tile_run<T, COMPRESS, 1, false>(a, tile, bx, by, bz);
 }
 
 // Reconstruction units of a batch of retrieval rounds, jobs [lo, hi) (one
@@ -1777,12 +1759,13 @@ int launch_spline(const pa_layout* L, const T* data, double eb, double rel_eb, c
     else if (plane_field(g))
         hipLaunchKernelGGL((plane_kernel<T, M>), dim3((unsigned)((ntiles + kPlaneWaves - 1) / kPlaneWaves)),
                            dim3(kThreads), 0, st, args);
-    else if (lone_tiles<T, M>(g.nx, g.nz))
+    else if (M == COMPRESS || lone_tiles<T>(g.nx, g.nz))
         hipLaunchKernelGGL((spline_kernel<T, M, 1>), dim3((unsigned)ntiles), dim3(kThreads), 0, st, args);
-    else
-        hipLaunchKernelGGL((spline_kernel<T, M, kGroup<T, M>>),
-                           dim3((unsigned)(groups_x<kGroup<T, M>>(g) * ((int64_t)g.gy * g.gz))),
-                           dim3(kGroup<T, M> * kThreads), 0, st, args);
+    else {
+        constexpr int P = M == COMPRESS ? 1 : kGroup<T>;
+        hipLaunchKernelGGL((spline_kernel<T, M, P>), dim3((unsigned)(groups_x<P>(g) * ((int64_t)g.gy * g.gz))),
+                           dim3(P * kThreads), 0, st, args);
+    }
     PA_LAUNCH_CHECK();
     return PA_OK;
 }
@@ -2084,7 +2067,7 @@ int pa::batch_keys_init(const BatchDev& b, hipStream_t st) {
 
 int pa::batch_spline(const BatchDev& b, hipStream_t st) {
     if (b.n_tile32 > 0) {
-        hipLaunchKernelGGL(batch_spline_kernel<float>, dim3((unsigned)b.n_tile32), dim3(kGroup<float, COMPRESS> * kThreads), 0, st, b.fields,
+        hipLaunchKernelGGL(batch_spline_kernel<float>, dim3((unsigned)b.n_tile32), dim3(kThreads), 0, st, b.fields,
                            b.p_tile, 0, b.nf32, (int64_t)0, b.n_tile32, b.xcd_order);
         PA_LAUNCH_CHECK();
     }
@@ -2106,17 +2089,15 @@ static int64_t spline_units(const pa_layout* L) {
     return (int64_t)groups_x<P>(g) * g.gy * g.gz;
 }
 
-int64_t pa::batch_tile_units(const pa_layout* L, int dtype) {
-    return dtype == PA_F32 ? spline_units<kGroup<float, COMPRESS>>(L) : spline_units<kGroup<double, COMPRESS>>(L);
-}
+int64_t pa::batch_tile_units(const pa_layout* L) { return spline_units<1>(L); }
 
 bool pa::retr_lone_tiles(int dtype, int64_t nx, int64_t nz) {
-    return dtype == PA_F32 && lone_tiles<float, DECOMPRESS>(nx, nz);
+    return dtype == PA_F32 && lone_tiles<float>(nx, nz);
 }
 
 int64_t pa::retr_tile_units(const pa_layout* L, int dtype) {
-    static_assert(kGroup<double, DECOMPRESS> == 1, "float64 tiles are taken one by one");
-    return dtype == PA_F32 && !retr_lone_tiles(dtype, L->nx, L->nz) ? spline_units<kGroup<float, DECOMPRESS>>(L) : spline_units<1>(L);
+    static_assert(kGroup<double> == 1, "float64 tiles are taken one by one");
+    return dtype == PA_F32 && !retr_lone_tiles(dtype, L->nx, L->nz) ? spline_units<kGroup<float>>(L) : spline_units<1>(L);
 }
 
 void pa::retr_level_ebs(RetrJob& j, double eb, double rel_eb) {
@@ -2141,7 +2122,7 @@ static int retr_launch(const RetrDev& r, int lo, int hi, int64_t base, int64_t n
 }
 
 int pa::retr_reconstruct(const RetrDev& r, hipStream_t st) {
-    int e = retr_launch<float, kGroup<float, DECOMPRESS>>(r, 0, r.njpair, 0, r.n_unitpair, st);
+    int e = retr_launch<float, kGroup<float>>(r, 0, r.njpair, 0, r.n_unitpair, st);
     if (e == PA_OK) e = retr_launch<float, 1>(r, r.njpair, r.nj32, r.n_unitpair, r.n_unit32 - r.n_unitpair, st);
     if (e == PA_OK) e = retr_launch<double, 1>(r, r.nj32, r.nj, r.n_unit32, r.n_unit - r.n_unit32, st);
     return e;

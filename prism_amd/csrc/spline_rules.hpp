@@ -13,7 +13,7 @@ namespace {
 
 constexpr int kThreads = 256;
 
-enum Mode { COMPRESS, DECOMPRESS, TUNE };
+enum Mode { COMPRESS, DECOMPRESS };
 
 template <typename T>
 __device__ __forceinline__ T cubic(T a, T b, T c, T d, bool natural = false) {

@@ -43,23 +43,23 @@ constexpr int slot_half() {
     return A == 0 ? U : (A == 1 ? (U == 1 ? kYO : U / 2 * kYP) : U * kZP);
 }
 
-// A workgroup holds kGroup tiles adjacent along x, 256 lanes each.  A float32
-// tile's rows are 64 bytes, half a cache line: a copy of a 512^3 float32 field
-// in the tiles' access pattern (halo included) takes 322 us, 248 us in pairs
+// A decompressing workgroup holds kGroup tiles adjacent along x, 256 lanes each.  A
+// float32 tile's rows are 64 bytes, half a cache line: a copy of a 512^3 float32
+// field in the tiles' access pattern (halo included) takes 322 us, 248 us in pairs
 // (258 us in fours).  Decompression, which is bound by its accesses, takes
 // pairs (round 4 of that field 287 us against 319 us one by one); compression,
 // which is bound by its stages, is faster with 256-lane workgroups (342
 // against 372 us: half as many waves meet at each of its 13 barriers).
-template <typename T, int M>
-constexpr int kGroup = sizeof(T) == 4 && M == DECOMPRESS ? 2 : 1;
+template <typename T>
+constexpr int kGroup = sizeof(T) == 4 ? 2 : 1;
 
 // A field of one tile along x has no tiles to pair, and its tiles are taken one by
 // one.  (With the second half of every workgroup idle instead, decompressing
 // 4 x 4096 x 4096 float32 values took 1122 us, 16 x 2048 x 2048 448; 671 and 338
 // one by one.)
-template <typename T, int M>
+template <typename T>
 inline bool lone_tiles(int64_t nx, int64_t nz) {
-    return kGroup<T, M> > 1 && nx <= 16 && nz > 1;
+    return kGroup<T> > 1 && nx <= 16 && nz > 1;
 }
 
 // IN: not the last tile along any axis, all 17^3 points inside the field
@@ -549,25 +549,24 @@ struct Columns0 {
     }
 };
 
-// The codes of the group's tiles, all in their slots, written out row by row.
+// The codes of the tile, all in their slots, written out row by row.
 // Level 0: a row lane takes its column's z = 0..15 (rows of 16 or 8 adjacent
-// codes per tile).  Level 1: the group's points with even coordinates, in two
-// passes of 8 adjacent codes per tile and row; levels 2 and 3 in one.
+// codes).  Level 1: the points with even coordinates, in two passes of 8 adjacent
+// codes per row; levels 2 and 3 in one.
 // Returns the magnitudes of the lane's codes (live_words).
 template <typename T, bool IN>
-__device__ __forceinline__ Mags codes_out(const Tile<T, IN>& m) {
-    constexpr int P = kGroup<T, COMPRESS>;
+__device__ __forceinline__ Mags codes_out(const Tile<T, IN>& t) {
     Mags g;
     {
-        const RowLane<P> r;
-        if (m.template in<0>(r.X) && m.template in<1>(r.y)) {
-            const T* src = m.s + r.slot(r.y, 0);
-            Columns0<int32_t, IN> c(m, m.qc_out, r.X, r.y);
+        const RowLane<1> r;
+        if (t.template in<0>(r.X) && t.template in<1>(r.y)) {
+            const T* src = t.s + r.slot(r.y, 0);
+            Columns0<int32_t, IN> c(t, t.qc_out, r.X, r.y);
             const bool on_even = (r.X | r.y) & 1;
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
-                if (m.template in<2>(2 * k + 1)) c.at_odd() = g.fine(slot_code(src[(2 * k + 1) * kZP]));
-                if (on_even && m.template in<2>(2 * k)) c.at_even() = g.fine(slot_code(src[2 * k * kZP]));
+                if (t.template in<2>(2 * k + 1)) c.at_odd() = g.fine(slot_code(src[(2 * k + 1) * kZP]));
+                if (on_even && t.template in<2>(2 * k)) c.at_even() = g.fine(slot_code(src[2 * k * kZP]));
                 c.next();
             }
         }
@@ -575,18 +574,15 @@ __device__ __forceinline__ Mags codes_out(const Tile<T, IN>& m) {
     const int v = thread_id();
 #pragma unroll
     for (int it = 0; it < 2; ++it) {
-        const int X = 2 * (v & (8 * P - 1)), y = 2 * ((v / (8 * P)) & 7), z = 2 * (v / (64 * P) + 4 * it);
-        if (((X | y | z) & 2) && m.in3(X, y, z))
-            m.qc_out[lm_at<1>(m, X, y, z)] = g.coarse(slot_code(m.s[(X >> 4) * kTileLds + tslot(X & 15, y, z)]));
+        const int x = 2 * (v & 7), y = 2 * ((v / 8) & 7), z = 2 * (v / 64 + 4 * it);
+        if (((x | y | z) & 2) && t.in3(x, y, z)) t.qc_out[lm_at<1>(t, x, y, z)] = g.coarse(slot_code(t.s[tslot(x, y, z)]));
     }
-    if (v < 64 * P) {
-        const int X = 4 * (v & (4 * P - 1)), y = 4 * ((v / (4 * P)) & 3), z = 4 * (v / (16 * P));
-        if (((X | y | z) & 4) && m.in3(X, y, z))
-            m.qc_out[lm_at<2>(m, X, y, z)] = g.coarse(slot_code(m.s[(X >> 4) * kTileLds + tslot(X & 15, y, z)]));
-    } else if (v < 64 * P + 8 * P) {
-        const int w = v - 64 * P, X = 8 * (w & (2 * P - 1)), y = 8 * ((w / (2 * P)) & 1), z = 8 * (w / (4 * P));
-        if (((X | y | z) & 8) && m.in3(X, y, z))
-            m.qc_out[lm_at<3>(m, X, y, z)] = g.coarse(slot_code(m.s[(X >> 4) * kTileLds + tslot(X & 15, y, z)]));
+    if (v < 64) {
+        const int x = 4 * (v & 3), y = 4 * ((v / 4) & 3), z = 4 * (v / 16);
+        if (((x | y | z) & 4) && t.in3(x, y, z)) t.qc_out[lm_at<2>(t, x, y, z)] = g.coarse(slot_code(t.s[tslot(x, y, z)]));
+    } else if (v < 72) {
+        const int w = v - 64, x = 8 * (w & 1), y = 8 * ((w / 2) & 1), z = 8 * (w / 4);
+        if (((x | y | z) & 8) && t.in3(x, y, z)) t.qc_out[lm_at<3>(t, x, y, z)] = g.coarse(slot_code(t.s[tslot(x, y, z)]));
     }
     return g;
 }
@@ -681,30 +677,29 @@ struct Column {
 // first LDS write so the tile costs one memory latency.  Points outside the
 // field are not read (no formula uses their slots).
 template <typename T, bool IN>
-__device__ __forceinline__ void tile_load(const Tile<T, IN>& t, const Tile<T, IN>& m, const T* __restrict__ data) {
+__device__ __forceinline__ void tile_load(const Tile<T, IN>& t, const T* __restrict__ data) {
     const uint32_t nx = (uint32_t)t.g.nx, nxy = nx * (uint32_t)t.g.ny;  // (fields have fewer than 2^31 values)
-    const T* base = data + ((uint64_t)m.oz * nxy + (uint64_t)m.oy * nx + m.ox);
+    const T* base = data + ((uint64_t)t.oz * nxy + (uint64_t)t.oy * nx + t.ox);
     T v[17], fy = (T)0, fx = (T)0, e = (T)0;
-    const RowLane<kGroup<T, COMPRESS>> r;
-    const bool on = m.template in<0>(r.X) && m.template in<1>(r.y);
+    const RowLane<1> r;
+    const bool on = t.template in<0>(r.X) && t.template in<1>(r.y);
     Column<const T, IN> p(base, nx, nxy, r.X, r.y);
 #pragma unroll
     for (int z = 0; z < 17; ++z) {
         v[z] = (T)0;
-        if (on && m.template in<2>(z)) v[z] = p.at();
+        if (on && t.template in<2>(z)) v[z] = p.at();
         p.next();
     }
-    if (m.in3(r.X, 16, r.y)) fy = base[(uint64_t)r.y * nxy + (16 * (uint64_t)nx + r.X)];
+    if (t.in3(r.X, 16, r.y)) fy = base[(uint64_t)r.y * nxy + (16 * (uint64_t)nx + r.X)];
     const int l = lane_id(), y = l & 15, z = l >> 4;
     int ex, ey, ez;
     const bool edge = edge_point(l, ex, ey, ez);
-    base += t.ox - m.ox;
     if (t.in3(16, y, z)) fx = base[(uint64_t)z * nxy + ((uint64_t)y * nx + 16)];
     if (edge && t.in3(ex, ey, ez)) e = base[(uint64_t)ez * nxy + ((uint64_t)ey * nx + ex)];
-    T* d = m.s + r.slot(r.y, 0);
+    T* d = t.s + r.slot(r.y, 0);
 #pragma unroll
     for (int k = 0; k < 17; ++k) d[k * kZP] = v[k];
-    m.s[r.slot(16, r.y)] = fy;
+    t.s[r.slot(16, r.y)] = fy;
     t.s[tslot(16, y, z)] = fx;
     if (edge) t.s[tslot(ex, ey, ez)] = e;
 }
