@@ -67,7 +67,8 @@ def _compress_need(t: torch.Tensor) -> int:
     L = pipeline.layout(nx, ny, nz)
     lib = pipeline.lib()
     bound = lib.pa_compress_bound(pipeline.C.byref(L), pipeline.DTYPES[t.dtype])
-    return int(bound + 4 * L.code_len + L.host_size + (L.nchunks + 1) * 8 + L.n4 * t.element_size() + 8192)
+    encoder = lib.pa_encode_workspace(pipeline.C.byref(L))
+    return int(bound + 4 * L.code_len + L.host_size + encoder + L.n4 * t.element_size() + 8192)
 
 
 def _result_bytes(req: Request) -> int:
