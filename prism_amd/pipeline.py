@@ -201,13 +201,14 @@ def compress(data: torch.Tensor, eb: float, rel: bool = True, progressive: bool 
     st = _stream()
     dev = data.device
     V = C.c_void_p
+    lb, Lp = lib(), C.byref(L)
     # the small per-call buffers in one allocation (byte offsets): bounds
     # double[16] at 0, the encoder's workspace at 128 (its error word first,
     # so that the one host read below takes it with the bounds), then min/max
     # double[4], scores double[15], flags uint8[8], cum int64[128], sizes
     # int64[2] and the tuner's workspace from e = 128 + encoder workspace
-    tws_bytes = max(8, lib().pa_autotune_workspace(C.byref(L)))
-    ews_bytes = lib().pa_encode_workspace(C.byref(L))
+    tws_bytes = max(8, lb.pa_autotune_workspace(Lp))
+    ews_bytes = lb.pa_encode_workspace(Lp)
     e = 128 + (ews_bytes + 127) // 128 * 128
     small = torch.empty((e + 1216 + tws_bytes + 7) // 8, dtype=torch.float64, device=dev)
     sp = small.data_ptr()
@@ -216,40 +217,40 @@ def compress(data: torch.Tensor, eb: float, rel: bool = True, progressive: bool 
         V(sp + e + 1216))
     # planes that hold no bit are neither written nor read where that pays, but
     # where the planes are handed out
-    live = not return_parts and bool(lib().pa_live_planes(C.byref(L)))
+    live = not return_parts and bool(lb.pa_live_planes(Lp))
     if live:
-        check(lib().pa_encode_prepare(C.byref(L), p_ews, ews_bytes, st), "pa_encode_prepare")
+        check(lb.pa_encode_prepare(Lp, p_ews, ews_bytes, st), "pa_encode_prepare")
     if rel:  # extrema, auto-tuning and the level bounds share one launch sequence
         with tm("extrema"):
-            check(lib().pa_extrema_autotune(_p(data), dt, C.byref(L), p_mm, float(eb), p_bounds, p_scores, p_flags,
+            check(lb.pa_extrema_autotune(_p(data), dt, Lp, p_mm, float(eb), p_bounds, p_scores, p_flags,
                                             p_tws, tws_bytes, st), "pa_extrema_autotune")
     else:
         with tm("autotune"):
-            check(lib().pa_autotune(_p(data), dt, C.byref(L), p_scores, p_flags, p_tws, tws_bytes, st), "pa_autotune")
-        check(lib().pa_level_bounds(None, float(eb), dt, p_bounds, st), "pa_level_bounds")
+            check(lb.pa_autotune(_p(data), dt, Lp, p_scores, p_flags, p_tws, tws_bytes, st), "pa_autotune")
+        check(lb.pa_level_bounds(None, float(eb), dt, p_bounds, st), "pa_level_bounds")
     qc = torch.empty(L.code_len, dtype=torch.int32, device=dev)
     anchors = torch.empty(L.n4, dtype=data.dtype, device=dev)
     with tm("predict"):
         if live:
-            check(lib().pa_spline_construct_live(_p(data), dt, C.byref(L), p_bounds, p_flags, _p(qc), _p(anchors), p_ews,
+            check(lb.pa_spline_construct_live(_p(data), dt, Lp, p_bounds, p_flags, _p(qc), _p(anchors), p_ews,
                                                  ews_bytes, st), "pa_spline_construct_live")
         else:
-            check(lib().pa_spline_construct_dev(_p(data), dt, C.byref(L), p_bounds, p_flags, _p(qc), _p(anchors), st),
+            check(lb.pa_spline_construct_dev(_p(data), dt, Lp, p_bounds, p_flags, _p(qc), _p(anchors), st),
                   "pa_spline_construct_dev")
     bp = _empty(L.host_size)
     mode = PA_MODE_NB if progressive else PA_MODE_SM
     with tm("shuffle"):
         if live:
-            check(lib().pa_bitshuffle_live(_p(qc), C.byref(L), mode, _p(bp), p_ews, ews_bytes, st), "pa_bitshuffle_live")
+            check(lb.pa_bitshuffle_live(_p(qc), Lp, mode, _p(bp), p_ews, ews_bytes, st), "pa_bitshuffle_live")
         else:
-            check(lib().pa_bitshuffle(_p(qc), C.byref(L), mode, _p(bp), st), "pa_bitshuffle")
-    bound = lib().pa_compress_bound(C.byref(L), dt)
+            check(lb.pa_bitshuffle(_p(qc), Lp, mode, _p(bp), st), "pa_bitshuffle")
+    bound = lb.pa_compress_bound(Lp, dt)
     out = _empty(bound)
-    encode = lib().pa_lossless_encode_live if live else lib().pa_lossless_encode
+    encode = lb.pa_lossless_encode_live if live else lb.pa_lossless_encode
     with tm("encode"):
-        check(encode(_p(bp), C.byref(L), _p(out), p_cum, p_sizes, p_ews, ews_bytes, st), "pa_lossless_encode")
+        check(encode(_p(bp), Lp, _p(out), p_cum, p_sizes, p_ews, ews_bytes, st), "pa_lossless_encode")
     with tm("merge"):  # the stream length goes to bounds[15] (int64 bits)
-        check(lib().pa_compress_merge(_p(out), C.byref(L), dt, p_sizes, p_flags, V(sp + 8), p_cum, _p(anchors),
+        check(lb.pa_compress_merge(_p(out), Lp, dt, p_sizes, p_flags, V(sp + 8), p_cum, _p(anchors),
                                       V(sp + 120), st), "pa_compress_merge")
     # the one host read: stream length, status, range, the encoder's error word
     vals = _host_read(small[0:17])
