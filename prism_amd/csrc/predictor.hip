@@ -1205,8 +1205,9 @@ __global__ __launch_bounds__(kThreads) void line_kernel(SplineArgs<T> a) {
 __host__ __device__ inline bool line_field(const Geom& g) { return g.ny == 1 && g.nz == 1; }
 
 // Waves per SIMD the registers must leave room for: float64, what the LDS
-// allows (4 workgroups of 4 waves per CU); float32, 6 (8 would spill: 512^3
-// compression 469 against 372 us).
+// allows (4 workgroups of 4 waves per CU); float32, 6 (80 registers; asked for 8
+// waves, the compression kernel spilled and took 469 us on 512^3, 372 with 6, before
+// its codes left as rows).
 template <typename T>
 constexpr int kTileWaves = sizeof(T) == 4 ? 6 : 4;
 
